@@ -37,9 +37,7 @@ namespace sphgpu {
 
 namespace {
 
-constexpr int kSortThreads = 256;
-constexpr int kSortItems = 16;
-constexpr int kSortTile = kSortThreads * kSortItems;
+constexpr int kSortTile = 4096;  // elements of a radix-sort workgroup
 
 struct TreeShape {
     int dim;
@@ -161,19 +159,32 @@ __global__ void k_keys(const double *__restrict__ x, const double *__restrict__ 
 // and every node boundary the build uses lies at depth <= D).  flag[1] gets 1
 // if some cell of depth D holds more.
 
-__global__ __launch_bounds__(kSortThreads) void k_radix_hist(const unsigned long long *__restrict__ key, int n,
-                                                            int shift, unsigned int *__restrict__ hist, int nblocks)
+// 1024 threads with four keys each, loaded before the first count: with 256
+// threads and 16 keys a tile took 6.9 us at 1M particles (245 tiles) and 6.0
+// at 14k (four tiles), the latency of the loads one after the other; now 4.8
+// and 4.3.
+constexpr int kScatterThreads = 1024;
+constexpr int kScatterItems = kSortTile / kScatterThreads;
+constexpr int kScatterWaves = kScatterThreads / kWave;
+
+__global__ __launch_bounds__(kScatterThreads) void k_radix_hist(const unsigned long long *__restrict__ key, int n,
+                                                                int shift, unsigned int *__restrict__ hist, int nblocks)
 {
     __shared__ unsigned int cnt[256];
-    cnt[threadIdx.x] = 0;
-    __syncthreads();
+    if (threadIdx.x < 256) cnt[threadIdx.x] = 0;
     const int base = blockIdx.x * kSortTile;
-    for (int r = 0; r < kSortItems; ++r) {
-        const int e = base + r * kSortThreads + threadIdx.x;
-        if (e < n) atomicAdd(&cnt[(unsigned)(key[e] >> shift) & 255u], 1u);
+    unsigned d[kScatterItems];
+#pragma unroll
+    for (int r = 0; r < kScatterItems; ++r) {
+        const int e = base + r * kScatterThreads + threadIdx.x;
+        d[r] = e < n ? (unsigned)(key[e] >> shift) & 255u : 256u;
     }
     __syncthreads();
-    hist[threadIdx.x * nblocks + blockIdx.x] = cnt[threadIdx.x];
+#pragma unroll
+    for (int r = 0; r < kScatterItems; ++r)
+        if (d[r] < 256u) atomicAdd(&cnt[d[r]], 1u);
+    __syncthreads();
+    if (threadIdx.x < 256) hist[threadIdx.x * nblocks + blockIdx.x] = cnt[threadIdx.x];
 }
 
 // ---- multi-block exclusive scan of unsigned counts -----------------------------
@@ -344,56 +355,170 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_apply(const unsigned *in,
     }
 }
 
-__global__ __launch_bounds__(kSortThreads) void k_radix_scatter(
+// order LDS accesses between the lanes of one wavefront
+__device__ __forceinline__ void sort_wave_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// One digit of a stable pass for a wavefront's 64 elements: returns the
+// element's rank among the wave's elements of the same digit so far, and adds
+// the 64 to the wave's own digit counters (LDS, no barrier: the counters are
+// private to the wave, and its LDS operations run in order).  Lanes past the
+// last element pass digit 255: they come after every element, so they only
+// count where nothing follows.
+__device__ __forceinline__ unsigned wave_digit_rank(unsigned d, unsigned long long lt, unsigned *cnt)
+{
+    // lanes holding the same digit
+    unsigned long long same = ~0ull;
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+        const bool bit = (d >> b) & 1u;
+        const unsigned long long bal = __ballot(bit);
+        same &= bit ? bal : ~bal;
+    }
+    const int rank = __popcll(same & lt);
+    const unsigned before = cnt[d];
+    sort_wave_fence();
+    if (rank == 0) cnt[d] = before + __popcll(same);
+    sort_wave_fence();
+    return before + rank;
+}
+
+// One stable pass over a tile.  What bounds it is the serial chain of a tile's
+// rounds (245 tiles at 1M particles, one per CU): 16 rounds of 256 elements
+// with four barriers each took 18.4 us a pass, 14.4 at 14k.  Sixteen
+// wavefronts rank a contiguous sixteenth of the tile each, in four rounds
+// against counters of their own, and the workgroup meets twice: 12.8 us at 1M
+// (the scattered 12-byte stores are most of what is left), 8.1 at 14k.
+
+// the digit counts of the tile's waves, in place, to each wave's first
+// destination: run = the first destination of digit `tid` in the tile
+__device__ __forceinline__ void wave_digit_starts(unsigned (*wcnt)[256], int tid, unsigned run)
+{
+    unsigned c[kScatterWaves];
+#pragma unroll
+    for (int q = 0; q < kScatterWaves; ++q) c[q] = wcnt[q][tid];
+#pragma unroll
+    for (int q = 0; q < kScatterWaves; ++q) {
+        wcnt[q][tid] = run;
+        run += c[q];
+    }
+}
+
+__global__ __launch_bounds__(kScatterThreads) void k_radix_scatter(
     const unsigned long long *__restrict__ key_in, const int *__restrict__ val_in, unsigned long long *__restrict__ key_out,
     int *__restrict__ val_out, int n, int shift, const unsigned int *__restrict__ hist, int nblocks)
 {
-    constexpr int kWaves = kSortThreads / kWave;
-    __shared__ unsigned int base[256];
-    __shared__ unsigned int running[256];
-    __shared__ unsigned int wcnt[kWaves][256];
+    __shared__ unsigned int wcnt[kScatterWaves][256];
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int w = tid / kWave;
-    base[tid] = hist[tid * nblocks + blockIdx.x];
-    running[tid] = 0;
     const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    const int tile = blockIdx.x * kSortTile;
-    for (int r = 0; r < kSortItems; ++r) {
-        for (int q = 0; q < kWaves; ++q) wcnt[q][tid] = 0;
-        __syncthreads();
-        const int e = tile + r * kSortThreads + tid;
-        const bool valid = e < n;
-        unsigned long long k = 0;
-        int v = 0;
-        unsigned d = 256;  // invalid lanes take a digit no valid lane has
-        if (valid) {
-            k = key_in[e];
-            v = val_in[e];
-            d = (unsigned)(k >> shift) & 255u;
+    const int first = blockIdx.x * kSortTile + w * (kWave * kScatterItems) + lane;
+    unsigned long long k[kScatterItems];
+    int v[kScatterItems];
+    unsigned rank[kScatterItems];
+#pragma unroll
+    for (int r = 0; r < kScatterItems; ++r) {
+        const int e = first + r * kWave;
+        k[r] = e < n ? key_in[e] : ~0ull;
+        v[r] = e < n ? val_in[e] : 0;
+    }
+    const unsigned base = tid < 256 ? hist[tid * nblocks + blockIdx.x] : 0u;
+    for (int q = lane; q < 256; q += kWave) wcnt[w][q] = 0;
+    sort_wave_fence();
+#pragma unroll
+    for (int r = 0; r < kScatterItems; ++r) rank[r] = wave_digit_rank((unsigned)(k[r] >> shift) & 255u, lt, wcnt[w]);
+    __syncthreads();
+    if (tid < 256) wave_digit_starts(wcnt, tid, base);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kScatterItems; ++r)
+        if (first + r * kWave < n) {
+            const unsigned dst = wcnt[w][(unsigned)(k[r] >> shift) & 255u] + rank[r];
+            key_out[dst] = k[r];
+            val_out[dst] = v[r];
         }
-        // lanes holding the same digit (9 ballots: 8 digit bits + validity)
-        unsigned long long same = __ballot(1);
-        for (int b = 0; b < 9; ++b) {
-            const bool bit = (d >> b) & 1u;
-            const unsigned long long bal = __ballot(bit);
-            same &= bit ? bal : ~bal;
+}
+
+// All passes of a small sort in one workgroup: at these sizes a pass of three
+// launches costs their latency alone (hist 4.3 us, scan 3.3, scatter 14.7 at
+// 4096 particles), so the elements go back and forth between the two buffers
+// inside one launch, 7 us a pass.  Element order, and with it the result, is
+// that of the tiled passes (both are stable).  One tile is the limit: at 14k
+// (four times the rounds of one CU) it took 25 us a pass, the tiled passes
+// take 16.  Ends in buffer a for an even number of passes, in b for an odd one.
+constexpr int kSmallMax = kSortTile;
+
+__global__ __launch_bounds__(kScatterThreads) void k_sort_small(unsigned long long *key_a, int *val_a,
+                                                                unsigned long long *key_b, int *val_b, int n,
+                                                                int passes)
+{
+    __shared__ unsigned int wcnt[kScatterWaves][256];
+    __shared__ unsigned int wtot[4];
+    const int tid = threadIdx.x;
+    const int lane = tid & (kWave - 1);
+    const int w = tid / kWave;
+    const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    const int items = (n + kScatterThreads - 1) / kScatterThreads;  // rounds per wave
+    const int first = w * (kWave * items) + lane;
+    unsigned long long *kin = key_a, *kout = key_b;
+    int *vin = val_a, *vout = val_b;
+    for (int p = 0; p < passes; ++p) {
+        const int shift = 8 * p;
+        unsigned long long k[kScatterItems];
+        int v[kScatterItems];
+        unsigned rank[kScatterItems];
+#pragma unroll
+        for (int r = 0; r < kScatterItems; ++r) {
+            const int e = first + r * kWave;
+            const bool in = r < items && e < n;
+            k[r] = in ? kin[e] : ~0ull;
+            v[r] = in ? vin[e] : 0;
         }
-        const int rank = __popcll(same & lt);
-        if (valid && rank == 0) wcnt[w][d] = __popcll(same);
-        __syncthreads();
-        if (valid) {
-            unsigned int pre = 0;
-            for (int q = 0; q < w; ++q) pre += wcnt[q][d];
-            const unsigned int dst = base[d] + running[d] + pre + rank;
-            key_out[dst] = k;
-            val_out[dst] = v;
+        for (int q = lane; q < 256; q += kWave) wcnt[w][q] = 0;
+        sort_wave_fence();
+#pragma unroll
+        for (int r = 0; r < kScatterItems; ++r) {
+            if (r >= items) break;  // uniform
+            rank[r] = wave_digit_rank((unsigned)(k[r] >> shift) & 255u, lt, wcnt[w]);
         }
         __syncthreads();
-        unsigned int tot = 0;
-        for (int q = 0; q < kWaves; ++q) tot += wcnt[q][tid];
-        running[tid] += tot;
+        // exclusive scan of the digits' counts (digit tid, four wavefronts)
+        unsigned sum = 0, x = 0;
+        if (tid < 256) {
+#pragma unroll
+            for (int q = 0; q < kScatterWaves; ++q) sum += wcnt[q][tid];
+            x = sum;
+            for (int off = 1; off < kWave; off <<= 1) {
+                const unsigned y = __shfl_up(x, off, kWave);
+                if (lane >= off) x += y;
+            }
+            if (lane == kWave - 1) wtot[w] = x;
+        }
         __syncthreads();
+        if (tid < 256) {
+            unsigned run = x - sum;
+            for (int q = 0; q < w; ++q) run += wtot[q];
+            wave_digit_starts(wcnt, tid, run);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kScatterItems; ++r)
+            if (r < items && first + r * kWave < n) {
+                const unsigned dst = wcnt[w][(unsigned)(k[r] >> shift) & 255u] + rank[r];
+                kout[dst] = k[r];
+                vout[dst] = v[r];
+            }
+        __syncthreads();  // the next pass reads what the whole workgroup wrote
+        unsigned long long *tk = kin;
+        kin = kout;
+        kout = tk;
+        int *tv = vin;
+        vin = vout;
+        vout = tv;
     }
 }
 
@@ -1016,12 +1141,22 @@ int tree_build(sphgpu_ctx *c)
             cut = key_bits - c->dim * ((key_bits - 8 * skip) / c->dim);
         }
     }
-    for (int p = skip; p < passes; ++p) {
+    // up to one tile of elements: all passes in one launch (k_sort_small)
+    const bool small = n <= kSmallMax;
+    if (small) {
+        hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(kScatterThreads), 0, c->stream, t.key, t.perm, t.key_alt, t.perm_alt,
+                           n, passes);
+        if (passes & 1) {
+            std::swap(t.key, t.key_alt);
+            std::swap(t.perm, t.perm_alt);
+        }
+    }
+    for (int p = skip; !small && p < passes; ++p) {
         const int shift = 8 * p;
-        hipLaunchKernelGGL(k_radix_hist, dim3(nb), dim3(kSortThreads), 0, c->stream, (const unsigned long long *)t.key, n,
+        hipLaunchKernelGGL(k_radix_hist, dim3(nb), dim3(kScatterThreads), 0, c->stream, (const unsigned long long *)t.key, n,
                            shift, t.hist, nb);
         scan_counts(c->stream, t.hist, t.hist, 256 * nb, t.scan_tmp, false);
-        hipLaunchKernelGGL(k_radix_scatter, dim3(nb), dim3(kSortThreads), 0, c->stream,
+        hipLaunchKernelGGL(k_radix_scatter, dim3(nb), dim3(kScatterThreads), 0, c->stream,
                            (const unsigned long long *)t.key, (const int *)t.perm, t.key_alt, t.perm_alt, n, shift,
                            (const unsigned int *)t.hist, nb);
         std::swap(t.key, t.key_alt);
