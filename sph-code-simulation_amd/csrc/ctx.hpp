@@ -91,6 +91,8 @@ struct Tree {
     // gravity walk records (one per node, refreshed by each gravity call)
     GravNode *gnode = nullptr;
     int gnode_cap = 0;
+    double *gpart = nullptr;         // sums of a walk in gpart_seg pieces, [gpart_seg][4][n]
+    int gpart_seg = 0;
     // root geometry (device): center[3], edge
     double *root = nullptr;
     int node_cap = 0;

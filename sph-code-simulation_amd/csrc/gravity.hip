@@ -18,9 +18,12 @@
 // leaf members of its own reference walk, in the same pre-order, while node
 // records are wave-uniform loads and member records are loaded once per wave
 // instead of once per lane.  The pair and monopole terms run in the pair
-// precision T with compensated sums taken in blocks of at most 16 terms.
+// precision T with compensated sums taken in blocks of at most 16 terms.  The
+// node range is cut into pieces walked by different wavefronts; their sums are
+// added in node order in FP64.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 
 #include "ctx.hpp"
@@ -82,11 +85,14 @@ template <typename T> struct GravArgs {
     const double *x64[3];
     RecView<T> rv;
     const GravNode *__restrict__ node;
-    double *acc[3];
-    double *phi;
     double theta2, G;
     Box box;
     long long *stats;
+    // the walk in nseg pieces: piece s takes the nodes
+    // [n_nodes s / nseg, n_nodes (s + 1) / nseg) and writes its sums to
+    // part[(4 s + c) n + i], c = phi, a_x, a_y, a_z
+    int nseg;
+    double *part;
 };
 
 // one record per node, pre-order: centre of mass, edge^2 (the reference's
@@ -135,7 +141,15 @@ __global__ __launch_bounds__(256) void k_gravity(GravArgs<T> a)
     __shared__ GravStage<T> stage[4];
     GravStage<T> &st = stage[(threadIdx.x >> 6) & 3];
     const int lane = threadIdx.x & (kWave - 1);
-    const int i0 = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    // The pieces of a workgroup's particles are neighbours in the logical
+    // order, rotated by a hash of the workgroup: the piece with the particles'
+    // own surroundings is the heavy one, and any regular stride between the
+    // heavy pieces sends them to the same shader engines (two pieces at 1M
+    // particles: 5.1 ms at the same instruction count, against 3.4 ms).
+    const int block = xcd_block(blockIdx.x, gridDim.x);
+    const int group = block / a.nseg;
+    const int seg = (int)(((unsigned)block + (((unsigned)group * 0x9E3779B1u) >> 16)) % (unsigned)a.nseg);
+    const int i0 = group * blockDim.x + threadIdx.x;
     if ((i0 & ~(kWave - 1)) >= a.n) return;  // whole wave beyond the particles
     const bool valid = i0 < a.n;
     const int i = valid ? i0 : a.n - 1;
@@ -169,12 +183,41 @@ __global__ __launch_bounds__(256) void k_gravity(GravArgs<T> a)
         for (int k = 0; k < D; ++k) ac[k].fold();
     };
     int since_fold = 0;  // node steps since the last fold (wave-uniform)
-    long long inter = 0;
+    int inter = 0;
     // the lane takes part in the walk from node `resume` on; a lane that
     // accepted a node's monopole resumes at the node's subtree end
     int resume = valid ? 0 : INT_MAX;
-    int node = 0;
-    while (node < a.n_nodes) {
+    // BHNode::calc_force opening test (src/bhtree.cpp:350-358): d and d^2 to
+    // the node's centre of mass, and whether this lane opens the node
+    auto opens = [&](const GravNode &g, double d[3], double &d2) -> bool {
+        const double cm[3] = {g.cx, g.cy, g.cz};
+#pragma unroll
+        for (int k = 0; k < D; ++k) {
+            d[k] = grav_rij<P, double>(ri[k], cm[k], a.box, k);
+            d2 = (k == 0) ? d[k] * d[k] : d2 + d[k] * d[k];
+        }
+        return (g.l2 > a.theta2 * d2) || (d2 < g.l2);
+    };
+    int node = (int)((long long)a.n_nodes * seg / a.nseg);
+    const int node_end = (int)((long long)a.n_nodes * (seg + 1) / a.nseg);
+    if (node > 0) {
+        // a later piece: a lane that accepts an ancestor of the first node has
+        // that subtree in the ancestor's piece and resumes behind it
+        int anc = 0;
+        while (anc != node) {
+            const GravNode g = a.node[anc];
+            double d[3] = {0, 0, 0}, d2 = 0.0;
+            if (anc >= resume && !opens(g, d, d2)) resume = g.skip;
+            // the child whose subtree holds the first node
+            int ch = anc + 1, sk = a.node[ch].skip;
+            while (sk <= node) {
+                ch = sk;
+                sk = a.node[ch].skip;
+            }
+            anc = ch;
+        }
+    }
+    while (node < node_end) {
         // a lane adds at most one monopole per node step
         if (++since_fold == 16) {
             fold();
@@ -183,15 +226,9 @@ __global__ __launch_bounds__(256) void k_gravity(GravArgs<T> a)
         const GravNode g = a.node[node];
         const bool act = node >= resume;
         double d[3] = {0, 0, 0};
-        const double cm[3] = {g.cx, g.cy, g.cz};
         double d2 = 0.0;
-#pragma unroll
-        for (int k = 0; k < D; ++k) {
-            d[k] = grav_rij<P, double>(ri[k], cm[k], a.box, k);
-            d2 = (k == 0) ? d[k] * d[k] : d2 + d[k] * d[k];
-        }
-        // BHNode::calc_force opening test (src/bhtree.cpp:350-358)
-        const bool open = act && ((g.l2 > a.theta2 * d2) || (d2 < g.l2));
+        const bool opened = opens(g, d, d2);
+        const bool open = act && opened;
         if (act && !open) {
             // monopole (src/bhtree.cpp:387-392)
             const T r_inv = (sizeof(T) == 4) ? trsqrt(T(d2)) : tdiv(T(1.0), tsqrt(T(d2)));
@@ -289,15 +326,47 @@ __global__ __launch_bounds__(256) void k_gravity(GravArgs<T> a)
         ++node;
     }
     if (valid) {
-        a.phi[i] = (double)phi.get();
+        double *const q = a.part + 4 * (size_t)seg * a.n + i;
+        q[0] = (double)phi.get();
 #pragma unroll
-        for (int k = 0; k < D; ++k) a.acc[k][i] += (double)ac[k].get();
+        for (int k = 0; k < D; ++k) q[(size_t)(k + 1) * a.n] = (double)ac[k].get();
     }
     for (int off = kWave / 2; off > 0; off >>= 1) inter += __shfl_xor(inter, off, kWave);
     if (lane == 0) atomicAdd(stat_ptr(a.stats, 10), (unsigned long long)inter);
 }
 
-template <typename T> void launch_gravity(sphgpu_ctx *c)
+// the pieces' sums in node order (FP64, deterministic), one thread per
+// particle and component
+__global__ void k_gravity_sum(int n, int nseg, const double *__restrict__ part, double *__restrict__ phi, double *ax,
+                              double *ay, double *az)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, c = blockIdx.y;
+    if (i >= n) return;
+    const double *const q = part + (size_t)c * n + i;
+    double s = 0.0;
+#pragma unroll 8
+    for (int g = 0; g < nseg; ++g) s += q[4 * (size_t)g * n];
+    if (c == 0) phi[i] = s;
+    else (c == 1 ? ax : c == 2 ? ay : az)[i] += s;
+}
+
+// Pieces of the walk.  One wavefront walks the tree for 64 particles, a serial
+// chain of a thousand node steps: 800 us for 14k particles, whose 224
+// wavefronts leave most of the chip idle.  The pre-order node range is
+// therefore split until about kGravWaves wavefronts are there to be scheduled
+// (8 fit a SIMD, 8192 the chip; the pieces of a walk are very uneven, so
+// several times that).  Evrard, 14k particles: 801 us -> 103 (pieces capped at
+// 32: 167, at 64: 132); 200k: 1284 -> 1026 (20 pieces); 1M, bound by VALU issue:
+// 3452 -> 3368 (4 pieces).
+constexpr int kGravWaves = 65536;
+constexpr int kGravSegMax = 128;
+int grav_pieces(int n, int n_nodes)
+{
+    const int waves = (n + kWave - 1) / kWave;
+    return std::max(1, std::min({kGravWaves / waves, kGravSegMax, n_nodes}));
+}
+
+template <typename T> void launch_gravity(sphgpu_ctx *c, int nseg)
 {
     GravArgs<T> a;
     a.n = c->n;
@@ -305,13 +374,13 @@ template <typename T> void launch_gravity(sphgpu_ctx *c)
     for (int k = 0; k < 3; ++k) a.x64[k] = c->pos[k < c->dim ? k : 0];
     a.rv = rec_view<T>(c);
     a.node = c->tree.gnode;
-    for (int k = 0; k < 3; ++k) a.acc[k] = c->acc[k];
-    a.phi = c->sc[S_PHI];
     a.theta2 = c->prm.theta * c->prm.theta;
     a.G = c->prm.gravity_constant;
     a.box = c->box;
     a.stats = c->dstats;
-    const dim3 g(grid_for(c->n, 256)), b(256);
+    a.nseg = nseg;
+    a.part = c->tree.gpart;
+    const dim3 g(grid_for(c->n, 256) * nseg), b(256);
 #define LAUNCH(D)                                                                          \
     if (c->box.periodic) hipLaunchKernelGGL((k_gravity<D, T, true>), g, b, 0, c->stream, a); \
     else hipLaunchKernelGGL((k_gravity<D, T, false>), g, b, 0, c->stream, a);
@@ -343,9 +412,20 @@ int gravity(sphgpu_ctx *c)
     hipLaunchKernelGGL(k_grav_nodes, dim3(grid_for(t.n_nodes, 256)), dim3(256), 0, c->stream, t.n_nodes, t.node_cap,
                        t.com, t.edge, t.mass, t.start, t.end, t.skip, t.level, t.gnode);
     time_end(c);
+    const int nseg = grav_pieces(c->n, t.n_nodes);
+    if (nseg > t.gpart_seg) {
+        if (t.gpart) hipFree(t.gpart);
+        t.gpart = nullptr;
+        t.gpart_seg = 0;
+        if (hipMalloc((void **)&t.gpart, sizeof(double) * 4 * (size_t)nseg * c->n) != hipSuccess)
+            return fail(c, SPHGPU_E_NOMEM, "gravity piece sums");
+        t.gpart_seg = nseg;
+    }
     time_begin(c, "gravity");
-    if (c->prm.pair_precision == SPHGPU_PAIR_FP64) launch_gravity<double>(c);
-    else launch_gravity<float>(c);
+    if (c->prm.pair_precision == SPHGPU_PAIR_FP64) launch_gravity<double>(c, nseg);
+    else launch_gravity<float>(c, nseg);
+    hipLaunchKernelGGL(k_gravity_sum, dim3(grid_for(c->n, 256), c->dim + 1), dim3(256), 0, c->stream, c->n, nseg,
+                       (const double *)t.gpart, c->sc[S_PHI], c->acc[0], c->acc[1], c->acc[2]);
     time_end(c);
     HIPCHK(c, hipGetLastError());
     return 0;

@@ -1054,7 +1054,7 @@ void tree_free(sphgpu_ctx *c)
     Tree &t = c->tree;
     void *ps[] = {t.key, t.key_alt, t.perm, t.perm_alt, t.kdig, t.lam, t.sync_words, t.leaf_end, t.ncount, t.nbase, t.start,
                   t.end, t.skip, t.level, t.center, t.edge, t.ks, t.mass, t.com, t.bmax1, t.bmax2, t.bsum1,
-                  t.bsum2, t.root, t.hist, t.nbox, t.nlink, t.scan_tmp, t.nhalf, t.nchild, t.child, t.ccount, t.gnode};
+                  t.bsum2, t.root, t.hist, t.nbox, t.nlink, t.scan_tmp, t.nhalf, t.nchild, t.child, t.ccount, t.gnode, t.gpart};
     for (void *p : ps)
         if (p) hipFree(p);
     if (t.host_words) hipHostFree(t.host_words);

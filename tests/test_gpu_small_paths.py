@@ -55,3 +55,55 @@ def test_key_sort_order(n, dim):
     c.build_tree()
     np.testing.assert_array_equal(c.tree_dump()["members"], _key_order(p, f[ics.F_POS:ics.F_POS + dim]))
     c.close()
+
+
+def _hk_sum(x, m, h, g):
+    """Direct softened sum (src/bhtree.cpp:319-345, 362-378), FP64."""
+    d = x[:, :, None] - x[:, None, :]
+    r = np.sqrt((d * d).sum(axis=0))
+    np.fill_diagonal(r, 1.0)
+
+    def fg(e):
+        u = r / e
+        f1 = (-0.5 * u * u * (1 / 3 - 3 / 20 * u * u + u ** 3 / 20) + 1.4) / e
+        f2 = -1 / (15 * r) + (-u * u * (4 / 3 - u + 0.3 * u * u - u ** 3 / 30) + 1.6) / e
+        g1 = (4 / 3 - 1.2 * u * u + 0.5 * u ** 3) / e ** 3
+        g2 = (-1 / 15 + 8 / 3 * u ** 3 - 3 * u ** 4 + 1.2 * u ** 5 - u ** 6 / 6) / r ** 3
+        return np.where(u < 1, f1, np.where(u < 2, f2, 1 / r)), np.where(u < 1, g1, np.where(u < 2, g2, 1 / r ** 3))
+
+    fi, gi = fg(np.broadcast_to(0.5 * h[:, None], r.shape))
+    fj, gj = fg(np.broadcast_to(0.5 * h[None, :], r.shape))
+    w = g * np.broadcast_to(m[None, :], r.shape).copy()
+    np.fill_diagonal(w, 0.0)
+    return -(0.5 * w * (fi + fj)).sum(axis=1), -(d * (0.5 * w * (gi + gj))).sum(axis=2)
+
+
+@pytest.mark.parametrize("prec,tol", [(ics.PAIR_FP64, 1e-12), (ics.PAIR_FP32, 2e-6)])
+@pytest.mark.parametrize("n,leaf", [(2, 1), (9, 1), (63, 4), (64, 64), (65, 1), (300, 8), (1500, 32)])
+def test_gravity_pieces_direct_sum(n, leaf, prec, tol):
+    """With theta = 0 every node is opened, so the walk's pieces (as many as the
+    nodes, at the smallest sizes) must add up to the direct sum.  FP32: 20 u of
+    the summed magnitudes (positions rounded to FP32 move a term by a few u;
+    the sums are compensated), FP64 far below."""
+    rng = np.random.default_rng([n, leaf])
+    p = ics.default_params(3)
+    p.update(use_gravity=1, theta=0.0, leaf_particle_num=leaf, pair_precision=prec, gravity_constant=0.7)
+    f = ics.empty_fields(n)
+    f[ics.F_POS:ics.F_POS + 3] = rng.uniform(-1, 1, (3, n))
+    f[ics.F_MASS] = rng.uniform(0.5, 1.5, n) / n
+    f[ics.F_DENS] = f[ics.F_ENE] = 1.0
+    f[ics.F_SML] = rng.uniform(0.1, 0.5, n)
+    c = sphgpu.Context(p, n)
+    c.upload(f)
+    c.build_tree()
+    c.gravity()
+    out = c.download()
+    c.close()
+    phi, acc = _hk_sum(f[ics.F_POS:ics.F_POS + 3], f[ics.F_MASS], f[ics.F_SML], 0.7)
+    np.testing.assert_allclose(out[ics.F_PHI], phi, rtol=tol)
+    # acceleration on the scale of the terms' magnitudes, not of their sum
+    x = f[ics.F_POS:ics.F_POS + 3]
+    d = x[:, :, None] - x[:, None, :]
+    r2 = (d * d).sum(axis=0) + np.eye(n)
+    scale = (0.7 * f[ics.F_MASS][None, :] / r2 * (1 - np.eye(n))).sum(axis=1)
+    assert (np.abs(out[ics.F_ACC:ics.F_ACC + 3] - acc) / scale).max() < tol
