@@ -9,18 +9,19 @@
 // src/gsph/g_fluid_force.cpp:93).
 //
 // Here a 64-lane wavefront owns 64 consecutive particles in key order (a
-// compact region of space).  The wave walks the pre-ordered node array
-// stacklessly, 64 nodes per step: lane q tests node w0 + q against the
-// group's FP32 bounding box widened by the group's largest radius (and the
-// node's kernel_size for is_ij), conservatively padded for FP32 rounding; the
-// walk then advances through the window on the wave-uniform reach mask
-// (entered -> next node, pruned -> skip) and loads the next window where it
-// leaves this one.  Members of entered leaves are queued, 64 at a time, in a
-// per-lane candidate buffer; a flush loads the 64 candidate records in one
-// gather and broadcasts them lane by lane, and every lane evaluates the
-// reference's FP64 predicate for its own particle (behind an FP32 prefilter
-// that only settles candidates whose FP32 distance lies outside a proven
-// rounding band), so the resulting sets are exactly the reference's:
+// compact region of space; 32, 16 or 8 with several lanes each in smaller
+// sets).  The wave walks the tree breadth first from the root, 64 frontier
+// nodes per step: lane q tests its node against the group's FP32 bounding box
+// widened by the group's largest radius (and the node's kernel_size for
+// is_ij), conservatively padded for FP32 rounding; reached internal nodes put
+// their children on the next frontier, reached leaves go to a queue.  64 queued
+// leaves at a time, one per lane, are tested against every particle's own
+// sphere, and the members of those that some sphere reaches fill 64-candidate
+// batches; a flush loads a batch's records in one gather, drops those beyond
+// the group, and every lane evaluates the reference's FP64 predicate for its
+// own particle (behind an FP32 prefilter that only settles candidates whose
+// FP32 distance lies outside a proven rounding band), so the resulting sets are
+// exactly the reference's:
 //   is_ij = 0 :  r_ij^2 < hs_i^2
 //   is_ij = 1 :  sqrt(r_ij^2) < max(h_i, h_j)  and  r_ij^2 != 0
 // The group test only prunes; it never decides membership.
@@ -83,6 +84,33 @@ SPH_DEV void wave_lds_fence()
 
 SPH_DEV float rdl(float v, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane)); }
 SPH_DEV int rdl(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+
+// inclusive scans over the wavefront's lanes in data-parallel-primitive moves
+// (row shifts by 1, 2, 4, 8 inside rows of 16 lanes, then the row totals
+// broadcast to the rows behind); every lane must be active
+SPH_DEV int wave_scan_add(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+    return v;
+}
+SPH_DEV int wave_scan_max(int v)
+{
+    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x111, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x112, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x114, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x118, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x142, 0xa, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(-1, v, 0x143, 0xc, 0xf, false));
+    return v;
+}
+// the value of lane ^ 1 and lane ^ 2 of the quad
+SPH_DEV int quad_xor1(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, false); }
+SPH_DEV int quad_xor2(int v) { return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xf, 0xf, false); }
 
 // |minimum-image distance| along one axis in FP32: r^2 only needs |d|, and
 // |d| < L inside the box, so min(|d|, L - |d|) is the minimum image (the
@@ -177,13 +205,20 @@ SPH_DEV void test_range_expand(const float4 *srec, int t0, int t1, const float m
     ku = kl & ~kk;
 }
 
-template <int D, int IS_IJ>
+// LP lanes per particle (1, 2, 4 or 8): a wavefront owns 64 / LP consecutive
+// particles, and the lanes of a particle test a contiguous LP-th of each
+// candidate batch each; their kept candidates follow one another in the list,
+// so the lists do not depend on LP.
+template <int D, int IS_IJ, int LP>
 __global__ __launch_bounds__(256, 4) void k_search(SearchArgs a)
 {
+    constexpr int PW = kWave / LP;   // particles per wavefront
+    constexpr int CH = kWave / LP;   // candidates of a batch per lane
     const int lane = threadIdx.x & (kWave - 1);
+    const int part = lane / LP, sl = lane % LP;
     const int group = (xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x) / kWave;
-    const int i = group * kWave + lane;
-    if (group * kWave >= a.n) return;
+    const int i = group * PW + part;
+    if (group * PW >= a.n) return;
     const bool valid = i < a.n;
     const int ii = valid ? i : (a.n - 1);
     const float4 pfi = a.posf[ii];
@@ -215,19 +250,31 @@ __global__ __launch_bounds__(256, 4) void k_search(SearchArgs a)
     int *const col = a.idx + list_slot(ii, 0, a.cap);
     int visits = 0, tests = 0, windows = 0, leaves = 0;
     int reach = 0;
-    const int p_end = min(group * kWave + kWave, a.n);
-    int sub = group * kWave;
+    const int p_end = min(group * PW + PW, a.n);
+    int sub = group * PW;
     // candidate buffer: lane q holds the q-th pending candidate index
     int cand = 0, nb = 0;
 
     // per-wave LDS broadcast buffer of the pending candidates
-    __shared__ float4 s_rec[4][kWave];
+    // (with LP > 1 one record of padding between the parts that the lanes of a
+    // particle read at the same time, which keeps them on different banks)
+    __shared__ float4 s_rec[4][kWave + LP];
     __shared__ int s_idx[4][kWave];
-    float4 *srec = s_rec[(threadIdx.x / kWave) & 3];
-    int *sidx = s_idx[(threadIdx.x / kWave) & 3];
+    const int wv = (threadIdx.x / kWave) & 3;
+    float4 *srec = s_rec[wv];
+    int *sidx = s_idx[wv];
+    // per-wave particles (x, y, z, radius), the queue of reached leaves, and
+    // the expansion of their members into candidates
+    __shared__ float4 s_part[4][PW];
+    __shared__ int s_leaf[4][2 * kWave];
+    __shared__ int s_mark[4][kWave];
+    float4 *spart = s_part[wv];
+    int *sleaf = s_leaf[wv], *smark = s_mark[wv];
+    int nlq = 0;  // leaves in the queue
+    if (sl == 0) spart[part] = make_float4(xf[0], xf[1], xf[2], Rf);
     // per-wave breadth-first frontiers (current and next level)
     __shared__ int s_fr[4][2][kFrontier];
-    int *sfr[2] = {s_fr[(threadIdx.x / kWave) & 3][0], s_fr[(threadIdx.x / kWave) & 3][1]};
+    int *sfr[2] = {s_fr[wv][0], s_fr[wv][1]};
     // per-piece state used by flush: group centre, and whether candidates can
     // be pre-shifted to the minimum image seen from the group centre
     float g[3] = {0, 0, 0};
@@ -312,29 +359,38 @@ __global__ __launch_bounds__(256, 4) void k_search(SearchArgs a)
         const unsigned long long kb = __ballot(keepc);
         if (keepc) {
             const int pos = __popcll(kb & ((1ull << lane) - 1ull));
-            srec[pos] = rec;
+            srec[LP > 1 ? pos + pos / CH : pos] = rec;
             sidx[pos] = cand;
         }
         nb = __popcll(kb);
         tests += nb;
         wave_lds_fence();
         unsigned km0 = 0, km1 = 0, ku0 = 0, ku1 = 0;
-        const int n0 = min(nb, 32);
+        const int n0 = min(nb, LP > 1 ? CH : 32);
+        const float4 *const sr = srec + (LP > 1 ? sl * (CH + 1) : 0);
         if (expand) {
-            test_range_expand<D>(srec, 0, n0, m2y, Tlo, Thi, km0, ku0);
-            if (nb > 32) test_range_expand<D>(srec, 32, nb, m2y, Tlo, Thi, km1, ku1);
+            test_range_expand<D>(sr, 0, n0, m2y, Tlo, Thi, km0, ku0);
+            if (LP == 1 && nb > 32) test_range_expand<D>(sr, 32, nb, m2y, Tlo, Thi, km1, ku1);
         } else if (!a.box.periodic || shift) {
-            test_range<D, IS_IJ, true>(srec, 0, n0, xf, Lf, Rf, R2lo, R2hi, delta, z2, km0, ku0);
-            if (nb > 32) test_range<D, IS_IJ, true>(srec, 32, nb, xf, Lf, Rf, R2lo, R2hi, delta, z2, km1, ku1);
+            test_range<D, IS_IJ, true>(sr, 0, n0, xf, Lf, Rf, R2lo, R2hi, delta, z2, km0, ku0);
+            if (LP == 1 && nb > 32) test_range<D, IS_IJ, true>(sr, 32, nb, xf, Lf, Rf, R2lo, R2hi, delta, z2, km1, ku1);
         } else {
-            test_range<D, IS_IJ, false>(srec, 0, n0, xf, Lf, Rf, R2lo, R2hi, delta, z2, km0, ku0);
-            if (nb > 32) test_range<D, IS_IJ, false>(srec, 32, nb, xf, Lf, Rf, R2lo, R2hi, delta, z2, km1, ku1);
+            test_range<D, IS_IJ, false>(sr, 0, n0, xf, Lf, Rf, R2lo, R2hi, delta, z2, km0, ku0);
+            if (LP == 1 && nb > 32) test_range<D, IS_IJ, false>(sr, 32, nb, xf, Lf, Rf, R2lo, R2hi, delta, z2, km1, ku1);
         }
         unsigned long long km = ((unsigned long long)km1 << 32) | km0;
         unsigned long long ku = ((unsigned long long)ku1 << 32) | ku0;
+        // this lane's candidates: batch entries t0 .. t0 + nmy - 1
+        const int t0 = LP > 1 ? sl * CH : 0;
+        const int nmy = LP > 1 ? max(0, min(CH, nb - t0)) : nb;
+        const unsigned long long all = (nmy == 64) ? ~0ull : ((1ull << nmy) - 1ull);
         if (!fast) {  // no FP32 band for this lane: FP64 decides every candidate
             km = 0;
-            ku = (nb == 64) ? ~0ull : ((1ull << nb) - 1ull);
+            ku = all;
+        }
+        if (LP > 1) {  // a shorter last part was tested past its end
+            km &= all;
+            ku &= all;
         }
         if (!mine) km = ku = 0;
         if (__ballot(ku != 0ull) != 0ull) {
@@ -342,17 +398,32 @@ __global__ __launch_bounds__(256, 4) void k_search(SearchArgs a)
             while (ku) {
                 const int t = __ffsll((long long)ku) - 1;
                 ku &= ku - 1;
-                if (exact(sidx[t])) km |= 1ull << t;
+                if (exact(sidx[t0 + t])) km |= 1ull << t;
             }
         }
         // append the kept candidates in candidate order, four ranks per
         // round: the four LDS reads are issued together, so a round waits
         // once for LDS instead of once per kept candidate
         const int nkl = __popcll(km);
-        int nk = nkl;
-        for (int off = kWave / 2; off > 0; off >>= 1) nk = max(nk, __shfl_xor(nk, off, kWave));
-        if (count + nkl > a.cap) over = true;
-        for (int r = 0; r < nk; r += 4) {
+        int before = 0, total = nkl;  // kept by the particle's lanes ahead, and by all
+        if (LP >= 2) {
+            const int o = quad_xor1(total);
+            before += (sl & 1) ? o : 0;
+            total += o;
+        }
+        if (LP >= 4) {
+            const int o = quad_xor2(total);
+            before += (sl & 2) ? o : 0;
+            total += o;
+        }
+        if (LP >= 8) {
+            const int o = __shfl_xor(total, 4, kWave);
+            before += (sl & 4) ? o : 0;
+            total += o;
+        }
+        const int row = count + before;
+        if (row + nkl > a.cap) over = true;
+        for (int r = 0; __ballot(km != 0ull); r += 4) {
             int t[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
@@ -361,14 +432,14 @@ __global__ __launch_bounds__(256, 4) void k_search(SearchArgs a)
             }
             int j[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) j[u] = sidx[t[u]];
+            for (int u = 0; u < 4; ++u) j[u] = sidx[t0 + t[u]];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const int q = count + u;
+                const int q = row + r + u;
                 if (r + u < nkl && q < a.cap) col[q * kWave] = j[u];
             }
-            count += max(0, min(4, nkl - r));
         }
+        count += total;
         wave_lds_fence();
         nb = 0;
     };
@@ -475,35 +546,81 @@ __global__ __launch_bounds__(256, 4) void k_search(SearchArgs a)
             }
             return r;
         };
-        // an entered leaf held by lane o: queue its members if some lane's
-        // own sphere reaches the leaf's box
-        auto visit_leaf = [&](int o, const float4 &bx, const float2 &bh, const int4 &lk) {
-            const float lc3[3] = {rdl(bx.x, o), rdl(bx.y, o), rdl(bx.z, o)};
-            const float lh[3] = {rdl(bx.w, o), rdl(bh.x, o), rdl(bh.y, o)};
-            float rl = Rf;
-            if (IS_IJ) rl = fmaxf(rl, fabsf(__int_as_float(rdl(lk.w, o))));
-            rl = rl * kReachRel + padX;
-            float dist2 = 0.f;
+        // The first `cnt` leaves of the queue, one per lane: each lane counts
+        // the piece's particles whose own sphere reaches its leaf's box
+        // (particles broadcast from LDS), and the members of the leaves with
+        // any become candidates, in leaf order.  One leaf at a time with the
+        // particles in the lanes instead cost 45 instructions per leaf (123
+        // leaves per wavefront at 1M particles, up to 356 with small leaves)
+        // in one serial chain.
+        auto process_leaves = [&](int cnt) {
+            int lb = 0, le = 0, hits = 0;
+            if (lane < cnt) {
+                const int k = sleaf[lane];
+                const float4 bx = a.nbox[k];
+                const float2 bh = a.nhalf[k];
+                const int4 lk = a.nlink[k];
+                lb = lk.x;
+                le = lk.y;
+                const float lc3[3] = {bx.x, bx.y, bx.z};
+                const float lh[3] = {bx.w, bh.x, bh.y};
+                const int p1 = sub_end - group * PW;
+                for (int p = sub - group * PW; p < p1; ++p) {
+                    const float4 pq = spart[p];
+                    const float px[3] = {pq.x, pq.y, pq.z};
+                    float rl = pq.w;
+                    if (IS_IJ) rl = fmaxf(rl, fabsf(__int_as_float(lk.w)));
+                    rl = rl * kReachRel + padX;
+                    float dist2 = 0.f;
 #pragma unroll
-            for (int q = 0; q < D; ++q) {
-                const float e = fmaxf(abs_min_image_f(lc3[q] - xf[q], a.box.periodic, Lf[q]) - lh[q], 0.f);
-                dist2 = (q == 0) ? e * e : dist2 + e * e;
-            }
-            const bool own = mine && dist2 <= rl * rl;
-            if (__ballot(own)) {
-                ++leaves;
-                // members this lane's own sphere would have to test in a
-                // per-particle walk (the search's algorithmic work)
-                if (own) reach += rdl(lk.y, o) - rdl(lk.x, o);
-                int s = rdl(lk.x, o);
-                const int e = rdl(lk.y, o);
-                while (s < e) {
-                    const int take = min(e - s, kWave - nb);
-                    if (lane >= nb && lane < nb + take) cand = s + (lane - nb);
-                    nb += take;
-                    s += take;
-                    if (nb == kWave) flush(mine);
+                    for (int q = 0; q < D; ++q) {
+                        const float e = fmaxf(abs_min_image_f(lc3[q] - px[q], a.box.periodic, Lf[q]) - lh[q], 0.f);
+                        dist2 = (q == 0) ? e * e : dist2 + e * e;
+                    }
+                    hits += dist2 <= rl * rl ? 1 : 0;
                 }
+            }
+            leaves += __popcll(__ballot(hits > 0));
+            // members the particles' own spheres would have to test in
+            // per-particle walks (the search's algorithmic work)
+            reach += hits * (le - lb);
+            const int m = hits > 0 ? le - lb : 0;
+            const int incl = wave_scan_add(m);
+            const int total = __builtin_amdgcn_readlane(incl, kWave - 1);
+            const int excl = incl - m;
+            // slot s of the expansion holds member s - excl of the last leaf
+            // with members that starts at or before s
+            int carry = 0;
+            for (int s0 = 0; s0 < total;) {
+                const int take = min(total - s0, kWave - nb);
+                smark[lane] = -1;
+                wave_lds_fence();
+                if (m > 0 && excl >= s0 && excl < s0 + take) smark[excl - s0] = lane;
+                wave_lds_fence();
+                // lane nb + x of the batch takes slot s0 + x
+                const int x = lane - nb;
+                const int own = max(carry, wave_scan_max(x >= 0 && x < take ? smark[x] : -1));
+                const int bias = __shfl(lb - excl, own, kWave);
+                if (x >= 0 && x < take) cand = bias + s0 + x;
+                carry = __builtin_amdgcn_readlane(own, nb + take - 1);
+                wave_lds_fence();
+                nb += take;
+                s0 += take;
+                if (nb == kWave) flush(mine);
+            }
+        };
+        // reached leaves wait in the queue until it holds 64
+        auto queue_leaves = [&](unsigned long long lm, int node) {
+            if ((lm >> lane) & 1ull) sleaf[nlq + __popcll(lm & ((1ull << lane) - 1ull))] = node;
+            nlq += __popcll(lm);
+            wave_lds_fence();
+            if (nlq >= kWave) {
+                process_leaves(kWave);
+                nlq -= kWave;
+                const int v = sleaf[kWave + lane];
+                wave_lds_fence();
+                sleaf[lane] = v;
+                wave_lds_fence();
             }
         };
         // Depth-first walk of the pre-order node range [wb, we) (a whole
@@ -545,7 +662,7 @@ __global__ __launch_bounds__(256, 4) void k_search(SearchArgs a)
                     const int o = off + step;
                     node = w0 + o;
                     if ((mask >> o) & 1ull) {
-                        visit_leaf(o, bx, bh, lk);
+                        queue_leaves(1ull << o, k);
                         ++node;
                     } else {
                         node = rdl(lk.z, o);
@@ -587,20 +704,12 @@ __global__ __launch_bounds__(256, 4) void k_search(SearchArgs a)
                 }
                 visits += min(kWave, nf - base);
                 const bool is_leaf = lk.w < 0;
-                unsigned long long lm = __ballot(act && reach && is_leaf);
-                while (lm) {
-                    const int o = __ffsll((long long)lm) - 1;
-                    lm &= lm - 1;
-                    visit_leaf(o, bx, bh, lk);
-                }
+                const unsigned long long lm = __ballot(act && reach && is_leaf);
+                if (lm) queue_leaves(lm, node);
                 const bool expand = act && reach && !is_leaf;
                 const int cnt = expand ? ch.y : 0;
-                int incl = cnt;
-                for (int off = 1; off < kWave; off <<= 1) {
-                    const int t = __shfl_up(incl, off, kWave);
-                    if (lane >= off) incl += t;
-                }
-                const int total = __shfl(incl, kWave - 1, kWave);
+                const int incl = wave_scan_add(cnt);
+                const int total = __builtin_amdgcn_readlane(incl, kWave - 1);
                 if (nn + total <= kFrontier) {
                     const int pos = nn + incl - cnt;
                     if (expand) {
@@ -629,13 +738,15 @@ __global__ __launch_bounds__(256, 4) void k_search(SearchArgs a)
             nxt = t;
             nf = nn;
         }
+        if (nlq) process_leaves(nlq);
+        nlq = 0;
         if (nb) flush(mine);
         sub = sub_end;
     }
-    if (valid) a.cnt[i] = count < a.cap ? count : a.cap;
+    if (valid && sl == 0) a.cnt[i] = count < a.cap ? count : a.cap;
     if (over) atomicOr(a.overflow, 1);
     // candidate statistics
-    int c = valid ? count : 0;
+    int c = valid && sl == 0 ? count : 0;
     for (int off = kWave / 2; off > 0; off >>= 1) c += __shfl_xor(c, off, kWave);
     for (int off = kWave / 2; off > 0; off >>= 1) nexact += __shfl_xor(nexact, off, kWave);
     long long reach_w = reach;
@@ -649,6 +760,30 @@ __global__ __launch_bounds__(256, 4) void k_search(SearchArgs a)
         atomicAdd(stat_ptr(a.stats, 16), (unsigned long long)leaves);
         atomicAdd(stat_ptr(a.stats, 20), (unsigned long long)reach_w);
     }
+}
+
+// Lanes per particle of a search over n particles.  A wavefront's search is one
+// serial chain (walk, candidate batches, appends) of 50 to 300 us, and the chip
+// holds 4096 of these wavefronts: fewer particles per wavefront shorten the
+// chain but walk the tree more often.  Measured (us, 1 / 2 / 4 / 8 lanes): 500
+// particles in 1D 49 / 35 / 29 / 26, 4k 2D 69 / 38 / 28 / 24, 14k 3D 158 / 107
+// / 71 / 49, 65k 2D 109 / 69 / 59 / 81, 104k 3D 231 / 171 / 175 / 199, 204k 3D
+// 270 / 240 / 246, 262k 3D 141 / 143 / 185, 1M 3D 979 / 1063 / 1311.
+int search_lanes(int n) { return n <= 32768 ? 8 : n <= 98304 ? 4 : n < 262144 ? 2 : 1; }
+
+template <int D, int LP>
+void launch_search_lp(const SearchArgs &a, int is_ij, dim3 grid, dim3 block, hipStream_t st)
+{
+    if (is_ij) hipLaunchKernelGGL((k_search<D, 1, LP>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((k_search<D, 0, LP>), grid, block, 0, st, a);
+}
+
+template <int D> void launch_search(const SearchArgs &a, int is_ij, int lp, dim3 grid, dim3 block, hipStream_t st)
+{
+    if (lp == 8) launch_search_lp<D, 8>(a, is_ij, grid, block, st);
+    else if (lp == 4) launch_search_lp<D, 4>(a, is_ij, grid, block, st);
+    else if (lp == 2) launch_search_lp<D, 2>(a, is_ij, grid, block, st);
+    else launch_search_lp<D, 1>(a, is_ij, grid, block, st);
 }
 
 } // namespace
@@ -725,14 +860,12 @@ int search(sphgpu_ctx *c, Lists &l, int is_ij, const double *radius, bool defer,
         a.stats = c->dstats;
         if (!flag_cleared) HIPCHK(c, hipMemsetAsync(c->dflag, 0, sizeof(int), c->stream));
         flag_cleared = false;  // a repeated search after growing the lists clears it here
-        const int groups = (c->n + kWave - 1) / kWave;
-        const dim3 grid(grid_for((long long)groups * kWave, 256)), block(256);
+        const int lp = search_lanes(c->n);
+        const dim3 grid(grid_for((long long)c->n * lp, 256)), block(256);
         time_begin(c, is_ij ? "search_force" : "search_pre");
-#define LAUNCH(D)                                                                                   \
-    if (is_ij) hipLaunchKernelGGL((k_search<D, 1>), grid, block, 0, c->stream, a);                  \
-    else hipLaunchKernelGGL((k_search<D, 0>), grid, block, 0, c->stream, a);
-        if (c->dim == 1) { LAUNCH(1) } else if (c->dim == 2) { LAUNCH(2) } else { LAUNCH(3) }
-#undef LAUNCH
+        if (c->dim == 1) launch_search<1>(a, is_ij, lp, grid, block, c->stream);
+        else if (c->dim == 2) launch_search<2>(a, is_ij, lp, grid, block, c->stream);
+        else launch_search<3>(a, is_ij, lp, grid, block, c->stream);
         time_end(c);
         HIPCHK(c, hipGetLastError());
         if (defer) {

@@ -107,3 +107,39 @@ def test_gravity_pieces_direct_sum(n, leaf, prec, tol):
     r2 = (d * d).sum(axis=0) + np.eye(n)
     scale = (0.7 * f[ics.F_MASS][None, :] / r2 * (1 - np.eye(n))).sum(axis=1)
     assert (np.abs(out[ics.F_ACC:ics.F_ACC + 3] - acc) / scale).max() < tol
+
+
+@pytest.mark.parametrize("dim,periodic", [(3, 1), (3, 0), (2, 1), (1, 0)])
+@pytest.mark.parametrize("n", [7, 64, 65, 32768, 32769, 98304, 98305, 262143, 262144])
+def test_search_sets_by_size(n, dim, periodic):
+    """Neighbour sets at the sizes where the search changes its lanes per
+    particle, both predicates, exact against FP64 distances from a sample of
+    particles (the first, the last and random ones).  Small and large leaves."""
+    rng = np.random.default_rng([n, dim])
+    p = ics.default_params(dim)
+    p.update(periodic=periodic, leaf_particle_num=1 if n % 2 else 20, range_min=[0.0] * 3,
+             range_max=[1.0 if k < dim else 0.0 for k in range(3)])
+    f = ics.empty_fields(n)
+    x = rng.random((dim, n))
+    f[ics.F_POS:ics.F_POS + dim] = x
+    f[ics.F_MASS] = 1.0 / n
+    f[ics.F_DENS] = f[ics.F_ENE] = 1.0
+    # about 20 neighbours, radii within a factor of 1.5
+    h = {1: 10.0 / n, 2: (20 / np.pi / n) ** 0.5, 3: (15 / np.pi / n) ** (1 / 3)}[dim] * rng.uniform(0.8, 1.2, n)
+    h = np.minimum(h, 0.4)
+    c = sphgpu.Context(p, n)
+    c.upload(f)
+    c.build_tree()
+    pick = np.unique(np.concatenate([[0, n - 1], rng.integers(0, n, 60)]))
+    for is_ij in (0, 1):
+        cnt, lists = c.neighbor_sets(h, is_ij, cap=160)
+        for i in pick:
+            d = x[:, i:i + 1] - x
+            if periodic:
+                d = np.where(np.abs(d) <= np.abs(np.abs(d) - 1.0), d, d - np.sign(d))
+            r2 = d[0] * d[0]
+            for k in range(1, dim):
+                r2 = r2 + d[k] * d[k]
+            want = (np.sqrt(r2) < np.maximum(h[i], h)) & (r2 != 0.0) if is_ij else r2 < h[i] * h[i]
+            np.testing.assert_array_equal(np.sort(lists[i, :cnt[i]]), np.flatnonzero(want))
+    c.close()
