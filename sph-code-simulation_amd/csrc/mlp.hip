@@ -20,7 +20,7 @@ struct MLP {
     float *m = nullptr, *v = nullptr;   // Adam moments
     float *grad = nullptr;   // reduced gradient + loss
     float *gpart = nullptr, *lpart = nullptr;  // per-tile partials
-    int part_blocks = 0;
+    int part_blocks = 0, loss_blocks = 0;
     int step = 0;
     bool trained = false;
 };
@@ -132,6 +132,7 @@ __device__ void wave_gemm(const bf16_t *A, int lda, const bf16_t *Bt, int ldb, i
     for (int t = wave; t < (M / 16) * tn_count; t += nw) {
         const int tm = t / tn_count, tn = t % tn_count;
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
         for (int k0 = 0; k0 < K; k0 += 32) {
             const bf16x8 a = *reinterpret_cast<const bf16x8 *>(A + (tm * 16 + (lane & 15)) * lda + k0 + 8 * (lane >> 4));
             const bf16x8 b = *reinterpret_cast<const bf16x8 *>(Bt + (tn * 16 + (lane & 15)) * ldb + k0 + 8 * (lane >> 4));
@@ -141,7 +142,15 @@ __device__ void wave_gemm(const bf16_t *A, int lda, const bf16_t *Bt, int ldb, i
     }
 }
 
-__global__ __launch_bounds__(256) void k_mlp_fwd_bwd(const float *__restrict__ rows, long long n_rows, long long row0,
+// 16 wavefronts: a batch of 1024 rows is 16 workgroups, so its time is one
+// workgroup's chain of ten barrier-separated stages, and every stage (16 tiles
+// of 16x16, or 4096 elements) splits over them, with the 64-row sums unrolled.
+// 4 wavefronts and rolled sums took 25.2 us, 16 and rolled sums 22.0, this 11.9.
+constexpr int kTrainThreads = 1024;
+
+// kGrad = false: the loss only (the evaluation after training)
+template <bool kGrad>
+__global__ __launch_bounds__(kTrainThreads) void k_mlp_fwd_bwd(const float *__restrict__ rows, long long n_rows, long long row0,
                                                       long long batch, const float *__restrict__ w, float gamma,
                                                       float *__restrict__ gpart, float *__restrict__ lpart)
 {
@@ -149,11 +158,13 @@ __global__ __launch_bounds__(256) void k_mlp_fwd_bwd(const float *__restrict__ r
     const int tid = threadIdx.x;
     const long long base = row0 + (long long)blockIdx.x * kTile;
     // parameters -> LDS (bf16 copies for the MFMA operands)
-    for (int e = tid; e < kMlpH * kK1; e += blockDim.x) {
+#pragma unroll
+    for (int e = tid; e < kMlpH * kK1; e += kTrainThreads) {
         const int o = e / kK1, k = e % kK1;
         L.W1[o][k] = (bf16_t)(k < kMlpIn ? w[kOffW1 + o * kMlpIn + k] : 0.f);
     }
-    for (int e = tid; e < kMlpH * kMlpH; e += blockDim.x) {
+#pragma unroll
+    for (int e = tid; e < kMlpH * kMlpH; e += kTrainThreads) {
         const int o = e / kMlpH, k = e % kMlpH;
         const bf16_t v2 = (bf16_t)w[kOffW2 + o * kMlpH + k];
         L.W2[o][k] = v2;
@@ -162,14 +173,17 @@ __global__ __launch_bounds__(256) void k_mlp_fwd_bwd(const float *__restrict__ r
         L.W3[o][k] = v3;
         L.W3T[k][o] = v3;
     }
-    if (tid < kMlpH) {
-        L.b1[tid] = w[kOffB1 + tid];
-        L.b2[tid] = w[kOffB2 + tid];
-        L.b3[tid] = w[kOffB3 + tid];
-        L.w4[tid] = w[kOffW4 + tid];
+    // the biases by the last wavefront but one, the rows' features by the last
+    if (tid >= kTrainThreads - 2 * kMlpH && tid < kTrainThreads - kMlpH) {
+        const int o = tid - (kTrainThreads - 2 * kMlpH);
+        L.b1[o] = w[kOffB1 + o];
+        L.b2[o] = w[kOffB2 + o];
+        L.b3[o] = w[kOffB3 + o];
+        L.w4[o] = w[kOffW4 + o];
     }
-    if (tid < kTile) {
-        const long long r = base + tid;
+    if (tid >= kTrainThreads - kTile) {
+        const int row = tid - (kTrainThreads - kTile);
+        const long long r = base + row;
         float x[6] = {0, 0, 0, 0, 0, 0};
         float y = 0.f, wt = 0.f;
         if (r < row0 + batch && r < n_rows) {
@@ -179,13 +193,14 @@ __global__ __launch_bounds__(256) void k_mlp_fwd_bwd(const float *__restrict__ r
             y = __logf(q[6] / p_m);
             wt = 1.f;
         }
+#pragma unroll
         for (int k = 0; k < kK1; ++k) {
             const bf16_t v = (bf16_t)(k < kMlpIn ? x[k] : 0.f);
-            L.X[tid][k] = v;
-            L.XT[k][tid] = v;
+            L.X[row][k] = v;
+            L.XT[k][row] = v;
         }
-        L.y[tid] = y;
-        L.wt[tid] = wt;
+        L.y[row] = y;
+        L.wt[row] = wt;
     }
     __syncthreads();
     // forward: z1 = X W1^T + b1, z2 = H1 W2^T + b2, z3 = H2 W3^T + b3
@@ -206,8 +221,25 @@ __global__ __launch_bounds__(256) void k_mlp_fwd_bwd(const float *__restrict__ r
     });
     __syncthreads();
     const float inv_b = 1.0f / (float)batch;
+    if (!kGrad) {
+        // squared errors, summed over the tile in row order
+        if (tid < kTile) {
+            float out = w[kOffB4];
+            for (int o = 0; o < kMlpH; ++o) out = __builtin_fmaf(L.w4[o], L.F[tid][o], out);
+            const float d = out - L.y[tid];
+            L.loss[tid] = L.wt[tid] * d * d;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            float ls = 0.f;
+            for (int r = 0; r < kTile; ++r) ls += L.loss[r];
+            lpart[blockIdx.x] = ls * inv_b;
+        }
+        return;
+    }
     if (tid < kTile) {
         float out = w[kOffB4];
+#pragma unroll
         for (int o = 0; o < kMlpH; ++o) out = __builtin_fmaf(L.w4[o], L.F[tid][o], out);
         const float d = out - L.y[tid];
         L.loss[tid] = L.wt[tid] * d * d;
@@ -216,22 +248,33 @@ __global__ __launch_bounds__(256) void k_mlp_fwd_bwd(const float *__restrict__ r
     __syncthreads();
     float *gp = gpart + (size_t)blockIdx.x * kMlpParams;
     // output layer: dw4 = sum dout relu(z3), db4 = sum dout; db3 = sum dz3
+    // (each sum by a wavefront of its own, in row order, its 64 rows unrolled so
+    // that their LDS reads are in flight together)
     if (tid < kMlpH) {
-        float s = 0.f, sb = 0.f;
-        for (int r = 0; r < kTile; ++r) {
-            s = __builtin_fmaf(L.dout[r], L.F[r][tid], s);
-            sb += (L.F[r][tid] > 0.f) ? L.dout[r] * L.w4[tid] : 0.f;
-        }
+        float s = 0.f;
+#pragma unroll
+        for (int r = 0; r < kTile; ++r) s = __builtin_fmaf(L.dout[r], L.F[r][tid], s);
         gp[kOffW4 + tid] = s;
-        gp[kOffB3 + tid] = sb;
-    }
-    if (tid == 0) {
-        float s = 0.f, ls = 0.f;
-        for (int r = 0; r < kTile; ++r) { s += L.dout[r]; ls += L.loss[r]; }
+    } else if (tid < 2 * kMlpH) {
+        const int o = tid - kMlpH;
+        const float w4 = L.w4[o];
+        float sb = 0.f;
+#pragma unroll
+        for (int r = 0; r < kTile; ++r) sb += (L.F[r][o] > 0.f) ? L.dout[r] * w4 : 0.f;
+        gp[kOffB3 + o] = sb;
+    } else if (tid == 2 * kMlpH) {
+        float s = 0.f;
+#pragma unroll
+        for (int r = 0; r < kTile; ++r) s += L.dout[r];
         gp[kOffB4] = s;
+    } else if (tid == 3 * kMlpH) {
+        float ls = 0.f;
+#pragma unroll
+        for (int r = 0; r < kTile; ++r) ls += L.loss[r];
         lpart[blockIdx.x] = ls * inv_b;
     }
-    for (int e = tid; e < kTile * kMlpH; e += blockDim.x) {
+#pragma unroll
+    for (int e = tid; e < kTile * kMlpH; e += kTrainThreads) {
         const int r = e / kMlpH, o = e % kMlpH;
         const float dz = (L.F[r][o] > 0.f) ? L.dout[r] * L.w4[o] : 0.f;
         const bf16_t v = (bf16_t)dz;
@@ -253,6 +296,7 @@ __global__ __launch_bounds__(256) void k_mlp_fwd_bwd(const float *__restrict__ r
     // db2 = sum dz2 ; dW2 = dZ2^T H1
     if (tid < kMlpH) {
         float s = 0.f;
+#pragma unroll
         for (int r = 0; r < kTile; ++r) s += L.F[r][tid];
         gp[kOffB2 + tid] = s;
     }
@@ -273,27 +317,55 @@ __global__ __launch_bounds__(256) void k_mlp_fwd_bwd(const float *__restrict__ r
     });
     if (tid < kMlpH) {
         float s = 0.f;
+#pragma unroll
         for (int r = 0; r < kTile; ++r) s += L.F[r][tid];
         gp[kOffB1 + tid] = s;
     }
 }
 
-// sum of the per-tile partial gradients in a fixed order (deterministic), then
-// optionally one Adam step on the FP32 master parameters
-__global__ void k_mlp_reduce_adam(const float *__restrict__ gpart, const float *__restrict__ lpart, int nblk,
-                                  float *__restrict__ grad, float *__restrict__ loss, float *__restrict__ w,
-                                  float *__restrict__ m, float *__restrict__ v, float lr, float b1c, float b2c,
-                                  int do_update)
+// Partial gradients of many tiles: each group of kRedTiles tiles is summed into
+// its first tile's block (thread p owns column p), so that the last sum runs
+// over tiles / kRedTiles blocks.  One chain over all tiles took 1 ms for 200k
+// rows (3125 tiles).
+constexpr int kRedTiles = 64;
+__global__ __launch_bounds__(256) void k_mlp_reduce_tiles(float *__restrict__ gpart, int nblk)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p == 0) {
-        float s = 0.f;
-        for (int b = 0; b < nblk; ++b) s += lpart[b];
-        *loss = s;
+    if (p >= kMlpParams) return;
+    const int b0 = blockIdx.y * kRedTiles, b1 = min(b0 + kRedTiles, nblk);
+    float g = 0.f;
+#pragma unroll 16
+    for (int b = b0; b < b1; ++b) g += gpart[(size_t)b * kMlpParams + p];
+    gpart[(size_t)b0 * kMlpParams + p] = g;
+}
+
+// loss of all tiles (one workgroup; FP64, fixed order)
+__global__ __launch_bounds__(256) void k_mlp_loss(const float *__restrict__ lpart, int nblk, float *__restrict__ loss)
+{
+    __shared__ double s[256];
+    double a = 0.0;
+    for (int b = threadIdx.x; b < nblk; b += 256) a += lpart[b];
+    s[threadIdx.x] = a;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if ((int)threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
+        __syncthreads();
     }
+    if (threadIdx.x == 0) *loss = (float)s[0];
+}
+
+// sum of the partial gradients (every stride-th block) in a fixed order
+// (deterministic), then optionally one Adam step on the FP32 master parameters
+__global__ __launch_bounds__(256) void k_mlp_reduce_adam(const float *__restrict__ gpart, int nblk, int stride,
+                                                         float *__restrict__ grad, float *__restrict__ w,
+                                                         float *__restrict__ m, float *__restrict__ v, float lr,
+                                                         float b1c, float b2c, int do_update)
+{
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= kMlpParams) return;
     float g = 0.f;
-    for (int b = 0; b < nblk; ++b) g += gpart[(size_t)b * kMlpParams + p];
+#pragma unroll 16
+    for (int b = 0; b < nblk; b += stride) g += gpart[(size_t)b * kMlpParams + p];
     grad[p] = g;
     if (!do_update) return;
     const float beta1 = 0.9f, beta2 = 0.999f, eps = 1e-8f;
@@ -373,25 +445,62 @@ int sphgpu_mlp_predict(sphgpu_ctx *c, const float *rows, int64_t n_rows, float *
     return 0;
 }
 
-// one pass of forward + backward over rows[row0, row0+batch) (device rows)
+// room for nblk tiles' partial results (the gradients only where wanted)
+static int mlp_parts(sphgpu_ctx *c, int nblk, bool grads)
+{
+    MLP *M = c->mlp;
+    if (nblk > M->loss_blocks) {
+        if (M->lpart) hipFree(M->lpart);
+        M->lpart = nullptr;
+        M->loss_blocks = 0;
+        HIPCHK(c, hipMalloc((void **)&M->lpart, sizeof(float) * (size_t)nblk));
+        M->loss_blocks = nblk;
+    }
+    if (grads && nblk > M->part_blocks) {
+        if (M->gpart) hipFree(M->gpart);
+        M->gpart = nullptr;
+        M->part_blocks = 0;
+        HIPCHK(c, hipMalloc((void **)&M->gpart, sizeof(float) * kMlpParams * (size_t)nblk));
+        M->part_blocks = nblk;
+    }
+    return 0;
+}
+
+// one pass of forward + backward over rows[row0, row0+batch) (device rows):
+// the gradient to dgrad, the loss to dloss when given, an Adam step on request
 static int mlp_pass(sphgpu_ctx *c, const float *drows, long long n_rows, long long row0, long long batch,
                     float *dgrad, float *dloss, bool update, float lr, int step)
 {
     MLP *M = c->mlp;
     const int nblk = (int)((batch + kTile - 1) / kTile);
-    if (nblk > M->part_blocks) {
-        if (M->gpart) hipFree(M->gpart);
-        if (M->lpart) hipFree(M->lpart);
-        M->part_blocks = nblk;
-        HIPCHK(c, hipMalloc((void **)&M->gpart, sizeof(float) * kMlpParams * (size_t)nblk));
-        HIPCHK(c, hipMalloc((void **)&M->lpart, sizeof(float) * (size_t)nblk));
-    }
-    hipLaunchKernelGGL(k_mlp_fwd_bwd, dim3(nblk), dim3(256), 0, c->stream, drows, n_rows, row0, batch,
+    const int rc = mlp_parts(c, nblk, true);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_mlp_fwd_bwd<true>, dim3(nblk), dim3(kTrainThreads), 0, c->stream, drows, n_rows, row0, batch,
                        (const float *)M->w, (float)c->prm.gamma, M->gpart, M->lpart);
+    if (dloss) hipLaunchKernelGGL(k_mlp_loss, dim3(1), dim3(256), 0, c->stream, (const float *)M->lpart, nblk, dloss);
+    int stride = 1;
+    if (nblk > kRedTiles) {
+        stride = kRedTiles;
+        hipLaunchKernelGGL(k_mlp_reduce_tiles, dim3(grid_for(kMlpParams, 256), grid_for(nblk, kRedTiles)), dim3(256), 0,
+                           c->stream, M->gpart, nblk);
+    }
     const float b1c = 1.f - std::pow(0.9f, (float)step), b2c = 1.f - std::pow(0.999f, (float)step);
     hipLaunchKernelGGL(k_mlp_reduce_adam, dim3(grid_for(kMlpParams, 256)), dim3(256), 0, c->stream,
-                       (const float *)M->gpart, (const float *)M->lpart, nblk, dgrad, dloss, M->w, M->m, M->v, lr,
-                       b1c, b2c, update ? 1 : 0);
+                       (const float *)M->gpart, nblk, stride, dgrad, M->w, M->m, M->v, lr, b1c, b2c, update ? 1 : 0);
+    HIPCHK(c, hipGetLastError());
+    return 0;
+}
+
+// the loss over all rows (forward only)
+static int mlp_loss(sphgpu_ctx *c, const float *drows, long long n_rows, float *dloss)
+{
+    MLP *M = c->mlp;
+    const int nblk = (int)((n_rows + kTile - 1) / kTile);
+    const int rc = mlp_parts(c, nblk, false);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_mlp_fwd_bwd<false>, dim3(nblk), dim3(kTrainThreads), 0, c->stream, drows, n_rows, 0ll, n_rows,
+                       (const float *)M->w, (float)c->prm.gamma, (float *)nullptr, M->lpart);
+    hipLaunchKernelGGL(k_mlp_loss, dim3(1), dim3(256), 0, c->stream, (const float *)M->lpart, nblk, dloss);
     HIPCHK(c, hipGetLastError());
     return 0;
 }
@@ -443,14 +552,14 @@ int sphgpu_mlp_train(sphgpu_ctx *c, const float *rows, int64_t n_rows, int epoch
         for (long long b = 0; b < nb && !rc; ++b) {
             const long long r0 = b * batch;
             const long long bs = std::min<long long>(batch, n_rows - r0);
-            rc = mlp_pass(c, d, n_rows, r0, bs, M->grad, M->grad + kMlpParams, true, lr, ++M->step);
+            rc = mlp_pass(c, d, n_rows, r0, bs, M->grad, nullptr, true, lr, ++M->step);
         }
     }
     M->trained = true;
     M->img_dirty = true;
     if (!rc && final_loss) {
         // loss over the whole set with the final parameters
-        rc = mlp_pass(c, d, n_rows, 0, n_rows, M->grad, M->grad + kMlpParams, false, 0.f, 1);
+        rc = mlp_loss(c, d, n_rows, M->grad + kMlpParams);
         HIPCHK(c, hipMemcpyAsync(final_loss, M->grad + kMlpParams, sizeof(float), hipMemcpyDeviceToHost, c->stream));
     }
     HIPCHK(c, hipStreamSynchronize(c->stream));

@@ -143,3 +143,31 @@ def test_search_sets_by_size(n, dim, periodic):
             want = (np.sqrt(r2) < np.maximum(h[i], h)) & (r2 != 0.0) if is_ij else r2 < h[i] * h[i]
             np.testing.assert_array_equal(np.sort(lists[i, :cnt[i]]), np.flatnonzero(want))
     c.close()
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 4096, 4097, 8192, 12353])
+def test_mlp_gradient_by_rows(n):
+    """Loss and gradient over n rows, at the edges of the 64-row tiles and of
+    the 64 tiles whose partial gradients one chain sums, against the FP64
+    reference: bf16 operands (2^-9 relative rounding each, three layers deep)
+    leave the gradient's direction within 1e-3 and its norm within 5e-2."""
+    import sys
+    from pathlib import Path
+    sys.path.insert(0, str(Path(__file__).resolve().parents[1] / "oracle"))
+    import mlp_oracle as M
+    rng = np.random.default_rng(n)
+    rows = np.stack([rng.normal(0, 0.5, n), rng.uniform(0.3, 3, n), 10 ** rng.uniform(-1, 0.5, n),
+                     rng.normal(0, 0.5, n), rng.uniform(0.3, 3, n), 10 ** rng.uniform(-1, 0.5, n),
+                     10 ** rng.uniform(-1, 0.5, n)], 1).astype(np.float32)
+    p, f = ics.sedov_3d(4)
+    c = sphgpu.Context(p, f.shape[1])
+    c.mlp_init(seed=3)
+    loss, grad = c.mlp_loss_grad(rows)
+    want_loss, want = M.loss_grad(c.mlp_get_params(), rows, p["gamma"])
+    assert abs(loss - want_loss) < 2e-2 * want_loss
+    assert grad @ want > 0.999 * np.linalg.norm(grad) * np.linalg.norm(want)
+    assert abs(np.linalg.norm(grad) / np.linalg.norm(want) - 1) < 5e-2
+    # the evaluation after training is the loss of the same rows (a rate of 0
+    # leaves the weights): the same tiles' losses, summed in FP64
+    assert abs(c.mlp_train(rows, 1, 1000, 0.0) - loss) <= 1e-6 * loss
+    c.close()
