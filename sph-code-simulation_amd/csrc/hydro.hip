@@ -136,11 +136,84 @@ SPH_DEV void wave_add_atomic(long long *stats, int slot, long long v)
     if ((threadIdx.x & (kWave - 1)) == 0) atomicAdd(stat_ptr(stats, slot), (unsigned long long)v);
 }
 
-template <int D, int K, int TYPE, typename T>
+// ---- four lanes per particle (small sets) --------------------------------------
+// The pair loops below have a form for small sets in which the four lanes of a
+// quad share a particle: each evaluates one candidate of every group of four,
+// and the terms are added in candidate order by all four lanes (quad
+// broadcasts), so every sum sees the additions of the one-lane form and the
+// results are the same bits.  What bounds them in small sets is the serial
+// chain of one lane's list (gathers and arithmetic of 30 to 130 candidates, more
+// than once) with most of the chip idle.
+template <int U> SPH_DEV float quad_get(float v)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), U * 0x55, 0xf, 0xf, true));
+}
+template <int U> SPH_DEV double quad_get(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)b, U * 0x55, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), U * 0x55, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// the terms x of the quad's lanes, in lane order (lanes without a term pass 0:
+// the sums start at +0, and adding +0 changes none of them)
+template <typename A, typename T> SPH_DEV void quad_add(A &acc, T x)
+{
+    acc.add(quad_get<0>(x));
+    acc.add(quad_get<1>(x));
+    acc.add(quad_get<2>(x));
+    acc.add(quad_get<3>(x));
+}
+template <typename T> SPH_DEV void quad_sum(T &acc, T x)
+{
+    acc += quad_get<0>(x);
+    acc += quad_get<1>(x);
+    acc += quad_get<2>(x);
+    acc += quad_get<3>(x);
+}
+template <typename T> SPH_DEV void quad_sub(T &acc, T x)
+{
+    acc -= quad_get<0>(x);
+    acc -= quad_get<1>(x);
+    acc -= quad_get<2>(x);
+    acc -= quad_get<3>(x);
+}
+// slots q0 .. q0 + 3 of a sum that folds before every slot 15 mod 16 (the force
+// loops); fold_here says that slot q0 + 3 is such a slot
+template <typename A, typename T> SPH_DEV void quad_add_fold(A &acc, T x, bool fold_here)
+{
+    acc.add(quad_get<0>(x));
+    acc.add(quad_get<1>(x));
+    acc.add(quad_get<2>(x));
+    if (fold_here) acc.fold();
+    acc.add(quad_get<3>(x));
+}
+SPH_DEV int quad_swap1(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true); }
+SPH_DEV int quad_swap2(int v) { return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xf, 0xf, true); }
+SPH_DEV int quad_or(int v)
+{
+    v |= quad_swap1(v);
+    return v | quad_swap2(v);
+}
+SPH_DEV int quad_count(int v)
+{
+    v += quad_swap1(v);
+    return v + quad_swap2(v);
+}
+// counts of the quad's lanes before this one
+SPH_DEV int quad_before(int v, int sub)
+{
+    const int o1 = quad_swap1(v), o2 = quad_swap2(v + o1);
+    return ((sub & 1) ? o1 : 0) + ((sub & 2) ? o2 : 0);
+}
+
+// LP lanes per particle: 1, or 4 (see above)
+template <int D, int K, int TYPE, typename T, int LP>
 __global__ __launch_bounds__(256) void k_pre(PreArgs<T> a)
 {
     typedef typename V4T<T>::type V4;
-    const int i0 = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const int t0 = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const int i0 = t0 / LP, sub = t0 % LP;
     const bool valid = i0 < a.n;
     const int i = valid ? i0 : a.n - 1;
     const V4 *__restrict__ RP = a.rv.r[R_POSH];
@@ -179,12 +252,54 @@ __global__ __launch_bounds__(256) void k_pre(PreArgs<T> a)
             // sums run in candidate order
             // (in the FP32 form the next group's positions and masses are
             // loaded one group ahead as well, its indices two ahead)
-            constexpr bool kAhead = sizeof(T) == 4;
             constexpr bool kMassW = !(TYPE == SPHGPU_DISPH || TYPE == SPHGPU_GDISPH);
             // equal masses: m_j is the common value (the record holds the same
             // rounded number), one record load per candidate instead of two
             const bool mload = kMassW && !a.mass_uniform;
             const T mu = kMassW ? T(a.mass_u) : T(1);
+            if constexpr (LP == 4) {
+                // one candidate per lane and group; the next group's record is
+                // loaded one group ahead, its index two ahead
+                V4 pn{};
+                T wn = mu;
+                int jn = 0;
+                if (nc > 0) {
+                    jn = a.idx[list_slot(i, min(sub, nc - 1), a.cap)];
+                    pn = RP[jn];
+                    if (mload) wn = rec_mass(RV, jn);
+                    jn = a.idx[list_slot(i, min(kGroup + sub, nc - 1), a.cap)];
+                }
+                for (int q0 = 0; q0 < nc; q0 += kGroup) {
+                    if ((q0 & 15) == 0) {
+                        dn.fold();
+                        ddn.fold();
+                    }
+                    const V4 pg = pn;
+                    const T wg = wn;
+                    if (q0 + kGroup < nc) {
+                        pn = RP[jn];
+                        if (mload) wn = rec_mass(RV, jn);
+                        jn = a.idx[list_slot(i, min(q0 + 2 * kGroup + sub, nc - 1), a.cap)];
+                    }
+                    T r2;
+                    if constexpr (sizeof(T) == 4) {
+                        r2 = T(0);
+#pragma unroll
+                        for (int k = 0; k < D; ++k) {
+                            const T dk = abs_rij_axis(xi[k], k == 0 ? pg.x : k == 1 ? pg.y : pg.z, a.box, k);
+                            r2 = (k == 0) ? dk * dk : r2 + dk * dk;
+                        }
+                    } else {
+                        T d[3];
+                        r2 = rec_r2<D, T>(pg, xi, a.box, d);
+                    }
+                    const T r = tsqrt(r2);
+                    const bool out = q0 + sub >= nc || r >= h;
+                    quad_add(dn, out ? T(0) : wg * Kern<D, K, T>::w(r, h));
+                    quad_add(ddn, out ? T(0) : wg * Kern<D, K, T>::dhw(r, h));
+                }
+            } else {
+            constexpr bool kAhead = sizeof(T) == 4;
             int jn[kGroup];
             V4 pn[kGroup];
             T wn[kGroup];
@@ -262,6 +377,7 @@ __global__ __launch_bounds__(256) void k_pre(PreArgs<T> a)
                     ddn.add(wg[u] * Kern<D, K, T>::dhw(r, h));
                 }
             }
+            }
             const T dens = dn.get(), ddens = ddn.get();
             const T f = dens * powh<D>(h) - b;
             const T df = ddens * powh<D>(h) + T(D) * dens * powh_m1<D>(h);
@@ -337,6 +453,148 @@ __global__ __launch_bounds__(256) void k_pre(PreArgs<T> a)
     const bool bal_on = kBal && (do_bal || a.td_av);
     const bool disph_w = (TYPE == SPHGPU_DISPH) || (TYPE == SPHGPU_GDISPH && !do_bal);
     T bdiv = T(0), brot[3] = {0, 0, 0};
+    if constexpr (LP == 4) {
+        int jn = 0, jc = 0;
+        V4 pn{};
+        bool selfseen = false;
+        if (nc > 0) {
+            jc = a.idx[list_slot(i, min(sub, nc - 1), a.cap)];
+            pn = RP[jc];
+            jn = a.idx[list_slot(i, min(kGroup + sub, nc - 1), a.cap)];
+        }
+        for (int q0 = 0; q0 < nc; q0 += kGroup) {
+            if ((q0 & 15) == 0) {
+                dens_a.fold(); dhd_a.fold(); n_a.fold(); pres_a.fold(); dhp_a.fold(); dhn_a.fold();
+            }
+            const int j = jc;
+            const V4 pg = pn;
+            if (q0 + kGroup < nc) {
+                jc = jn;
+                pn = RP[jn];
+                jn = a.idx[list_slot(i, min(q0 + 2 * kGroup + sub, nc - 1), a.cap)];
+            }
+            T d[3];
+            const T r2 = rec_r2<D, T>(pg, xi, a.box, d);
+            const bool memb = q0 + sub < nc && member(j, r2);
+            // this lane's terms, zero without a member
+            T t_dens = T(0), t_dhd = T(0), t_n = T(0), t_pres = T(0), t_dhp = T(0);
+            T t_gd[3] = {0, 0, 0}, t_gu[3] = {0, 0, 0}, t_gv[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+            T t_div = T(0), t_rot[3] = {0, 0, 0};
+            bool row = false;
+            if (memb) {
+                const V4 vj = RV[j], tj = RT[j];
+                const T mj = vj.w, uj = tj.w;
+                ++w;
+                if (fl) {
+                    if (j == i) {
+                        selfseen = true;
+                    } else {
+                        bool nz = r2 != T(0);
+                        if (sizeof(T) == 4 && !((float)r2 > z2)) nz = r2_64(a.x64, xi64, j, a.box, D) != 0.0;
+                        coincident = coincident || !nz;
+                        row = true;
+                    }
+                }
+                const T r = tsqrt(r2);
+                const T wk = Kern<D, K, T>::w(r, h);
+                t_dens = mj * wk;
+                if (TYPE == SPHGPU_DISPH || TYPE == SPHGPU_GDISPH) {
+                    const T dh = Kern<D, K, T>::dhw(r, h);
+                    t_n = wk;
+                    t_pres = mj * uj * wk;
+                    t_dhp = mj * uj * dh;
+                    t_dhd = dh;
+                } else if (TYPE == SPHGPU_SSPH) {
+                    t_dhd = mj * Kern<D, K, T>::dhw(r, h);
+                }
+                if (j != i) {
+                    const T vjv[3] = {vj.x, vj.y, vj.z};
+                    T dot = T(0);
+#pragma unroll
+                    for (int k = 0; k < D; ++k) dot = (k == 0) ? d[k] * (vi[k] - vjv[k]) : dot + d[k] * (vi[k] - vjv[k]);
+                    const T vs = ci + tj.z - tdiv(T(3.0) * dot, r);
+                    if (vs > vsig) vsig = vs;
+                    if ((kGrad && grad_on) || (kBal && bal_on)) {
+                        const T cw = Kern<D, K, T>::dwc(r, h);
+                        T dw[3];
+#pragma unroll
+                        for (int k = 0; k < D; ++k) dw[k] = d[k] * cw;
+                        if (kGrad && grad_on) {
+                            const T mdu = mj * (uj - ui);
+                            T mdv[3];
+#pragma unroll
+                            for (int b2 = 0; b2 < D; ++b2) mdv[b2] = mj * (vjv[b2] - vi[b2]);
+#pragma unroll
+                            for (int k = 0; k < D; ++k) {
+                                t_gd[k] = dw[k] * mj;
+                                t_gu[k] = dw[k] * mdu;
+#pragma unroll
+                                for (int b2 = 0; b2 < D; ++b2) t_gv[b2][k] = dw[k] * mdv[b2];
+                            }
+                        }
+                        if (kBal && bal_on) {
+                            T vij[3];
+#pragma unroll
+                            for (int k = 0; k < D; ++k) vij[k] = vi[k] - vjv[k];
+                            const T wt = disph_w ? mj * uj : mj;
+                            T bdot = T(0);
+#pragma unroll
+                            for (int k = 0; k < D; ++k) bdot = (k == 0) ? vij[k] * dw[k] : bdot + vij[k] * dw[k];
+                            t_div = wt * bdot;
+                            if (D == 3) {
+                                t_rot[0] = (vij[1] * dw[2 % D] - vij[2 % D] * dw[1 % D]) * wt;
+                                t_rot[1] = (vij[2 % D] * dw[0] - vij[0] * dw[2 % D]) * wt;
+                                t_rot[2] = (vij[0] * dw[1 % D] - vij[1 % D] * dw[0]) * wt;
+                            } else if (D == 2) {
+                                t_rot[0] = (vij[0] * dw[1 % D] - vij[1 % D] * dw[0]) * wt;
+                            }
+                        }
+                    }
+                }
+            }
+            quad_add(dens_a, t_dens);
+            if (TYPE == SPHGPU_DISPH || TYPE == SPHGPU_GDISPH) {
+                quad_add(n_a, t_n);
+                quad_add(pres_a, t_pres);
+                quad_add(dhp_a, t_dhp);
+                quad_add(dhn_a, t_dhd);
+            } else if (TYPE == SPHGPU_SSPH) {
+                quad_add(dhd_a, t_dhd);
+            }
+            if (kGrad && grad_on) {
+#pragma unroll
+                for (int k = 0; k < D; ++k) {
+                    quad_sum(gdd[k], t_gd[k]);
+                    quad_sum(gdu[k], t_gu[k]);
+#pragma unroll
+                    for (int b2 = 0; b2 < D; ++b2) quad_sum(gdv[b2][k], t_gv[b2][k]);
+                }
+            }
+            if (kBal && bal_on) {
+                quad_sub(bdiv, t_div);
+                quad_sum(brot[0], t_rot[0]);
+                if (D == 3) {
+                    quad_sum(brot[1], t_rot[1]);
+                    quad_sum(brot[2], t_rot[2]);
+                }
+            }
+            if (fl) {
+                // the force list's rows in candidate order
+                const int c = row ? 1 : 0;
+                const int q = nrow + quad_before(c, sub);
+                if (row && q < a.fl_cap) a.fl_idx[list_slot(i, q, a.fl_cap)] = j;
+                nrow += quad_count(c);
+            }
+        }
+        w = quad_count(w);
+        coincident = quad_or(coincident ? 1 : 0) != 0;
+        if (quad_or(selfseen ? 1 : 0)) qself = 0;
+        const T v0 = quad_get<0>(vsig), v1 = quad_get<1>(vsig), v2 = quad_get<2>(vsig), v3 = quad_get<3>(vsig);
+        vsig = v0;
+        if (v1 > vsig) vsig = v1;
+        if (v2 > vsig) vsig = v2;
+        if (v3 > vsig) vsig = v3;
+    } else {
     // (FP32 form: the next group's positions are loaded one group ahead and
     // its indices two ahead)
     constexpr bool kAheadP = sizeof(T) == 4;
@@ -488,6 +746,7 @@ __global__ __launch_bounds__(256) void k_pre(PreArgs<T> a)
         }
     }
     }
+    }
     const T dens = dens_a.get();
     const T gm1 = T(a.gamma - 1.0);
     T pres, gradh = T(0);
@@ -510,7 +769,8 @@ __global__ __launch_bounds__(256) void k_pre(PreArgs<T> a)
         am[b] = mb[b] & ~(((qself >> 6) == b) ? 1ull << (qself & 63) : 0ull);
         na_bits += __popcll(am[b]);
     }
-    if (valid) {
+    const bool writer = valid && sub == 0;
+    if (writer) {
         a.sml[i] = h64;
         a.dens[i] = (double)dens;
         a.pres[i] = (double)pres;
@@ -523,7 +783,7 @@ __global__ __launch_bounds__(256) void k_pre(PreArgs<T> a)
         if (TYPE != SPHGPU_GSPH) a.rec_w[R_AUX][4 * (size_t)i + 0] = gradh;
         if (a.posf_w) a.posf_w[4 * (size_t)i + 3] = (float)h;
         if (fl) {
-            const int na = fl_rows ? nrow : na_bits;
+            const int na = (LP > 1 || fl_rows) ? nrow : na_bits;
             a.fl_cnt_a[i] = min(na, a.fl_cap);
             a.fl_cnt[i] = min(na, a.fl_cap);
             // complete only when every j with r < h_i was a candidate
@@ -537,15 +797,15 @@ __global__ __launch_bounds__(256) void k_pre(PreArgs<T> a)
         }
     }
     wave_min_atomic(a.hvs_min, valid ? (double)(h / vsig) : 1.7976931348623157e308);
-    wave_add_atomic(a.stats, 1, valid ? newton_iters : 0);
-    wave_add_atomic(a.stats, 2, valid ? newton_fail : 0);
-    if (!valid) return;
+    wave_add_atomic(a.stats, 1, writer ? newton_iters : 0);
+    wave_add_atomic(a.stats, 2, writer ? newton_fail : 0);
+    if (!writer) return;
 
     // The member sums (density, v_sig, MUSCL gradients, Balsara / AV) were
     // taken in the density pass; what is left is writing the force-list rows
     // (row r of every lane = its r-th member, from the member bits, so a
     // store covers one 256-byte row) and finishing the sums.
-    bool rows_pending = fl && !fl_rows;
+    bool rows_pending = LP == 1 && fl && !fl_rows;
 
     if (kGrad && grad_on) {
         // MUSCL gradients (summed in the density pass)
@@ -667,10 +927,16 @@ struct FlistArgs {
     double *dscal;
 };
 
+// The lanes of a quad take every fourth entry, four of them at a time (the
+// appends are atomic and ordered later, so the split changes nothing).  Bound
+// by the gathers of the neighbours' records; one lane per particle took 231 us
+// at 1M (Sedov, now 190; Evrard 88, now 89), 105 at 104k (36), 26 at 65k in 2D (13).
 template <int D, bool FP64>
 __global__ __launch_bounds__(256) void k_flist_scatter(FlistArgs a)
 {
-    const int i = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    constexpr int LP = 4;
+    const int t0 = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const int i = t0 / LP, sub = t0 % LP;
     if (i >= a.n) return;
     const int na = a.cnt_a[i];
     const float4 pi = a.posf[i];
@@ -681,11 +947,12 @@ __global__ __launch_bounds__(256) void k_flist_scatter(FlistArgs a)
     const float xf[3] = {pi.x, pi.y, pi.z};
     const float mk = fp32_margin_k(a.root, D);
     // members in groups of kGroup, each group's loads issued together
-    for (int q0 = 0; q0 < na; q0 += kGroup) {
+    for (int q0 = sub; q0 < na; q0 += LP * kGroup) {
     int jg[kGroup];
     float4 pg[kGroup];
     double hg[kGroup];
-    list_group(a.idx, i, q0, na, a.cap, jg);
+#pragma unroll
+    for (int u = 0; u < kGroup; ++u) jg[u] = a.idx[list_slot(i, min(q0 + LP * u, na - 1), a.cap)];
 #pragma unroll
     for (int u = 0; u < kGroup; ++u) pg[u] = a.posf[jg[u]];
     // FP32 rounding is monotone: rounded values that differ order h_i and
@@ -696,7 +963,7 @@ __global__ __launch_bounds__(256) void k_flist_scatter(FlistArgs a)
         hg[u] = (FP64 ? pg[u].w <= pi.w : pg[u].w == pi.w) ? a.sml[jg[u]] : 0.0;
 #pragma unroll
     for (int u = 0; u < kGroup; ++u) {
-        if (q0 + u >= na) break;
+        if (q0 + LP * u >= na) break;
         const int j = jg[u];
         const float4 pj = pg[u];
         // h_j > h_i: r < h_i <= h_j puts i in the list of j already
@@ -942,12 +1209,17 @@ SPH_DEV void pair_states(bool second, T gamma, T dt, const T d[3], T r, const T 
     left[3] = tsqrt(gamma * left[2] / left[1]);
 }
 
+// One quad per particle at every size: 1M Evrard 192 -> 152 us, 160k 2D DISPH
+// 72 -> 55, 16k SSPH FP64 79 -> 28 against one lane per particle (the pair loop
+// is a quarter as long and four times the wavefronts hide its gathers).
 template <int D, int K, int TYPE, typename T>
 __global__ __launch_bounds__(256) void k_force_sph(ForceArgs<T> a)
 {
+    constexpr int LP = 4;
     if (a.skip_if && (a.skip_if[0] | a.skip_if[2])) return;  // whole grid
     typedef typename V4T<T>::type V4;
-    const int i = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const int t0 = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const int i = t0 / LP, sub = t0 % LP;
     if (i >= a.n) return;
     const V4 *__restrict__ RP = a.rv.r[R_POSH];
     const V4 *__restrict__ RV = a.rv.r[R_VELM];
@@ -984,22 +1256,18 @@ __global__ __launch_bounds__(256) void k_force_sph(ForceArgs<T> a)
     // next pair's four records are loaded one pair ahead too and the index
     // two ahead
     constexpr bool kAhead = sizeof(T) == 4;
-    int j_next = nc > 0 ? a.idx[list_slot(i, 0, a.cap)] : 0;
+    int j_next = sub < nc ? a.idx[list_slot(i, sub, a.cap)] : 0;
     V4 n_p{}, n_v{}, n_t{}, n_a{};
     int j_after = 0;
-    if (kAhead && nc > 0) {
+    if (kAhead && sub < nc) {
         n_p = RP[j_next];
         n_v = RV[j_next];
         n_t = RT[j_next];
         n_a = RA[j_next];
-        if (nc > 1) j_after = a.idx[list_slot(i, 1, a.cap)];
+        if (sub + LP < nc) j_after = a.idx[list_slot(i, sub + LP, a.cap)];
     }
-    for (int q = 0; q < nc; ++q) {
-        if ((q & 15) == 15) {
-#pragma unroll
-            for (int k = 0; k < D; ++k) ac[k].fold();
-            de.fold();
-        }
+    for (int q0 = 0; q0 < nc; q0 += LP) {
+        const int q = q0 + sub;
         const int j = j_next;
         V4 pj, vj, tj, aj;
         if (kAhead) {
@@ -1007,16 +1275,16 @@ __global__ __launch_bounds__(256) void k_force_sph(ForceArgs<T> a)
             vj = n_v;
             tj = n_t;
             aj = n_a;
-            if (q + 1 < nc) {
+            if (q + LP < nc) {
                 j_next = j_after;
                 n_p = RP[j_next];
                 n_v = RV[j_next];
                 n_t = RT[j_next];
                 n_a = RA[j_next];
-                if (q + 2 < nc) j_after = a.idx[list_slot(i, q + 2, a.cap)];
+                if (q + 2 * LP < nc) j_after = a.idx[list_slot(i, q + 2 * LP, a.cap)];
             }
         } else {
-            if (q + 1 < nc) j_next = a.idx[list_slot(i, q + 1, a.cap)];
+            if (q + LP < nc) j_next = a.idx[list_slot(i, q + LP, a.cap)];
             pj = RP[j];
             vj = RV[j];
             tj = RT[j];
@@ -1108,10 +1376,12 @@ __global__ __launch_bounds__(256) void k_force_sph(ForceArgs<T> a)
             s2 = mj * (g2u_i * u_per_pres_j * f_ji * pst_j + T(0.5) * pi_ij);
             e1 = mj * g2upp_i * uj * f_ij * pst_i * vdwi + T(0.5) * mj * pi_ij * vdwij + dene_ac;
         }
+        const bool act = q < nc, fold_here = (q0 & 15) == 12 && q0 + 3 < nc;
 #pragma unroll
-        for (int k = 0; k < D; ++k) ac[k].add(-(dwi[k] * s1 + dwj[k] * s2));
-        de.add(e1);
+        for (int k = 0; k < D; ++k) quad_add_fold(ac[k], act ? -(dwi[k] * s1 + dwj[k] * s2) : T(0), fold_here);
+        quad_add_fold(de, act ? e1 : T(0), fold_here);
     }
+    if (sub) return;
 #pragma unroll
     for (int k = 0; k < D; ++k) a.acc[k][i] = (double)ac[k].get();
     a.dene[i] = (double)de.get();
@@ -1219,8 +1489,11 @@ SPH_DEV int solve_pair(const T l[4], const T r[4], T gamma, int refine64, const 
 // The pair-slot loop of the GSPH force.  Slot q holds each lane's q-th pair;
 // the reconstruction and the force run per lane, the learned guess (when
 // enabled) runs for the whole wavefront on MFMA between them.
-template <int D, int K, typename T, int SOLVER, bool LEARNED>
-SPH_DEV void force_gsph_slots(const ForceArgs<T> &a, int i, int nc, int nmax, const T xi[3], const T vi[3],
+// With LP = 4 lanes per particle slot q0 + sub is lane sub's, and the folds of
+// the sums follow those of the 64-particle wavefront of the one-lane form
+// (nfold: its longest list).
+template <int D, int K, typename T, int SOLVER, bool LEARNED, int LP>
+SPH_DEV void force_gsph_slots(const ForceArgs<T> &a, int i, int sub, int nc, int nmax, int nfold, const T xi[3], const T vi[3],
                               const T gdi[3], const T gpi[3], const T gvi[3][3], T hi, T rhoi, T presi, T ci,
                               T gamma, T rho2_inv_i, T dt, BlockAcc<T> ac[3], BlockAcc<T> &de, const MlpWeightsBF16 *wl,
                               MlpWaveLDS *wsc, bool valid)
@@ -1229,28 +1502,30 @@ SPH_DEV void force_gsph_slots(const ForceArgs<T> &a, int i, int nc, int nmax, co
     const V4 *__restrict__ RP = a.rv.r[R_POSH];
     const V4 *__restrict__ RV = a.rv.r[R_VELM];
     const V4 *__restrict__ RT = a.rv.r[R_THERMO];
-    long long iters = 0, wave_max_sum = 0, calls = 0, fallbacks = 0, learned = 0;
+    // (32-bit: at most 24 iterations for each of a list's pairs)
+    int iters = 0, wave_max_sum = 0, calls = 0, fallbacks = 0, learned = 0;
     // The next slot's pair index is loaded one slot ahead, so its record
     // gathers do not wait for it; in the FP32 form the next slot's records
     // are loaded one slot ahead too (the slot's arithmetic covers their
     // latency), and the index two slots ahead.
     constexpr bool kAhead = sizeof(T) == 4;
     const T ihi = tdiv(T(1.0), hi);
-    int j_next = nc > 0 ? a.idx[list_slot(i, 0, a.cap)] : 0;
+    int j_next = sub < nc ? a.idx[list_slot(i, sub, a.cap)] : 0;
     V4 n_p{}, n_v{}, n_t{}, n_g[4] = {};
     int j_after = 0;
-    if (kAhead && nc > 0) {
+    if (kAhead && sub < nc) {
         n_p = RP[j_next];
         n_v = RV[j_next];
         n_t = RT[j_next];
         if (a.gsph2)
 #pragma unroll
             for (int b = 0; b < 4; ++b) n_g[b] = a.rv.r[R_G0 + b][j_next];
-        if (nc > 1) j_after = a.idx[list_slot(i, 1, a.cap)];
+        if (sub + LP < nc) j_after = a.idx[list_slot(i, sub + LP, a.cap)];
     }
-    for (int q = 0; q < nmax; ++q) {
+    for (int q0 = 0; q0 < nmax; q0 += LP) {
+        const int q = q0 + sub;
         // the sums are compensated in blocks of 16 slots
-        if ((q & 15) == 15) {
+        if (LP == 1 && (q & 15) == 15) {
 #pragma unroll
             for (int k = 0; k < D; ++k) ac[k].fold();
             de.fold();
@@ -1266,7 +1541,7 @@ SPH_DEV void force_gsph_slots(const ForceArgs<T> &a, int i, int nc, int nmax, co
             c_t = n_t;
 #pragma unroll
             for (int b = 0; b < 4; ++b) c_g[b] = n_g[b];
-            if (q + 1 < nc) {
+            if (q + LP < nc) {
                 j_next = j_after;
                 n_p = RP[j_next];
                 n_v = RV[j_next];
@@ -1274,10 +1549,10 @@ SPH_DEV void force_gsph_slots(const ForceArgs<T> &a, int i, int nc, int nmax, co
                 if (a.gsph2)
 #pragma unroll
                     for (int b = 0; b < 4; ++b) n_g[b] = a.rv.r[R_G0 + b][j_next];
-                if (q + 2 < nc) j_after = a.idx[list_slot(i, q + 2, a.cap)];
+                if (q + 2 * LP < nc) j_after = a.idx[list_slot(i, q + 2 * LP, a.cap)];
             }
-        } else if (q + 1 < nc) {
-            j_next = a.idx[list_slot(i, q + 1, a.cap)];
+        } else if (q + LP < nc) {
+            j_next = a.idx[list_slot(i, q + LP, a.cap)];
         }
         T d[3] = {0, 0, 0}, e[3] = {0, 0, 0}, r = T(1), r_inv = T(1);
         T left[4] = {0, 1, 1, 1}, right[4] = {0, 1, 1, 1};
@@ -1386,6 +1661,7 @@ SPH_DEV void force_gsph_slots(const ForceArgs<T> &a, int i, int nc, int nmax, co
                 }
             }
         }
+        T t_ac[3] = {0, 0, 0}, t_de = T(0);  // this slot's terms (LP > 1)
         if (act) {
             T pstar, vstar;
             int fb = 0;
@@ -1421,11 +1697,19 @@ SPH_DEV void force_gsph_slots(const ForceArgs<T> &a, int i, int nc, int nmax, co
 #pragma unroll
             for (int k = 0; k < D; ++k) {
                 const T f = d[k] * cwi * s1 + d[k] * cwj * s2;
-                ac[k].add(-f);
+                if (LP == 1) ac[k].add(-f);
+                else t_ac[k] = -f;
                 const T dvk = e[k] * vstar - vi[k];
                 fv = (k == 0) ? f * dvk : fv + f * dvk;
             }
-            de.add(-fv);
+            if (LP == 1) de.add(-fv);
+            else t_de = -fv;
+        }
+        if (LP > 1) {
+            const bool fold_here = (q0 & 15) == 12 && q0 + 3 < nfold;
+#pragma unroll
+            for (int k = 0; k < D; ++k) quad_add_fold(ac[k], t_ac[k], fold_here);
+            quad_add_fold(de, t_de, fold_here);
         }
         if (SOLVER == SPHGPU_RIEMANN_ITERATIVE) {
             iters += it;
@@ -1440,7 +1724,16 @@ SPH_DEV void force_gsph_slots(const ForceArgs<T> &a, int i, int nc, int nmax, co
             wave_max_sum += m;
         }
     }
-    wave_add_atomic(a.stats, 3, valid ? nc : 0);
+    if (LP > 1) {
+        // a fold that the one-lane form reaches behind this wavefront's end
+        const int end = (nmax + LP - 1) / LP * LP;
+        if ((end | 15) < nfold) {
+#pragma unroll
+            for (int k = 0; k < D; ++k) ac[k].fold();
+            de.fold();
+        }
+    }
+    wave_add_atomic(a.stats, 3, valid && sub == 0 ? nc : 0);
     if (SOLVER == SPHGPU_RIEMANN_ITERATIVE) {
         wave_add_atomic(a.stats, 5, iters);
         if ((threadIdx.x & (kWave - 1)) == 0) atomicAdd(stat_ptr(a.stats, 6), (unsigned long long)wave_max_sum);
@@ -1450,11 +1743,12 @@ SPH_DEV void force_gsph_slots(const ForceArgs<T> &a, int i, int nc, int nmax, co
     }
 }
 
-template <int D, int K, typename T, int SOLVER, int LEARNED>
+template <int D, int K, typename T, int SOLVER, int LEARNED, int LP>
 __global__ __launch_bounds__(256) void k_force_gsph(ForceArgs<T> a)
 {
     if (a.skip_if && (a.skip_if[0] | a.skip_if[2])) return;  // whole grid
-    const int i0 = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const int t0 = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const int i0 = t0 / LP, sub = t0 % LP;
     const bool valid = i0 < a.n;
     const int i = valid ? i0 : a.n - 1;
     typedef typename V4T<T>::type V4;
@@ -1486,17 +1780,28 @@ __global__ __launch_bounds__(256) void k_force_gsph(ForceArgs<T> a)
         const int o = __shfl_xor(nmax, off, kWave);
         nmax = o > nmax ? o : nmax;
     }
+    int nfold = nmax;
+    if (LP > 1) {
+        // the longest list of the particle's block of 64 (a wavefront's
+        // particles lie in one block)
+        const int b = (i & ~(kWave - 1)) + (threadIdx.x & (kWave - 1));
+        nfold = b < a.n ? a.cnt[b] : 0;
+        for (int off = kWave / 2; off > 0; off >>= 1) {
+            const int o = __shfl_xor(nfold, off, kWave);
+            nfold = o > nfold ? o : nfold;
+        }
+    }
     if constexpr (LEARNED) {
         // the network's bf16 image is read from global memory (L2-resident);
         // LDS holds each wavefront's activation tiles
         __shared__ MlpWaveLDS wsc[4];
-        force_gsph_slots<D, K, T, SOLVER, true>(a, i, nc, nmax, xi, vi, gdi, gpi, gvi, hi, rhoi, presi, ci, gamma,
+        force_gsph_slots<D, K, T, SOLVER, true, LP>(a, i, sub, nc, nmax, nfold, xi, vi, gdi, gpi, gvi, hi, rhoi, presi, ci, gamma,
                                                rho2_inv_i, dt, ac, de, a.mlp.img, &wsc[(threadIdx.x >> 6) & 3], valid);
     } else {
-        force_gsph_slots<D, K, T, SOLVER, false>(a, i, nc, nmax, xi, vi, gdi, gpi, gvi, hi, rhoi, presi, ci, gamma,
+        force_gsph_slots<D, K, T, SOLVER, false, LP>(a, i, sub, nc, nmax, nfold, xi, vi, gdi, gpi, gvi, hi, rhoi, presi, ci, gamma,
                                                 rho2_inv_i, dt, ac, de, nullptr, nullptr, valid);
     }
-    if (valid) {
+    if (valid && sub == 0) {
 #pragma unroll
         for (int k = 0; k < D; ++k) a.acc[k][i] = (double)ac[k].get();
         a.dene[i] = (double)de.get();
@@ -1556,6 +1861,18 @@ __global__ __launch_bounds__(256) void k_riemann_batch_learned(int n, const doub
 }
 
 // ---------------------------------------------------------------------------------
+// Particles up to which a pair loop runs with a quad per particle.  The quad
+// form has a quarter of the serial chain and four times the wavefronts (one
+// lane per particle fills the chip from about 200k particles on), but repeats
+// the additions in four lanes.  Measured (us, one lane / quad):
+//   PreInteraction FP32: 4k FP64 83 / 29, 65k 2D 142 / 79, 104k 234 / 153,
+//     133k 173 / 185, 185k 148 / 179, 1M 684 / 811
+//   PreInteraction FP64: 16k 289 / 96, 262k 489 / 394, 1M 1419 / 1476
+//   GSPH force FP32: 104k 399 / 177, 133k 195 / 159, 185k 214 / 205, 262k 257 /
+//     272, 512k 479 / 525, 1M 1029 / 998
+//   GSPH force FP64: 4k 67 / 23, 262k 785 / 599, 1M 2317 / 2209: always a quad
+constexpr int kQuadPre32 = 131072, kQuadPre64 = 524288, kQuadGsph32 = 196608;
+
 template <int D, int K, int TYPE, typename T> void launch_pre(sphgpu_ctx *c)
 {
     PreArgs<T> a;
@@ -1603,7 +1920,10 @@ template <int D, int K, int TYPE, typename T> void launch_pre(sphgpu_ctx *c)
     a.tight = c->pre_rscale < 1.0 && c->prm.iterative_sml;
     a.pre_flag = c->dflag;
     a.alpha_in = c->alpha_snap_on ? c->alpha_snap : nullptr;
-    hipLaunchKernelGGL((k_pre<D, K, TYPE, T>), dim3(grid_for(c->n, 256)), dim3(256), 0, c->stream, a);
+    if (c->n <= (sizeof(T) == 8 ? kQuadPre64 : kQuadPre32))
+        hipLaunchKernelGGL((k_pre<D, K, TYPE, T, 4>), dim3(grid_for(4ll * c->n, 256)), dim3(256), 0, c->stream, a);
+    else
+        hipLaunchKernelGGL((k_pre<D, K, TYPE, T, 1>), dim3(grid_for(c->n, 256)), dim3(256), 0, c->stream, a);
 }
 
 template <int D> void launch_flist(sphgpu_ctx *c)
@@ -1628,8 +1948,9 @@ template <int D> void launch_flist(sphgpu_ctx *c)
     a.dscal = c->dscal;
     const dim3 g(grid_for(c->n, 256)), b(256);
     time_begin(c, "force_lists");
-    if (c->prm.pair_precision == SPHGPU_PAIR_FP64) hipLaunchKernelGGL((k_flist_scatter<D, true>), g, b, 0, c->stream, a);
-    else hipLaunchKernelGGL((k_flist_scatter<D, false>), g, b, 0, c->stream, a);
+    const dim3 g4(grid_for(4ll * c->n, 256));
+    if (c->prm.pair_precision == SPHGPU_PAIR_FP64) hipLaunchKernelGGL((k_flist_scatter<D, true>), g4, b, 0, c->stream, a);
+    else hipLaunchKernelGGL((k_flist_scatter<D, false>), g4, b, 0, c->stream, a);
     time_end(c);
     time_begin(c, "force_lists_order");
     hipLaunchKernelGGL(k_flist_order, g, b, 0, c->stream, a);
@@ -1728,23 +2049,34 @@ template <typename T> ForceArgs<T> force_args(sphgpu_ctx *c)
     return a;
 }
 
+template <int D, int K, typename T, int LP> void launch_force_gsph(sphgpu_ctx *c, const ForceArgs<T> &a)
+{
+    const dim3 g(grid_for((long long)LP * c->n, 256)), b(256);
+    if (c->prm.riemann_solver == SPHGPU_RIEMANN_HLL)
+        hipLaunchKernelGGL((k_force_gsph<D, K, T, SPHGPU_RIEMANN_HLL, 0, LP>), g, b, 0, c->stream, a);
+    else
+        // one kernel for both guesses (the network is off when a.mlp.w is
+        // null); this layout measured faster than a guess-free instantiation
+        hipLaunchKernelGGL((k_force_gsph<D, K, T, SPHGPU_RIEMANN_ITERATIVE, 1, LP>), g, b, 0, c->stream, a);
+}
+
 template <int D, int K, typename T> void launch_force(sphgpu_ctx *c, const int *skip_if)
 {
     ForceArgs<T> a = force_args<T>(c);
     a.skip_if = skip_if;
-    const dim3 g(grid_for(c->n, 256)), b(256);
+    const dim3 g4(grid_for(4ll * c->n, 256)), b(256);
     if (c->prm.sph_type == SPHGPU_SSPH) {
-        hipLaunchKernelGGL((k_force_sph<D, K, SPHGPU_SSPH, T>), g, b, 0, c->stream, a);
+        hipLaunchKernelGGL((k_force_sph<D, K, SPHGPU_SSPH, T>), g4, b, 0, c->stream, a);
     } else if (c->prm.sph_type == SPHGPU_DISPH) {
-        hipLaunchKernelGGL((k_force_sph<D, K, SPHGPU_DISPH, T>), g, b, 0, c->stream, a);
+        hipLaunchKernelGGL((k_force_sph<D, K, SPHGPU_DISPH, T>), g4, b, 0, c->stream, a);
     } else if (c->prm.sph_type == SPHGPU_GDISPH) {
-        hipLaunchKernelGGL((k_force_sph<D, K, SPHGPU_GDISPH, T>), g, b, 0, c->stream, a);
-    } else if (c->prm.riemann_solver == SPHGPU_RIEMANN_HLL) {
-        hipLaunchKernelGGL((k_force_gsph<D, K, T, SPHGPU_RIEMANN_HLL, 0>), g, b, 0, c->stream, a);
+        hipLaunchKernelGGL((k_force_sph<D, K, SPHGPU_GDISPH, T>), g4, b, 0, c->stream, a);
+    } else if constexpr (sizeof(T) == 8) {
+        launch_force_gsph<D, K, T, 4>(c, a);
+    } else if (c->n <= kQuadGsph32) {
+        launch_force_gsph<D, K, T, 4>(c, a);
     } else {
-        // one kernel for both guesses (the network is off when a.mlp.w is
-        // null); this layout measured faster than a guess-free instantiation
-        hipLaunchKernelGGL((k_force_gsph<D, K, T, SPHGPU_RIEMANN_ITERATIVE, 1>), g, b, 0, c->stream, a);
+        launch_force_gsph<D, K, T, 1>(c, a);
     }
 }
 

@@ -109,8 +109,8 @@ SPH_DEV int wave_scan_max(int v)
     return v;
 }
 // the value of lane ^ 1 and lane ^ 2 of the quad
-SPH_DEV int quad_xor1(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, false); }
-SPH_DEV int quad_xor2(int v) { return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xf, 0xf, false); }
+SPH_DEV int quad_xor1(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true); }
+SPH_DEV int quad_xor2(int v) { return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xf, 0xf, true); }
 
 // |minimum-image distance| along one axis in FP32: r^2 only needs |d|, and
 // |d| < L inside the box, so min(|d|, L - |d|) is the minimum image (the
