@@ -20,7 +20,7 @@
 // instead of once per lane.  The pair and monopole terms run in the pair
 // precision T with compensated sums taken in blocks of at most 16 terms.  The
 // node range is cut into pieces walked by different wavefronts; their sums are
-// added in node order in FP64.
+// added in a fixed order in FP64.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -88,10 +88,13 @@ template <typename T> struct GravArgs {
     double theta2, G;
     Box box;
     long long *stats;
-    // the walk in nseg pieces: piece s takes the nodes
-    // [n_nodes s / nseg, n_nodes (s + 1) / nseg) and writes its sums to
+    // the walk in 2 nside pieces: with c the node index of the wavefront's
+    // particles, pieces 2k and 2k + 1 take the nodes whose distance to c in
+    // pre-order is in [n_nodes k^2 / nside^2, n_nodes (k + 1)^2 / nside^2), to
+    // the right and to the left; piece s writes its sums to
     // part[(4 s + c) n + i], c = phi, a_x, a_y, a_z
-    int nseg;
+    int nside, ngroups;
+    const int *nbase;
     double *part;
 };
 
@@ -141,14 +144,16 @@ __global__ __launch_bounds__(256) void k_gravity(GravArgs<T> a)
     __shared__ GravStage<T> stage[4];
     GravStage<T> &st = stage[(threadIdx.x >> 6) & 3];
     const int lane = threadIdx.x & (kWave - 1);
-    // The pieces of a workgroup's particles are neighbours in the logical
-    // order, rotated by a hash of the workgroup: the piece with the particles'
-    // own surroundings is the heavy one, and any regular stride between the
-    // heavy pieces sends them to the same shader engines (two pieces at 1M
-    // particles: 5.1 ms at the same instruction count, against 3.4 ms).
-    const int block = xcd_block(blockIdx.x, gridDim.x);
-    const int group = block / a.nseg;
-    const int seg = (int)(((unsigned)block + (((unsigned)group * 0x9E3779B1u) >> 16)) % (unsigned)a.nseg);
+    // Workgroups are dispatched in order and round-robin over the XCDs: each XCD
+    // keeps one contiguous eighth of the particles and starts the pieces around
+    // the particles themselves, the heavy ones, before the far ones (heavy
+    // pieces that start last leave a long tail, and at a regular stride between
+    // light ones they all land on the same shader engines: two alternating
+    // halves took 5.1 ms at 1M particles at the instruction count of 3.4 ms).
+    const int gx = (a.ngroups + kNumXcd - 1) / kNumXcd;  // particle groups per XCD
+    const int kb = blockIdx.x / kNumXcd;
+    const int seg = kb / gx;
+    const int group = (blockIdx.x % kNumXcd) * gx + kb % gx;
     const int i0 = group * blockDim.x + threadIdx.x;
     if ((i0 & ~(kWave - 1)) >= a.n) return;  // whole wave beyond the particles
     const bool valid = i0 < a.n;
@@ -198,9 +203,14 @@ __global__ __launch_bounds__(256) void k_gravity(GravArgs<T> a)
         }
         return (g.l2 > a.theta2 * d2) || (d2 < g.l2);
     };
-    int node = (int)((long long)a.n_nodes * seg / a.nseg);
-    const int node_end = (int)((long long)a.n_nodes * (seg + 1) / a.nseg);
-    if (node > 0) {
+    const int mid = min((i0 & ~(kWave - 1)) + kWave / 2, a.n - 1);
+    const long long here = __builtin_amdgcn_readfirstlane(a.nbase[mid]);
+    const int k0 = seg >> 1;
+    const long long d0 = (long long)a.n_nodes * k0 * k0 / (a.nside * a.nside);
+    const long long d1 = (long long)a.n_nodes * (k0 + 1) * (k0 + 1) / (a.nside * a.nside);
+    int node = (int)((seg & 1) ? max(0ll, here - d1) : min((long long)a.n_nodes, here + d0));
+    const int node_end = (int)((seg & 1) ? max(0ll, here - d0) : min((long long)a.n_nodes, here + d1));
+    if (node > 0 && node < node_end) {
         // a later piece: a lane that accepts an ancestor of the first node has
         // that subtree in the ancestor's piece and resumes behind it
         int anc = 0;
@@ -335,7 +345,7 @@ __global__ __launch_bounds__(256) void k_gravity(GravArgs<T> a)
     if (lane == 0) atomicAdd(stat_ptr(a.stats, 10), (unsigned long long)inter);
 }
 
-// the pieces' sums in node order (FP64, deterministic), one thread per
+// the pieces' sums in a fixed order (FP64, deterministic), one thread per
 // particle and component
 __global__ void k_gravity_sum(int n, int nseg, const double *__restrict__ part, double *__restrict__ phi, double *ax,
                               double *ay, double *az)
@@ -350,23 +360,24 @@ __global__ void k_gravity_sum(int n, int nseg, const double *__restrict__ part, 
     else (c == 1 ? ax : c == 2 ? ay : az)[i] += s;
 }
 
-// Pieces of the walk.  One wavefront walks the tree for 64 particles, a serial
-// chain of a thousand node steps: 800 us for 14k particles, whose 224
-// wavefronts leave most of the chip idle.  The pre-order node range is
+// Pieces of the walk on each side of a wavefront's particles.  One wavefront
+// walks the tree for 64 particles, a serial chain of a thousand node steps: 800
+// us for 14k particles, whose 224 wavefronts leave most of the chip idle, and
+// in larger sets the last wavefronts leave a tail.  The pre-order node range is
 // therefore split until about kGravWaves wavefronts are there to be scheduled
-// (8 fit a SIMD, 8192 the chip; the pieces of a walk are very uneven, so
-// several times that).  Evrard, 14k particles: 801 us -> 103 (pieces capped at
-// 32: 167, at 64: 132); 200k: 1284 -> 1026 (20 pieces); 1M, bound by VALU issue:
-// 3452 -> 3368 (4 pieces).
+// (8 fit a SIMD, 8192 the chip).  Evrard, FP32: 14k particles 801 -> 117 us,
+// 200k 1284 -> 807 (with 16384 / 32768 / 131072 wavefronts 914 / 812 / 873), 1M
+// 3603 -> 2961 (3326 / 3251 / 2911); FP64: 14k 1565 -> 318, 278k 5156 -> 4270,
+// 606k 9380 -> 8293.
 constexpr int kGravWaves = 65536;
-constexpr int kGravSegMax = 128;
-int grav_pieces(int n, int n_nodes)
+constexpr int kGravSideMax = 64;
+int grav_sides(int n)
 {
     const int waves = (n + kWave - 1) / kWave;
-    return std::max(1, std::min({kGravWaves / waves, kGravSegMax, n_nodes}));
+    return std::max(1, std::min(kGravWaves / waves / 2, kGravSideMax));
 }
 
-template <typename T> void launch_gravity(sphgpu_ctx *c, int nseg)
+template <typename T> void launch_gravity(sphgpu_ctx *c, int nside)
 {
     GravArgs<T> a;
     a.n = c->n;
@@ -378,9 +389,11 @@ template <typename T> void launch_gravity(sphgpu_ctx *c, int nseg)
     a.G = c->prm.gravity_constant;
     a.box = c->box;
     a.stats = c->dstats;
-    a.nseg = nseg;
+    a.nside = nside;
+    a.ngroups = grid_for(c->n, 256);
+    a.nbase = c->tree.nbase;
     a.part = c->tree.gpart;
-    const dim3 g(grid_for(c->n, 256) * nseg), b(256);
+    const dim3 g((a.ngroups + kNumXcd - 1) / kNumXcd * kNumXcd * 2 * nside), b(256);
 #define LAUNCH(D)                                                                          \
     if (c->box.periodic) hipLaunchKernelGGL((k_gravity<D, T, true>), g, b, 0, c->stream, a); \
     else hipLaunchKernelGGL((k_gravity<D, T, false>), g, b, 0, c->stream, a);
@@ -412,7 +425,7 @@ int gravity(sphgpu_ctx *c)
     hipLaunchKernelGGL(k_grav_nodes, dim3(grid_for(t.n_nodes, 256)), dim3(256), 0, c->stream, t.n_nodes, t.node_cap,
                        t.com, t.edge, t.mass, t.start, t.end, t.skip, t.level, t.gnode);
     time_end(c);
-    const int nseg = grav_pieces(c->n, t.n_nodes);
+    const int nside = grav_sides(c->n), nseg = 2 * nside;
     if (nseg > t.gpart_seg) {
         if (t.gpart) hipFree(t.gpart);
         t.gpart = nullptr;
@@ -422,8 +435,8 @@ int gravity(sphgpu_ctx *c)
         t.gpart_seg = nseg;
     }
     time_begin(c, "gravity");
-    if (c->prm.pair_precision == SPHGPU_PAIR_FP64) launch_gravity<double>(c, nseg);
-    else launch_gravity<float>(c, nseg);
+    if (c->prm.pair_precision == SPHGPU_PAIR_FP64) launch_gravity<double>(c, nside);
+    else launch_gravity<float>(c, nside);
     hipLaunchKernelGGL(k_gravity_sum, dim3(grid_for(c->n, 256), c->dim + 1), dim3(256), 0, c->stream, c->n, nseg,
                        (const double *)t.gpart, c->sc[S_PHI], c->acc[0], c->acc[1], c->acc[2]);
     time_end(c);
