@@ -990,7 +990,8 @@ __global__ __launch_bounds__(256) void k_flist_scatter(FlistArgs a)
     }
 }
 
-constexpr int kRunSort = 16;
+constexpr int kRunSort = 16;         // entries sorted in one lane's registers
+constexpr int kRunWave = 4 * kWave;  // and by a whole wavefront
 
 __global__ __launch_bounds__(256) void k_flist_order(FlistArgs a)
 {
@@ -1004,11 +1005,11 @@ __global__ __launch_bounds__(256) void k_flist_order(FlistArgs a)
         __threadfence_system();
     }
     const int i = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    int nt = 0;
+    int nt = 0, na = 0, m = 0;
     if (i < a.n) {
-        const int na = a.cnt_a[i];
+        na = a.cnt_a[i];
         nt = min(a.cnt[i], a.cap);
-        const int m = nt - na;  // length of the appended run
+        m = nt - na;  // length of the appended run
         if (m > 1 && m <= kRunSort) {
             // short runs (the usual case): all loads issued together, an
             // odd-even transposition network in registers (kRunSort rounds
@@ -1029,8 +1030,8 @@ __global__ __launch_bounds__(256) void k_flist_order(FlistArgs a)
             for (int u = 0; u < kRunSort; ++u)
                 if (u < m) a.idx[list_slot(i, na + u, a.cap)] = v[u];
         }
-        // insertion sort of a longer appended run
-        for (int q = na + 1; m > kRunSort && q < nt; ++q) {
+        // insertion sort of a run longer than a wavefront holds
+        for (int q = na + 1; m > kRunWave && q < nt; ++q) {
             const int v = a.idx[list_slot(i, q, a.cap)];
             int p = q - 1;
             int u = a.idx[list_slot(i, p, a.cap)];
@@ -1042,6 +1043,38 @@ __global__ __launch_bounds__(256) void k_flist_order(FlistArgs a)
             a.idx[list_slot(i, p + 1, a.cap)] = v;
         }
         a.cnt[i] = nt;
+    }
+    // Longer runs, one after the other by the whole wavefront: each lane holds
+    // entries of the run (up to kRunWave of them) and its rank is the number of
+    // smaller ones (the entries of a run differ).  An insertion sort by the
+    // particle's own lane took 40 us for the runs of about 100 entries beside a
+    // density jump in 1D (now 17), 13 for 14k Evrard particles (7), 39 at 1M (24).
+    const int lane = threadIdx.x & (kWave - 1);
+    unsigned long long longer = __ballot(m > kRunSort && m <= kRunWave);
+    while (longer) {
+        const int o = __ffsll((long long)longer) - 1;
+        longer &= longer - 1;
+        const int io = __builtin_amdgcn_readlane(i, o), nao = __builtin_amdgcn_readlane(na, o);
+        const int mo = __builtin_amdgcn_readlane(m, o);
+        int v[kRunWave / kWave], rank[kRunWave / kWave];
+#pragma unroll
+        for (int u = 0; u < kRunWave / kWave; ++u) {
+            const int q = u * kWave + lane;
+            v[u] = q < mo ? a.idx[list_slot(io, nao + q, a.cap)] : INT_MAX;
+            rank[u] = 0;
+        }
+#pragma unroll
+        for (int w = 0; w < kRunWave / kWave; ++w) {
+            const int left = min(kWave, mo - w * kWave);
+            for (int k = 0; k < left; ++k) {
+                const int e = __builtin_amdgcn_readlane(v[w], k);
+#pragma unroll
+                for (int u = 0; u < kRunWave / kWave; ++u) rank[u] += e < v[u] ? 1 : 0;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kRunWave / kWave; ++u)
+            if (u * kWave + lane < mo) a.idx[list_slot(io, nao + rank[u], a.cap)] = v[u];
     }
     long long c = nt;
     for (int off = kWave / 2; off > 0; off >>= 1) c += __shfl_xor(c, off, kWave);

@@ -235,3 +235,46 @@ def test_quad_and_single_lane_forms_agree(limit, prec, over):
     assert np.isfinite(out[0]).all() and np.abs(out[0][ics.F_ACC]).max() > 0
     for row in range(out[0].shape[0]):
         np.testing.assert_array_equal(out[0][row], out[1][row], err_msg=f"field row {row}")
+
+
+@pytest.mark.parametrize("nn,reach", [(20, 0.0), (20, 0.15), (60, 0.35), (60, 0.6), (200, 0.9)])
+def test_force_list_runs_sorted(nn, reach):
+    """Force lists whose appended part (particles j with h_j > r >= h_i) is
+    short, of tens, of up to a few hundred entries (each sorted its own way): the
+    lists hold the exact pair sets, and two contexts agree bit for bit in the
+    forces whatever order the appends came in.  A sparse half with large h beside
+    a dense half gives the long runs; `reach` widens the sparse spacing."""
+    n_dense, n_sparse = 3000, 300
+    p = ics.default_params(1)
+    p.update(neighbor_number=nn, leaf_particle_num=4, gamma=1.4, pair_precision=ics.PAIR_FP32)
+    n = n_dense + n_sparse
+    f = ics.empty_fields(n)
+    rng = np.random.default_rng([nn, int(100 * reach)])
+    dx = 1.0 / n_dense
+    f[ics.F_POS] = np.concatenate([-(np.arange(n_dense) + 0.5) * dx, (np.arange(n_sparse) + 0.5) * dx * (1 + 20 * reach)])
+    f[ics.F_POS] += 0.1 * dx * rng.uniform(-1, 1, n)
+    f[ics.F_MASS] = dx
+    f[ics.F_DENS] = f[ics.F_ENE] = 1.0
+    f[ics.F_DENS, n_dense:] = 1.0 / (1 + 20 * reach)
+    f[ics.F_SOUND] = 1.0
+    runs = []
+    for _ in range(2):
+        c = sphgpu.Context(p, n)
+        c.upload(f)
+        c.build_tree()
+        for _ in range(4):
+            c.pre_interaction()
+        cnt, lists = c.neighbor_sets(None, 2, cap=4096)
+        c.fluid_force()
+        out = c.download()
+        c.close()
+        runs.append(out)
+    x, h = out[ics.F_POS], out[ics.F_SML]
+    tail = 0
+    for i in range(n_dense - 200, n, 3):
+        r = np.sqrt((x[i] - x) ** 2)
+        want = np.flatnonzero((r < np.maximum(h[i], h)) & (r != 0.0))
+        np.testing.assert_array_equal(np.sort(lists[i, :cnt[i]]), want)
+        tail = max(tail, int((r[want] >= h[i]).sum()))
+    print("longest appended run", tail)
+    np.testing.assert_array_equal(runs[0], runs[1])
