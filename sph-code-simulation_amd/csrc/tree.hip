@@ -48,70 +48,86 @@ struct TreeShape {
 };
 
 // ---- root geometry (src/bhtree.cpp:20-32 periodic, :67-103 bounding box) --
-__global__ void k_bbox_partial(const double *__restrict__ x, const double *__restrict__ y,
-                               const double *__restrict__ z, int n, int dim, double *__restrict__ part)
+// A workgroup's bounds from its threads': inside a wavefront by lane exchange,
+// the four wavefronts' through LDS (min and max are exact in any order).
+// Thread 0 gets the result.  All three axes are always taken (the caller
+// repeats axis 0 for missing ones): loops to a run-time dimension put the
+// bounds into scratch memory (29 us at 1M particles, now 9.4; 14k 10, now 4.5).
+__device__ __forceinline__ void block_bounds(double mn[3], double mx[3])
 {
-    __shared__ double smin[3][256], smax[3][256];
+    __shared__ double smin[4][3], smax[4][3];
+    for (int off = kWave / 2; off > 0; off >>= 1)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const double a = __shfl_xor(mn[k], off, kWave), b = __shfl_xor(mx[k], off, kWave);
+            mn[k] = a < mn[k] ? a : mn[k];
+            mx[k] = b > mx[k] ? b : mx[k];
+        }
+    const int w = threadIdx.x / kWave;
+    if ((threadIdx.x & (kWave - 1)) == 0)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            smin[w][k] = mn[k];
+            smax[w][k] = mx[k];
+        }
+    __syncthreads();
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int q = 1; q < 4; ++q)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                mn[k] = smin[q][k] < mn[k] ? smin[q][k] : mn[k];
+                mx[k] = smax[q][k] > mx[k] ? smax[q][k] : mx[k];
+            }
+}
+
+__global__ __launch_bounds__(256) void k_bbox_partial(const double *__restrict__ x, const double *__restrict__ y,
+                                                      const double *__restrict__ z, int n,
+                                                      double *__restrict__ part)
+{
     double mn[3] = {1.7976931348623157e308, 1.7976931348623157e308, 1.7976931348623157e308};
     double mx[3] = {-1.7976931348623157e308, -1.7976931348623157e308, -1.7976931348623157e308};
     const double *p[3] = {x, y, z};
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        for (int k = 0; k < dim; ++k) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
             const double v = p[k][i];
             mn[k] = v < mn[k] ? v : mn[k];
             mx[k] = v > mx[k] ? v : mx[k];
         }
     }
-    for (int k = 0; k < 3; ++k) { smin[k][threadIdx.x] = mn[k]; smax[k][threadIdx.x] = mx[k]; }
-    __syncthreads();
-    for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            for (int k = 0; k < 3; ++k) {
-                const double a = smin[k][threadIdx.x + s], b = smax[k][threadIdx.x + s];
-                if (a < smin[k][threadIdx.x]) smin[k][threadIdx.x] = a;
-                if (b > smax[k][threadIdx.x]) smax[k][threadIdx.x] = b;
-            }
-        }
-        __syncthreads();
-    }
+    block_bounds(mn, mx);
     if (threadIdx.x == 0)
+#pragma unroll
         for (int k = 0; k < 3; ++k) {
-            part[blockIdx.x * 6 + k] = smin[k][0];
-            part[blockIdx.x * 6 + 3 + k] = smax[k][0];
+            part[blockIdx.x * 6 + k] = mn[k];
+            part[blockIdx.x * 6 + 3 + k] = mx[k];
         }
 }
 
-// final bounds over the block partials: 256 threads, then a tree in LDS
-// (min and max are exact in any order)
+// final bounds over the block partials
 __global__ __launch_bounds__(256) void k_bbox_final(const double *__restrict__ part, int nblocks, int dim,
                                                     double *__restrict__ root)
 {
-    __shared__ double smin[3][256], smax[3][256];
     double mn[3] = {1.7976931348623157e308, 1.7976931348623157e308, 1.7976931348623157e308};
     double mx[3] = {-1.7976931348623157e308, -1.7976931348623157e308, -1.7976931348623157e308};
     for (int b = threadIdx.x; b < nblocks; b += blockDim.x)
+#pragma unroll
         for (int k = 0; k < 3; ++k) {
-            if (part[b * 6 + k] < mn[k]) mn[k] = part[b * 6 + k];
-            if (part[b * 6 + 3 + k] > mx[k]) mx[k] = part[b * 6 + 3 + k];
+            const double lo = part[b * 6 + k], hi = part[b * 6 + 3 + k];
+            mn[k] = lo < mn[k] ? lo : mn[k];
+            mx[k] = hi > mx[k] ? hi : mx[k];
         }
-    for (int k = 0; k < 3; ++k) { smin[k][threadIdx.x] = mn[k]; smax[k][threadIdx.x] = mx[k]; }
-    __syncthreads();
-    for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s)
-            for (int k = 0; k < 3; ++k) {
-                if (smin[k][threadIdx.x + s] < smin[k][threadIdx.x]) smin[k][threadIdx.x] = smin[k][threadIdx.x + s];
-                if (smax[k][threadIdx.x + s] > smax[k][threadIdx.x]) smax[k][threadIdx.x] = smax[k][threadIdx.x + s];
-            }
-        __syncthreads();
-    }
+    block_bounds(mn, mx);
     if (threadIdx.x != 0) return;
     double l = 0.0;
-    for (int k = 0; k < dim; ++k) {
-        root[k] = (smax[k][0] + smin[k][0]) * 0.5;
-        const double range = smax[k][0] - smin[k][0];
-        if (l < range) l = range;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const bool in = k < dim;
+        root[k] = in ? (mx[k] + mn[k]) * 0.5 : 0.0;
+        const double range = mx[k] - mn[k];
+        if (in && l < range) l = range;
     }
-    for (int k = dim; k < 3; ++k) root[k] = 0.0;
     root[3] = l;
 }
 
@@ -445,17 +461,17 @@ __global__ __launch_bounds__(kScatterThreads) void k_radix_scatter(
 
 // All passes of a small sort in one workgroup: at these sizes a pass of three
 // launches costs their latency alone (hist 4.3 us, scan 3.3, scatter 14.7 at
-// 4096 particles), so the elements go back and forth between the two buffers
-// inside one launch, 7 us a pass.  Element order, and with it the result, is
-// that of the tiled passes (both are stable).  One tile is the limit: at 14k
-// (four times the rounds of one CU) it took 25 us a pass, the tiled passes
-// take 16.  Ends in buffer a for an even number of passes, in b for an odd one.
+// 4096 particles), so all passes run in one launch with the elements going
+// through LDS between them (5 passes of 4096: 25 us).  Element order, and with it the result, is that of
+// the tiled passes (both are stable).  One tile is the limit: at 14k (four times
+// the rounds of one CU) a pass took 25 us, the tiled passes take 16.
 constexpr int kSmallMax = kSortTile;
 
-__global__ __launch_bounds__(kScatterThreads) void k_sort_small(unsigned long long *key_a, int *val_a,
-                                                                unsigned long long *key_b, int *val_b, int n,
-                                                                int passes)
+__global__ __launch_bounds__(kScatterThreads) void k_sort_small(unsigned long long *__restrict__ key, int *__restrict__ val,
+                                                                int n, int passes)
 {
+    __shared__ unsigned long long skey[kSmallMax];
+    __shared__ int sval[kSmallMax];
     __shared__ unsigned int wcnt[kScatterWaves][256];
     __shared__ unsigned int wtot[4];
     const int tid = threadIdx.x;
@@ -464,20 +480,18 @@ __global__ __launch_bounds__(kScatterThreads) void k_sort_small(unsigned long lo
     const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     const int items = (n + kScatterThreads - 1) / kScatterThreads;  // rounds per wave
     const int first = w * (kWave * items) + lane;
-    unsigned long long *kin = key_a, *kout = key_b;
-    int *vin = val_a, *vout = val_b;
+    unsigned long long k[kScatterItems];
+    int v[kScatterItems];
+    unsigned rank[kScatterItems];
+#pragma unroll
+    for (int r = 0; r < kScatterItems; ++r) {
+        const int e = first + r * kWave;
+        const bool in = r < items && e < n;
+        k[r] = in ? key[e] : ~0ull;
+        v[r] = in ? val[e] : 0;
+    }
     for (int p = 0; p < passes; ++p) {
         const int shift = 8 * p;
-        unsigned long long k[kScatterItems];
-        int v[kScatterItems];
-        unsigned rank[kScatterItems];
-#pragma unroll
-        for (int r = 0; r < kScatterItems; ++r) {
-            const int e = first + r * kWave;
-            const bool in = r < items && e < n;
-            k[r] = in ? kin[e] : ~0ull;
-            v[r] = in ? vin[e] : 0;
-        }
         for (int q = lane; q < 256; q += kWave) wcnt[w][q] = 0;
         sort_wave_fence();
 #pragma unroll
@@ -509,16 +523,26 @@ __global__ __launch_bounds__(kScatterThreads) void k_sort_small(unsigned long lo
         for (int r = 0; r < kScatterItems; ++r)
             if (r < items && first + r * kWave < n) {
                 const unsigned dst = wcnt[w][(unsigned)(k[r] >> shift) & 255u] + rank[r];
-                kout[dst] = k[r];
-                vout[dst] = v[r];
+                skey[dst] = k[r];
+                sval[dst] = v[r];
             }
-        __syncthreads();  // the next pass reads what the whole workgroup wrote
-        unsigned long long *tk = kin;
-        kin = kout;
-        kout = tk;
-        int *tv = vin;
-        vin = vout;
-        vout = tv;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kScatterItems; ++r) {
+            const int e = first + r * kWave;
+            if (r < items && e < n) {
+                k[r] = skey[e];
+                v[r] = sval[e];
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kScatterItems; ++r) {
+        const int e = first + r * kWave;
+        if (r < items && e < n) {
+            key[e] = k[r];
+            val[e] = v[r];
+        }
     }
 }
 
@@ -1128,7 +1152,7 @@ int tree_build(sphgpu_ctx *c)
     time_begin(c, "tree_keys");
     if (!c->prm.periodic) {
         const int nbb = std::min(c->red_blocks, grid_for(n, 256));
-        hipLaunchKernelGGL(k_bbox_partial, dim3(nbb), dim3(256), 0, c->stream, px, py, pz, n, c->dim, c->red);
+        hipLaunchKernelGGL(k_bbox_partial, dim3(nbb), dim3(256), 0, c->stream, px, py, pz, n, c->red);
         hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(256), 0, c->stream, (const double *)c->red, nbb, c->dim, t.root);
     }
     hipLaunchKernelGGL(k_keys, dim3(grid_for(n, 256)), dim3(256), 0, c->stream, px, py, pz, (const double *)t.root, sh,
@@ -1155,12 +1179,7 @@ int tree_build(sphgpu_ctx *c)
     // up to one tile of elements: all passes in one launch (k_sort_small)
     const bool small = n <= kSmallMax;
     if (small) {
-        hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(kScatterThreads), 0, c->stream, t.key, t.perm, t.key_alt, t.perm_alt,
-                           n, passes);
-        if (passes & 1) {
-            std::swap(t.key, t.key_alt);
-            std::swap(t.perm, t.perm_alt);
-        }
+        hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(kScatterThreads), 0, c->stream, t.key, t.perm, n, passes);
     }
     for (int p = skip; !small && p < passes; ++p) {
         const int shift = 8 * p;
