@@ -84,7 +84,6 @@ struct Tree {
     // nchild[k] = (offset into child, count); leaves have count 0
     int2 *nchild = nullptr;
     int *child = nullptr;
-    unsigned int *ccount = nullptr;   // child counts, scanned into offsets
     // hierarchy of block reductions over sorted particles (64 and 4096)
     double *bmax1 = nullptr, *bmax2 = nullptr;
     double *bsum1 = nullptr, *bsum2 = nullptr;  // [4][nb] : m, mx, my, mz
@@ -102,7 +101,8 @@ struct Tree {
     unsigned int *hist = nullptr;
     int hist_blocks = 0;
     // node count and the partial-sort check, read together by the host
-    int *sync_words = nullptr;         // [0] node count, [1] prefix run > leaf
+    int *sync_words = nullptr;         // [0] node count, [1] prefix run > leaf,
+                                       // [2] room taken in child
     int *host_words = nullptr;         // pinned host copy of sync_words
     hipEvent_t words_ready = nullptr;  // recorded after that copy
     // partial sorts order the keys on their top sorted_digits digits; a

@@ -137,9 +137,10 @@ __global__ void k_keys(const double *__restrict__ x, const double *__restrict__ 
                        int *__restrict__ perm, int *__restrict__ sync_words)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0) {  // node count, partial-sort check
+    if (i == 0) {  // node count, partial-sort check, child-list room
         sync_words[0] = 0;
         sync_words[1] = 0;
+        sync_words[2] = 0;
     }
     if (i >= sh.n) return;
     double pos[3] = {x[i], sh.dim > 1 ? y[i] : 0.0, sh.dim > 2 ? z[i] : 0.0};
@@ -591,8 +592,6 @@ __global__ void k_kdig(const unsigned long long *__restrict__ key, TreeShape sh,
 }
 
 // ---- 5. leaf level and node counts ----------------------------------------------
-constexpr int kMaxLevels = 64;
-
 constexpr int kLambdaThreads = 128;
 
 __global__ void k_lambda(const unsigned char *__restrict__ kdig, TreeShape sh, unsigned char *__restrict__ lam,
@@ -698,112 +697,51 @@ __global__ void k_lambda(const unsigned char *__restrict__ kdig, TreeShape sh, u
 }
 
 // ---- 6. node fill ------------------------------------------------------------------
-// first j >= lo whose key prefix (key >> shift) differs from p, searching
-// forward from lo with doubling steps, then bisecting the last step; nodes on
-// one particle's path are nested, so each level starts from the end of the
-// level below it and the search stays short
-__device__ int gallop_end(const unsigned long long *__restrict__ key, int n, int lo, unsigned long long p, int shift)
-{
-    if (lo >= n || (key[lo] >> shift) != p) return lo;
-    int step = 1;
-    int hi = lo + 1;
-    while (hi < n && (key[hi] >> shift) == p) {
-        lo = hi;
-        step <<= 1;
-        hi = min(n, lo + step);
-    }
-    // key[lo] has the prefix; the first differing position is in (lo, hi]
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if ((key[mid] >> shift) == p) lo = mid;
-        else hi = mid;
-    }
-    return hi;
-}
-
+// Start, level and geometry of the nodes that start at each particle (their
+// ends are found by k_node_records).  Loops over the axes are unrolled to three
+// with the dimension as a condition: to a run-time bound they put the centre
+// into scratch memory.
 __global__ void k_fill(const unsigned long long *__restrict__ key, const unsigned char *__restrict__ kdig,
-                       const unsigned char *__restrict__ lam, const int *__restrict__ leaf_end,
-                       const int *__restrict__ nbase, const double *__restrict__ root, TreeShape sh,
-                       const int *__restrict__ sync_words,
-                       int *__restrict__ nstart, int *__restrict__ nend, int *__restrict__ nskip,
-                       int *__restrict__ nlevel, double *__restrict__ ncenter, double *__restrict__ nedge, int cap,
-                       long long *__restrict__ stats)
+                       const unsigned char *__restrict__ lam, const int *__restrict__ nbase,
+                       const double *__restrict__ root, TreeShape sh, const int *__restrict__ sync_words,
+                       int *__restrict__ nstart, int *__restrict__ nlevel, double *__restrict__ ncenter,
+                       double *__restrict__ nedge, int cap)
 {
-    // the node count comes from the device (the host reads it while this
-    // runs); nothing is written when it exceeds the capacity or when the
+    // the node count comes from the device (the host reads it meanwhile);
+    // nothing is written when it exceeds the capacity or when the
     // partial-sort check failed (the build is then repeated)
-    const int total = sync_words[0];
-    if (total > cap || sync_words[1] != 0) return;
+    if (sync_words[0] > cap || sync_words[1] != 0) return;
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    int leaves = 0, depth = 0;
-    const int idx0 = (s < sh.n) ? nbase[s] : 0;
-    const int cnt = (s < sh.n) ? nbase[s + 1] - idx0 : 0;
-    if (cnt > 0) {
-        int idx = idx0;
-        const int L1 = lam[s];
-        const int ML = sh.ml;
-        depth = L1;
-        if (s == 0) {
-            nstart[idx] = 0;
-            nend[idx] = sh.n;
-            nskip[idx] = total;
-            nlevel[idx] = 1;
-            for (int k = 0; k < 3; ++k) ncenter[(size_t)k * cap + idx] = root[k];
-            nedge[idx] = root[3];
-            ++idx;
+    if (s >= sh.n) return;
+    int idx = nbase[s];
+    if (nbase[s + 1] == idx) return;
+    const int L1 = lam[s];
+    const int ML = sh.ml;
+    double c[3] = {root[0], root[1], root[2]};
+    double e = root[3];
+    auto put = [&](int level) {
+        nstart[idx] = s;
+        nlevel[idx] = level;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) ncenter[(size_t)k * cap + idx] = c[k];
+        nedge[idx] = e;
+        ++idx;
+    };
+    if (s == 0) put(1);
+    const int lmin = max(2, (int)kdig[s] + 1);
+    const unsigned long long kk = key[s];
+    // replay the centre recursion down the particle's path; its nodes from
+    // level lmin on start here
+    for (int L = 2; L <= L1; ++L) {
+        // centre of the child on the path, from level L - 1 (src/bhtree.cpp:233-239)
+        const unsigned dig = (unsigned)(kk >> (sh.bits * (ML - (L - 1)))) & ((1u << sh.bits) - 1u);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const double sg = ((dig >> k) & 1u) ? 1.0 : -1.0;
+            if (k < sh.dim) c[k] = c[k] + sg * e * 0.25;
         }
-        const int lmin = max(2, (int)kdig[s] + 1);
-        const unsigned long long kk = key[s];
-        // replay the centre recursion down to level lmin
-        double c[3] = {root[0], root[1], root[2]};
-        double e = root[3];
-        for (int d = 1; d < lmin; ++d) {
-            const unsigned dig = (unsigned)(kk >> (sh.bits * (ML - d))) & ((1u << sh.bits) - 1u);
-            for (int k = 0; k < sh.dim; ++k) {
-                const double sg = ((dig >> k) & 1u) ? 1.0 : -1.0;
-                c[k] = c[k] + sg * e * 0.25;
-            }
-            e = e * 0.5;
-        }
-        // top-down: start, level and geometry of the nodes on this path
-        for (int L = lmin, q = idx; L <= L1; ++L, ++q) {
-            const bool leaf = (L == L1);
-            nstart[q] = s;
-            nlevel[q] = leaf ? -L : L;
-            for (int k = 0; k < 3; ++k) ncenter[(size_t)k * cap + q] = c[k];
-            nedge[q] = e;
-            leaves += leaf ? 1 : 0;
-            // centre of the child on this particle's path
-            const unsigned dig = (unsigned)(kk >> (sh.bits * (ML - L))) & ((1u << sh.bits) - 1u);
-            for (int k = 0; k < sh.dim; ++k) {
-                const double sg = ((dig >> k) & 1u) ? 1.0 : -1.0;
-                c[k] = c[k] + sg * e * 0.25;
-            }
-            e = e * 0.5;
-        }
-        // bottom-up: the node at level L holds the particles sharing key's
-        // first L-1 digits; its end is at or after the end of the level below
-        int end_below = s + 1;
-        for (int L = L1, q = idx + (L1 - lmin); L >= lmin; --L, --q) {
-            int end;
-            if (L == L1 && L1 <= ML) end = leaf_end[s];
-            else {
-                const int shift = sh.bits * (ML - (L - 1));
-                end = (shift >= 64) ? sh.n : gallop_end(key, sh.n, end_below, kk >> shift, shift);
-            }
-            nend[q] = end;
-            nskip[q] = (end < sh.n) ? nbase[end] : total;
-            end_below = end;
-        }
-    }
-    // counters: one atomic per wavefront
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-        leaves += __shfl_xor(leaves, off, kWave);
-        depth = max(depth, __shfl_xor(depth, off, kWave));
-    }
-    if ((threadIdx.x & (kWave - 1)) == 0) {
-        if (leaves) atomicAdd(stat_ptr(stats, 11), (unsigned long long)leaves);
-        if (depth) atomicMax(stat_ptr(stats, 12), (unsigned long long)depth);
+        e = e * 0.5;
+        if (L >= lmin) put(L == L1 ? -L : L);
     }
 }
 
@@ -901,75 +839,167 @@ __global__ void k_node_ks(const int *__restrict__ nstart, const int *__restrict_
     nlink[idx] = l;
 }
 
-// FP32 walk records of the neighbour search (kernel_size is added by
-// k_node_ks).  Internal nodes keep their cell (centre rounded to nearest, half
-// edge rounded up); a leaf gets the bounding box of its members, which can be
-// much smaller than its cell.  FP32 rounding of the centre is covered by the
-// search's reach padding.
-__global__ void k_node_records(int total, int dim, const int *__restrict__ nstart, const int *__restrict__ nend,
-                               const int *__restrict__ nskip, const int *__restrict__ nlevel,
-                               const double *__restrict__ ncenter, const double *__restrict__ nedge, int cap,
-                               const double *__restrict__ px, const double *__restrict__ py,
-                               const double *__restrict__ pz, float4 *__restrict__ nbox, float2 *__restrict__ nhalf,
-                               int4 *__restrict__ nlink)
+// first j > s whose key prefix (key >> shift) differs from that of s, by the
+// kNodeLanes lanes of a group together: eight probes per step, at distances that
+// grow eightfold until one differs and shrink eightfold after
+__device__ int group_end(const unsigned long long *__restrict__ key, int n, int s, int shift, int sub)
 {
-    // kNodeLanes lanes per node share a leaf's member loop
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    const int idx = g / kNodeLanes, sub = g % kNodeLanes;
-    if (idx >= total) return;  // whole groups leave together
-    const int s = nstart[idx], e = nend[idx];
-    const bool leaf = nlevel[idx] < 0;
-    double c[3] = {ncenter[idx], ncenter[(size_t)cap + idx], ncenter[2 * (size_t)cap + idx]};
-    double h[3] = {0.5 * nedge[idx], 0.5 * nedge[idx], 0.5 * nedge[idx]};
-    if (leaf && e > s) {
-        const double *p[3] = {px, py, pz};
-        for (int k = 0; k < dim; ++k) {
-            double lo = p[k][s], hi = lo;
-            for (int j = s + 1 + sub; j < e; j += kNodeLanes) {
-                const double v = p[k][j];
-                lo = v < lo ? v : lo;
-                hi = v > hi ? v : hi;
+    const unsigned long long p = key[s] >> shift;
+    const int lane0 = (threadIdx.x & (kWave - 1)) - sub;
+    int lo = s;
+    auto equal_probes = [&](long long step) {
+        const long long j = lo + step * (sub + 1);
+        const bool eq = j < n && (key[j] >> shift) == p;
+        const unsigned bits = (unsigned)(__ballot(eq) >> lane0) & ((1u << kNodeLanes) - 1u);
+        return __ffs(~bits) - 1;
+    };
+    long long step = 1;
+    int e;
+    while ((e = equal_probes(step)) == kNodeLanes) {
+        lo += (int)(step * kNodeLanes);
+        step *= kNodeLanes;
+    }
+    lo += (int)(step * e);
+    while (step > 1) {
+        step /= kNodeLanes;
+        e = min(equal_probes(step), kNodeLanes - 1);
+        lo += (int)(step * e);
+    }
+    return lo + 1;
+}
+
+// Per node: its end and skip, and the FP32 walk records of the neighbour search
+// (kernel_size is added by k_node_ks).  Internal nodes keep their cell (centre
+// rounded to nearest, half edge rounded up); a leaf gets the bounding box of its
+// members, which can be much smaller than its cell.  FP32 rounding of the centre
+// is covered by the search's reach padding.  The ends used to be found by the
+// thread of the node's first particle, level by level; the first particle's
+// chain of searches up to the root took most of that kernel's 21 us at 500
+// particles and 44 at 1M (node fill and records together 24 -> 10 us and 60 ->
+// 41).  The node count is read on the device, so the launch does not wait for
+// the host to know it.
+__global__ __launch_bounds__(256) void k_node_records(
+    const int *__restrict__ sync_words, TreeShape sh, const unsigned long long *__restrict__ key,
+    const int *__restrict__ leaf_end, const int *__restrict__ nbase, const int *__restrict__ nstart,
+    int *__restrict__ nend, int *__restrict__ nskip, const int *__restrict__ nlevel, const double *__restrict__ ncenter,
+    const double *__restrict__ nedge, int cap, const double *__restrict__ px, const double *__restrict__ py,
+    const double *__restrict__ pz, float4 *__restrict__ nbox, float2 *__restrict__ nhalf, int4 *__restrict__ nlink,
+    long long *__restrict__ stats)
+{
+    const int total = sync_words[0];
+    if (total > cap || sync_words[1] != 0) return;
+    int leaves = 0, depth = 0;
+    // kNodeLanes lanes per node share its search and a leaf's member loop
+    const int sub = threadIdx.x % kNodeLanes;
+    for (long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x; g / kNodeLanes < total;
+         g += (long long)gridDim.x * blockDim.x) {
+        const int idx = (int)(g / kNodeLanes);
+        const int s = nstart[idx], lv = nlevel[idx];
+        const bool leaf = lv < 0;
+        const int L = leaf ? -lv : lv;
+        // the node at level L holds the particles sharing key's first L - 1 digits
+        int e = sh.n;
+        if (leaf && L <= sh.ml) e = leaf_end[s];
+        else if (L > 1) e = group_end(key, sh.n, s, sh.bits * (sh.ml - (L - 1)), sub);
+        double c[3] = {ncenter[idx], ncenter[(size_t)cap + idx], ncenter[2 * (size_t)cap + idx]};
+        double h[3] = {0.5 * nedge[idx], 0.5 * nedge[idx], 0.5 * nedge[idx]};
+        if (leaf && e > s) {
+            const double *p[3] = {px, py, pz};
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                if (k >= sh.dim) break;
+                double lo = p[k][s], hi = lo;
+                for (int j = s + 1 + sub; j < e; j += kNodeLanes) {
+                    const double v = p[k][j];
+                    lo = v < lo ? v : lo;
+                    hi = v > hi ? v : hi;
+                }
+                for (int off = kNodeLanes / 2; off > 0; off >>= 1) {
+                    const double ol = __shfl_xor(lo, off, kNodeLanes), oh = __shfl_xor(hi, off, kNodeLanes);
+                    lo = ol < lo ? ol : lo;
+                    hi = oh > hi ? oh : hi;
+                }
+                c[k] = 0.5 * (lo + hi);
+                // half extent, and rounding of the centre in FP64
+                h[k] = 0.5 * (hi - lo) + 4.0 * 1.1102230246251565e-16 * (fabs(lo) + fabs(hi));
             }
-            for (int off = kNodeLanes / 2; off > 0; off >>= 1) {
-                const double ol = __shfl_xor(lo, off, kNodeLanes), oh = __shfl_xor(hi, off, kNodeLanes);
-                lo = ol < lo ? ol : lo;
-                hi = oh > hi ? oh : hi;
-            }
-            c[k] = 0.5 * (lo + hi);
-            // half extent, and rounding of the centre in FP64
-            h[k] = 0.5 * (hi - lo) + 4.0 * 1.1102230246251565e-16 * (fabs(lo) + fabs(hi));
+        }
+        if (sub == 0) {
+            const int skip = e < sh.n ? nbase[e] : total;
+            nend[idx] = e;
+            nskip[idx] = skip;
+            nbox[idx] = make_float4((float)c[0], (float)c[1], (float)c[2], float_up(h[0]));
+            nhalf[idx] = make_float2(float_up(h[1]), float_up(h[2]));
+            nlink[idx] = make_int4(s, e, skip, leaf ? (int)0x80000000 : 0);
+            leaves += leaf ? 1 : 0;
+            depth = max(depth, leaf ? L : 0);
         }
     }
-    if (sub) return;
-    nbox[idx] = make_float4((float)c[0], (float)c[1], (float)c[2], float_up(h[0]));
-    nhalf[idx] = make_float2(float_up(h[1]), float_up(h[2]));
-    nlink[idx] = make_int4(s, e, nskip[idx], leaf ? (int)0x80000000 : 0);
+    // counters: one atomic per wavefront
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+        leaves += __shfl_xor(leaves, off, kWave);
+        depth = max(depth, __shfl_xor(depth, off, kWave));
+    }
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+        if (leaves) atomicAdd(stat_ptr(stats, 11), (unsigned long long)leaves);
+        if (depth) atomicMax(stat_ptr(stats, 12), (unsigned long long)depth);
+    }
 }
 
-// child lists: count the direct children of each internal node (its
-// sibling chain k+1, skip[k+1], ... below skip[k]) ...
-__global__ void k_child_count(int total, const int *__restrict__ nskip, const int *__restrict__ nlevel,
-                              unsigned int *__restrict__ ccount)
+// Child lists: the direct children of each internal node (its sibling chain
+// k+1, skip[k+1], ... below skip[k]), stored contiguously.  Where a node's list
+// lies is of no consequence, so each workgroup takes room for its lists with one
+// atomic (sync_words[2]; one per wavefront serialises: 18 us for 87k nodes);
+// counting, scanning the counts and writing took three to five launches (15 us
+// at 500 particles, 29 at 1M; now 3.6 and 6.1).
+constexpr int kChildThreads = 1024;
+template <int D>
+__global__ __launch_bounds__(kChildThreads) void k_children(int *__restrict__ sync_words, int cap, const int *__restrict__ nskip,
+                                                  const int *__restrict__ nlevel, int2 *__restrict__ nchild,
+                                                  int *__restrict__ child)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= total) return;
-    unsigned int c = 0;
-    if (nlevel[k] > 0)
-        for (int ch = k + 1; ch < nskip[k]; ch = nskip[ch]) ++c;
-    ccount[k] = c;
-}
-
-// ... and write them at the scanned offsets
-__global__ void k_child_write(int total, const int *__restrict__ nskip, const int *__restrict__ nlevel,
-                              const unsigned int *__restrict__ coff, int2 *__restrict__ nchild, int *__restrict__ child)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= total) return;
-    const int off = (int)coff[k];
-    int c = 0;
-    if (nlevel[k] > 0)
-        for (int ch = k + 1; ch < nskip[k]; ch = nskip[ch]) child[off + c++] = ch;
-    nchild[k] = make_int2(off, c);
+    const int total = sync_words[0];
+    if (total > cap || sync_words[1] != 0) return;
+    __shared__ int wsum[kChildThreads / kWave], room;
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    for (int k0 = blockIdx.x * kChildThreads; k0 < total; k0 += gridDim.x * kChildThreads) {
+        const int k = k0 + threadIdx.x;
+        int ch[1 << D], c = 0;
+        const int last = k < total && nlevel[k] > 0 ? nskip[k] : 0;
+        int next = k + 1;
+#pragma unroll
+        for (int u = 0; u < (1 << D); ++u) {
+            ch[u] = next;
+            if (next < last) {
+                ++c;
+                next = nskip[next];
+            }
+        }
+        int incl = c;
+        for (int off = 1; off < kWave; off <<= 1) {
+            const int t = __shfl_up(incl, off, kWave);
+            if (lane >= off) incl += t;
+        }
+        if (lane == kWave - 1) wsum[w] = incl;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            int sum = 0;
+#pragma unroll
+            for (int q = 0; q < kChildThreads / kWave; ++q) {
+                const int t = wsum[q];
+                wsum[q] = sum;
+                sum += t;
+            }
+            room = atomicAdd(sync_words + 2, sum);
+        }
+        __syncthreads();
+        const int at = room + wsum[w] + incl - c;
+        __syncthreads();  // before the next round writes them
+#pragma unroll
+        for (int u = 0; u < (1 << D); ++u)
+            if (u < c) child[at + u] = ch[u];
+        if (k < total) nchild[k] = make_int2(at, c);
+    }
 }
 
 struct SumTables {
@@ -1052,7 +1082,7 @@ int tree_alloc(sphgpu_ctx *c)
     t.hist_blocks = (n + kSortTile - 1) / kSortTile;
     bool ok = al((void **)&t.key, 8ull * n) && al((void **)&t.key_alt, 8ull * n) && al((void **)&t.perm, 4ull * n) &&
               al((void **)&t.perm_alt, 4ull * n) && al((void **)&t.kdig, n) && al((void **)&t.lam, n) &&
-              al((void **)&t.sync_words, 4ull * 2) &&
+              al((void **)&t.sync_words, 4ull * 4) &&
               al((void **)&t.leaf_end, 4ull * n) && al((void **)&t.ncount, 4ull * (n + 1)) &&
               al((void **)&t.nbase, 4ull * (n + 1)) && al((void **)&t.start, 4ull * t.node_cap) &&
               al((void **)&t.end, 4ull * t.node_cap) && al((void **)&t.skip, 4ull * t.node_cap) &&
@@ -1064,7 +1094,7 @@ int tree_alloc(sphgpu_ctx *c)
               al((void **)&t.root, 8ull * 8) && al((void **)&t.hist, 4ull * 256 * t.hist_blocks) &&
               al((void **)&t.nbox, 16ull * t.node_cap) && al((void **)&t.nlink, 16ull * t.node_cap) &&
               al((void **)&t.nhalf, 8ull * t.node_cap) && al((void **)&t.nchild, 8ull * t.node_cap) &&
-              al((void **)&t.child, 4ull * (t.node_cap + 8)) && al((void **)&t.ccount, 4ull * t.node_cap);
+              al((void **)&t.child, 4ull * (t.node_cap + 8));
     const long long scan_max = std::max<long long>(std::max<long long>(n + 1, 256ll * t.hist_blocks), t.node_cap);
     ok = ok && al((void **)&t.scan_tmp, 4ull * ((scan_max + kScanTile - 1) / kScanTile + 1));
     ok = ok && hipHostMalloc((void **)&t.host_words, 4ull * 2, hipHostMallocDefault) == hipSuccess &&
@@ -1089,7 +1119,7 @@ void tree_free(sphgpu_ctx *c)
     Tree &t = c->tree;
     void *ps[] = {t.key, t.key_alt, t.perm, t.perm_alt, t.kdig, t.lam, t.sync_words, t.leaf_end, t.ncount, t.nbase, t.start,
                   t.end, t.skip, t.level, t.center, t.edge, t.ks, t.mass, t.com, t.bmax1, t.bmax2, t.bsum1,
-                  t.bsum2, t.root, t.hist, t.nbox, t.nlink, t.scan_tmp, t.nhalf, t.nchild, t.child, t.ccount, t.gnode, t.gpart};
+                  t.bsum2, t.root, t.hist, t.nbox, t.nlink, t.scan_tmp, t.nhalf, t.nchild, t.child, t.gnode, t.gpart};
     for (void *p : ps)
         if (p) hipFree(p);
     if (t.host_words) hipHostFree(t.host_words);
@@ -1215,9 +1245,34 @@ int tree_build(sphgpu_ctx *c)
     HIPCHK(c, hipMemcpyAsync(t.host_words, t.sync_words, 2 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipEventRecord(t.words_ready, c->stream));
     hipLaunchKernelGGL(k_fill, dim3(grid_for(n, 128)), dim3(128), 0, c->stream, (const unsigned long long *)t.key,
-                       (const unsigned char *)t.kdig, (const unsigned char *)t.lam, (const int *)t.leaf_end,
-                       (const int *)t.nbase, (const double *)t.root, sh, (const int *)t.sync_words, t.start, t.end,
-                       t.skip, t.level, t.center, t.edge, t.node_cap, c->dstats);
+                       (const unsigned char *)t.kdig, (const unsigned char *)t.lam, (const int *)t.nbase,
+                       (const double *)t.root, sh, (const int *)t.sync_words, t.start, t.level, t.center, t.edge,
+                       t.node_cap);
+    HIPCHK(c, hipGetLastError());
+    time_end(c);
+    // the node passes loop over the device's node count; their grids follow the
+    // last build's (or a guess), so nothing waits for the host here.  Positions
+    // are read from the permuted (key-ordered) arrays.
+    px = c->pos[0];
+    py = c->dim > 1 ? c->pos[1] : c->pos[0];
+    pz = c->dim > 2 ? c->pos[2] : c->pos[0];
+    time_begin(c, "tree_node_records");
+    const long long guess = std::min<long long>(t.node_cap, (t.n_nodes > 0 ? t.n_nodes : n / 4) * 5ll / 4 + 256);
+    hipLaunchKernelGGL(k_node_records, dim3(grid_for(guess * kNodeLanes, 256)), dim3(256), 0, c->stream,
+                       (const int *)t.sync_words, sh, (const unsigned long long *)t.key, (const int *)t.leaf_end,
+                       (const int *)t.nbase, (const int *)t.start, t.end, t.skip, (const int *)t.level,
+                       (const double *)t.center, (const double *)t.edge, t.node_cap, px, py, pz, t.nbox, t.nhalf,
+                       t.nlink, c->dstats);
+    const dim3 gc(grid_for(guess, kChildThreads)), bc(kChildThreads);
+    if (c->dim == 1)
+        hipLaunchKernelGGL(k_children<1>, gc, bc, 0, c->stream, t.sync_words, t.node_cap, (const int *)t.skip,
+                           (const int *)t.level, t.nchild, t.child);
+    else if (c->dim == 2)
+        hipLaunchKernelGGL(k_children<2>, gc, bc, 0, c->stream, t.sync_words, t.node_cap, (const int *)t.skip,
+                           (const int *)t.level, t.nchild, t.child);
+    else
+        hipLaunchKernelGGL(k_children<3>, gc, bc, 0, c->stream, t.sync_words, t.node_cap, (const int *)t.skip,
+                           (const int *)t.level, t.nchild, t.child);
     HIPCHK(c, hipGetLastError());
     time_end(c);
     // the pair records depend on the permuted particle state only: they are
@@ -1248,24 +1303,9 @@ int tree_build(sphgpu_ctx *c)
         return fail(c, SPHGPU_E_NO_FREE_NODE, "There is no free node.");
     }
     t.n_nodes = total;
-    time_begin(c, "tree_node_records");
-    hipLaunchKernelGGL(k_node_records, dim3(grid_for((long long)total * kNodeLanes, 256)), dim3(256), 0, c->stream, total, c->dim,
-                       (const int *)t.start, (const int *)t.end, (const int *)t.skip, (const int *)t.level,
-                       (const double *)t.center, (const double *)t.edge, t.node_cap, (const double *)c->pos[0],
-                       (const double *)(c->dim > 1 ? c->pos[1] : c->pos[0]),
-                       (const double *)(c->dim > 2 ? c->pos[2] : c->pos[0]), t.nbox, t.nhalf, t.nlink);
-    hipLaunchKernelGGL(k_child_count, dim3(grid_for(total, 256)), dim3(256), 0, c->stream, total,
-                       (const int *)t.skip, (const int *)t.level, t.ccount);
-    scan_counts(c->stream, (const unsigned *)t.ccount, t.ccount, total, t.scan_tmp, false);
-    hipLaunchKernelGGL(k_child_write, dim3(grid_for(total, 256)), dim3(256), 0, c->stream, total,
-                       (const int *)t.skip, (const int *)t.level, (const unsigned *)t.ccount, t.nchild, t.child);
-    HIPCHK(c, hipGetLastError());
-    // mass and centre of mass per node (needed by the gravity walk); the
-    // positions are read from the permuted (key-ordered) arrays
-    px = c->pos[0];
-    py = c->dim > 1 ? c->pos[1] : c->pos[0];
-    pz = c->dim > 2 ? c->pos[2] : c->pos[0];
+    // mass and centre of mass per node (needed by the gravity walk)
     if (c->prm.use_gravity) {
+        time_begin(c, "tree_node_mass");
         const int nb1 = (n + 63) / 64, nb2 = (nb1 + 63) / 64;
         hipLaunchKernelGGL(k_block_sum4, dim3(grid_for((long long)nb1 * 64, 256)), dim3(256), 0, c->stream,
                            (const double *)c->sc[S_MASS], px, c->dim > 1 ? py : nullptr, c->dim > 2 ? pz : nullptr, n,
@@ -1275,9 +1315,9 @@ int tree_build(sphgpu_ctx *c)
         SumTables st{c->sc[S_MASS], px, c->dim > 1 ? py : nullptr, c->dim > 2 ? pz : nullptr, t.bsum1, t.bsum2, nb1, nb2};
         hipLaunchKernelGGL(k_node_mass, dim3(grid_for((long long)total * kNodeLanes, 128)), dim3(128), 0, c->stream, (const int *)t.start,
                            (const int *)t.end, total, st, t.mass, t.com, t.node_cap);
+        time_end(c);
+        HIPCHK(c, hipGetLastError());
     }
-    time_end(c);
-    HIPCHK(c, hipGetLastError());
     t.valid = true;
     c->sorted_valid = true;
     return 0;

@@ -278,3 +278,41 @@ def test_force_list_runs_sorted(nn, reach):
         tail = max(tail, int((r[want] >= h[i]).sum()))
     print("longest appended run", tail)
     np.testing.assert_array_equal(runs[0], runs[1])
+
+
+@pytest.mark.parametrize("dim,leaf", [(1, 1), (2, 1), (3, 1), (3, 8), (2, 70)])
+@pytest.mark.parametrize("n", [1, 2, 9, 64, 65, 513, 4097, 70001])
+def test_tree_ranges_and_children(n, dim, leaf):
+    """Node ranges (found eight probes at a time), pre-order and the partition of
+    every node's members by its children, for random and coincident particles,
+    and for a second build after the particles moved (its launches are sized by
+    the first one's nodes, here far fewer)."""
+    p, f = _random_state(n, dim, seed=leaf)
+    p["leaf_particle_num"] = leaf
+    c = sphgpu.Context(p, n)
+    packed = f.copy()
+    packed[ics.F_POS:ics.F_POS + dim] = 0.5  # one cell to the last level
+    # (a chain of 21 nodes exceeds the pool of 5 n + 1 below five particles)
+    for state in (packed, f) if n > 4 else (f, f):
+        c.upload(state)
+        c.build_tree()
+        d = c.tree_dump()
+        members, first, count, level = d["members"], d["first"], d["count"], d["level"]
+        x = state[ics.F_POS:ics.F_POS + dim][:, members]
+        assert first[0] == 0 and count[0] == n and level[0] == 1
+        parents, used = [], np.zeros(len(level), dtype=int)
+        for k in range(len(level)):
+            while parents and level[parents[-1]] >= level[k]:
+                parents.pop()
+            if parents:
+                q = parents[-1]
+                assert level[k] == level[q] + 1 and first[k] == first[q] + used[q]
+                used[q] += count[k]
+            parents.append(k)
+            inside = x[:, first[k]:first[k] + count[k]]
+            assert (np.abs(inside - d["center"][k, :dim, None]) <= 0.5 * d["edge"][k]).all()
+        leafs = d["is_leaf"] == 1
+        assert (used[~leafs] == count[~leafs]).all() and (used[leafs] == 0).all()
+        assert ((count[leafs] <= leaf) | (level[leafs] == p["max_tree_level"] + 1)).all()
+        assert (count[~leafs][1:] > leaf).all()
+    c.close()
