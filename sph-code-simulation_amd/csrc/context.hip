@@ -249,7 +249,7 @@ int sphgpu_create(const sphgpu_params *p, int n, sphgpu_ctx **out)
     }
     for (int s = 0; s < S_NSCALAR && ok; ++s) ok = alloc((void **)&c->sc[s], dn);
     for (int g = 0; g < kNGrad && ok; ++g) ok = alloc((void **)&c->grad[g], dn);
-    for (int a = 0; a < 16 && ok; ++a) ok = alloc((void **)&c->alt[a], dn);
+    for (int a = 0; a < kAlt && ok; ++a) ok = alloc((void **)&c->alt[a], dn);
     ok = ok && alloc((void **)&c->id, sizeof(int) * n) && alloc((void **)&c->id_alt, sizeof(int) * n) &&
          alloc((void **)&c->neighbor, sizeof(int) * n);
     for (int r = 0; r < R_NREC && ok; ++r) ok = alloc((void **)&c->rec32[r], sizeof(float4) * (size_t)n);
@@ -296,7 +296,7 @@ int sphgpu_destroy(sphgpu_ctx *c)
     }
     for (int s = 0; s < S_NSCALAR; ++s) hipFree(c->sc[s]);
     for (int g = 0; g < kNGrad; ++g) hipFree(c->grad[g]);
-    for (int a = 0; a < 16; ++a) hipFree(c->alt[a]);
+    for (int a = 0; a < kAlt; ++a) hipFree(c->alt[a]);
     hipFree(c->id); hipFree(c->id_alt); hipFree(c->neighbor);
     for (int r = 0; r < R_NREC; ++r) {
         hipFree(c->rec32[r]);
@@ -450,8 +450,7 @@ static int integrate_impl(sphgpu_ctx *c, int nsteps)
         if ((rc = pre_interaction_deferred(c))) return rc;
         if ((rc = fluid_force(c))) return rc;  // settles the deferred search first
         if ((rc = gravity(c))) return rc;
-        if ((rc = correct(c))) return rc;
-        if ((rc = advance_time(c))) return rc;
+        if ((rc = correct(c, true))) return rc;
     }
     return 0;
 }

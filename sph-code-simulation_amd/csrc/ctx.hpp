@@ -36,6 +36,10 @@ enum SField {
 //            (gv2 gv3 gv4 gv5) (gv6 gv7 gv8 0), gv index = 3*component + axis
 enum RecField { R_POSH, R_VELM, R_THERMO, R_AUX, R_G0, R_G1, R_G2, R_G3, R_NREC };
 
+// rows of the permutation's double buffers: the 20 that a time step permutes
+// in 3D go in one launch
+constexpr int kAlt = 20;
+
 // GSPH gradient rows in FP64 (grad_d[3], grad_p[3], grad_v[9])
 constexpr int kNGrad = 15;
 
@@ -155,7 +159,7 @@ struct sphgpu_ctx {
     double *grad[sphgpu::kNGrad] = {};
     int *id = nullptr, *neighbor = nullptr;
     // permutation double-buffers for the persistent fields
-    double *alt[16] = {};
+    double *alt[sphgpu::kAlt] = {};
     int *id_alt = nullptr;
     // pair records: FP32 always (they also feed the search prefilter), FP64
     // in FP64 pair mode
@@ -293,12 +297,12 @@ int gravity(sphgpu_ctx *c);
 
 // integrate.hip
 int predict(sphgpu_ctx *c);
-int correct(sphgpu_ctx *c);
+// advance: also Simulation::update_time (the time step's last two calls)
+int correct(sphgpu_ctx *c, bool advance = false);
 int timestep(sphgpu_ctx *c);
 int energy_momentum(sphgpu_ctx *c, double out[7]);
 int refresh_mirrors(sphgpu_ctx *c);
 int init_fields(sphgpu_ctx *c);
-int advance_time(sphgpu_ctx *c);
 
 // mlp.hip
 int mlp_create(sphgpu_ctx *c);

@@ -22,7 +22,7 @@ struct IntArgs {
     const double *acc[3];
     double *ene, *ene_p, *sound;
     const double *dene;
-    const double *dscal;
+    double *dscal;
     double c_sound;
     Box box;
 };
@@ -49,11 +49,13 @@ __global__ void k_predict(IntArgs a)
     }
 }
 
-__global__ void k_correct(IntArgs a)
+__global__ void k_correct(IntArgs a, int advance)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= a.n) return;
     const double dt = a.dscal[0];
+    // Simulation::update_time, src/simulation.cpp
+    if (advance && i == 0) a.dscal[1] = a.dscal[1] + dt;
     for (int k = 0; k < a.dim; ++k) a.vel[k][i] = a.vel_p[k][i] + a.acc[k][i] * (0.5 * dt);
     a.ene[i] = a.ene_p[i] + a.dene[i] * (0.5 * dt);
     a.sound[i] = __builtin_sqrt(a.c_sound * a.ene[i]);
@@ -114,8 +116,6 @@ __global__ __launch_bounds__(256) void k_dt_final(const double *__restrict__ par
         dscal[0] = (s[0] < dt_sound) ? s[0] : dt_sound;  // std::min(dt_sound, dt_force)
     }
 }
-
-__global__ void k_advance_time(double *dscal) { dscal[1] = dscal[1] + dscal[0]; }
 
 // kinetic, thermal, potential, P_x, P_y, P_z partial sums per block
 __global__ void k_energy_partial(int n, int dim, int grav, const double *vx, const double *vy, const double *vz,
@@ -227,10 +227,10 @@ int predict(sphgpu_ctx *c)
     return 0;
 }
 
-int correct(sphgpu_ctx *c)
+int correct(sphgpu_ctx *c, bool advance)
 {
     time_begin(c, "correct");
-    hipLaunchKernelGGL(k_correct, dim3(grid_for(c->n, 256)), dim3(256), 0, c->stream, int_args(c));
+    hipLaunchKernelGGL(k_correct, dim3(grid_for(c->n, 256)), dim3(256), 0, c->stream, int_args(c), advance ? 1 : 0);
     time_end(c);
     HIPCHK(c, hipGetLastError());
     c->mirror_dirty = true;
@@ -257,13 +257,6 @@ int timestep(sphgpu_ctx *c)
     hipLaunchKernelGGL(k_dt_final, dim3(1), dim3(256), 0, c->stream, (const double *)c->red, nb, c->prm.cfl_sound,
                        c->dscal);
     time_end(c);
-    HIPCHK(c, hipGetLastError());
-    return 0;
-}
-
-int advance_time(sphgpu_ctx *c)
-{
-    hipLaunchKernelGGL(k_advance_time, dim3(1), dim3(1), 0, c->stream, c->dscal);
     HIPCHK(c, hipGetLastError());
     return 0;
 }

@@ -548,10 +548,16 @@ __global__ __launch_bounds__(kScatterThreads) void k_sort_small(unsigned long lo
 }
 
 // ---- 3. permutation of the particle state -----------------------------------
+// up to kAlt rows of doubles and two of ints in one launch: below some 100k
+// particles a launch costs more than the rows it moves (500 particles: 5.1 us
+// for all rows, one launch of 16 rows and one of the ints took 4.6 + 3.0)
 struct GatherBatch {
-    const double *src[16];
-    double *dst[16];
+    const double *src[kAlt];
+    double *dst[kAlt];
     int count;
+    const int *isrc[2];
+    int *idst[2];
+    int icount;
 };
 
 __global__ void k_gather_batch(GatherBatch b, const int *__restrict__ perm, int n)
@@ -560,42 +566,43 @@ __global__ void k_gather_batch(GatherBatch b, const int *__restrict__ perm, int 
     if (i >= n) return;
     const int s = perm[i];
     for (int f = 0; f < b.count; ++f) b.dst[f][i] = b.src[f][s];
-}
-
-__global__ void k_gather_int2(const int *__restrict__ a, int *__restrict__ ad, const int *__restrict__ b,
-                              int *__restrict__ bd, const int *__restrict__ perm, int n)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int s = perm[i];
-    ad[i] = a[s];
-    bd[i] = b[s];
+    for (int f = 0; f < b.icount; ++f) b.idst[f][i] = b.isrc[f][s];
 }
 
 // ---- 4. first differing level ---------------------------------------------------
-// also the partial-sort check (cut >= 0): flag[1] = 1 when particles i and
-// i + leaf share the sorted top digits (key >> cut), see k_prefix_runs
+// first level at which keys a and b (of neighbouring positions) differ
+__device__ int first_difference(unsigned long long a, unsigned long long b, const TreeShape &sh)
+{
+    const unsigned long long x = a ^ b;
+    if (x == 0) return sh.ml + 1;
+    const int msb = 63 - __clzll((long long)x);
+    return sh.ml - msb / sh.bits;
+}
+// the partial-sort check at position i (cut >= 0): flag[1] = 1 when particles i
+// and i + leaf share the sorted top digits (key >> cut)
+__device__ void check_prefix(const unsigned long long *key, const TreeShape &sh, int i, int cut, int *flag)
+{
+    const bool bad = i + sh.leaf < sh.n && (key[i] >> cut) == (key[i + sh.leaf] >> cut);
+    if (__ballot(bad) && (threadIdx.x & (kWave - 1)) == 0) atomicOr(flag + 1, 1);
+}
+
+// (leaves of more than 64 particles; k_lambda does it itself otherwise)
 __global__ void k_kdig(const unsigned long long *__restrict__ key, TreeShape sh, unsigned char *__restrict__ kdig,
                        int cut, int *__restrict__ flag)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (cut >= 0) {
-        const bool bad = i + sh.leaf < sh.n && (key[i] >> cut) == (key[i + sh.leaf] >> cut);
-        if (__ballot(bad) && (threadIdx.x & (kWave - 1)) == 0) atomicOr(flag + 1, 1);
-    }
+    if (cut >= 0) check_prefix(key, sh, i, cut, flag);
     if (i >= sh.n) return;
     if (i == 0) { kdig[0] = 0; return; }
-    const unsigned long long x = key[i - 1] ^ key[i];
-    if (x == 0) { kdig[i] = (unsigned char)(sh.ml + 1); return; }
-    const int msb = 63 - __clzll((long long)x);
-    kdig[i] = (unsigned char)(sh.ml - msb / sh.bits);
+    kdig[i] = (unsigned char)first_difference(key[i - 1], key[i], sh);
 }
 
 // ---- 5. leaf level and node counts ----------------------------------------------
 constexpr int kLambdaThreads = 128;
 
-__global__ void k_lambda(const unsigned char *__restrict__ kdig, TreeShape sh, unsigned char *__restrict__ lam,
-                         int *__restrict__ leaf_end, int *__restrict__ ncount)
+__global__ void k_lambda(const unsigned long long *__restrict__ key, unsigned char *__restrict__ kdig, TreeShape sh,
+                         unsigned char *__restrict__ lam, int *__restrict__ leaf_end, int *__restrict__ ncount, int cut,
+                         int *__restrict__ flag)
 {
     // per thread and level t: the nearest boundary with kdig <= t to the
     // left (offset <= 0) and to the right (offset >= 1) of i, in LDS (a
@@ -610,10 +617,12 @@ __global__ void k_lambda(const unsigned char *__restrict__ kdig, TreeShape sh, u
         const int wb = blockIdx.x * B - sh.leaf;
         for (int t = threadIdx.x; t < B + 2 * sh.leaf; t += B) {
             const int j = wb + t;
-            s_kd[t] = (j < 0 || j >= sh.n) ? (unsigned char)0 : kdig[j];
+            s_kd[t] = (j <= 0 || j >= sh.n) ? (unsigned char)0 : (unsigned char)first_difference(key[j - 1], key[j], sh);
         }
+        if (cut >= 0) check_prefix(key, sh, i, cut, flag);
         __syncthreads();
         if (i >= sh.n) return;
+        kdig[i] = s_kd[i - wb];
         const unsigned char *const kw = s_kd + (i - wb);  // kw[x] = kdig[i + x]
         // With pmL(d) = min kdig over [i - d, i] and pmR(e) = min kdig over
         // (i, i + e] (kdig[n] = 0), the node of level t + 1 around i starts
@@ -746,19 +755,33 @@ __global__ void k_fill(const unsigned long long *__restrict__ key, const unsigne
 }
 
 // ---- 7. block hierarchy and node reductions ------------------------------------------
-__global__ void k_block_max(const double *__restrict__ in, int n, double *__restrict__ out)
+// maxima over blocks of 64 (out1) and of 4096 values (out2), one workgroup of
+// 16 wavefronts per 4096: bound by the launch up to some 100k values (4.1 us at
+// 500 and 4.2 at 65k, against 2 x 3 us for a launch per level)
+__global__ __launch_bounds__(1024) void k_block_max(const double *__restrict__ in, int n, double *__restrict__ out1,
+                                                    double *__restrict__ out2)
 {
-    // one 64-lane wave per block of 64 values
-    const int b = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int i = b * kWave + lane;
-    if ((long long)b * kWave >= n) return;
-    double v = (i < n) ? in[i] : 0.0;
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-        const double o = __shfl_down(v, off, kWave);
-        v = o > v ? o : v;
+    __shared__ double part[16];
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    double top = 0.0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int b = blockIdx.x * 64 + r * 16 + w;
+        const long long i = (long long)b * kWave + lane;
+        double v = i < n ? in[i] : 0.0;
+        for (int off = kWave / 2; off > 0; off >>= 1) {
+            const double o = __shfl_xor(v, off, kWave);
+            v = o > v ? o : v;
+        }
+        if (lane == 0 && (long long)b * kWave < n) out1[b] = v;
+        top = v > top ? v : top;
     }
-    if (lane == 0) out[b] = v;
+    if (lane == 0) part[w] = top;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int q = 0; q < 16; ++q) top = part[q] > top ? part[q] : top;
+        out2[blockIdx.x] = top;
+    }
 }
 
 __global__ void k_block_sum4(const double *__restrict__ m, const double *__restrict__ x, const double *__restrict__ y,
@@ -1152,18 +1175,22 @@ static int permute_state(sphgpu_ctx *c)
             for (int a = 0; a < c->dim; ++a) fields.push_back(&c->grad[6 + 3 * a + k]);
         }
     }
-    for (size_t off = 0; off < fields.size(); off += 16) {
+    for (size_t off = 0; off < fields.size(); off += kAlt) {
         GatherBatch b;
-        b.count = (int)std::min<size_t>(16, fields.size() - off);
+        b.count = (int)std::min<size_t>(kAlt, fields.size() - off);
         for (int f = 0; f < b.count; ++f) {
             b.src[f] = *fields[off + f];
             b.dst[f] = c->alt[f];
         }
+        // the ids and neighbour counts ride on the first batch
+        b.icount = off == 0 ? 2 : 0;
+        b.isrc[0] = c->id;
+        b.idst[0] = c->id_alt;
+        b.isrc[1] = c->neighbor;
+        b.idst[1] = c->tree.perm_alt;
         hipLaunchKernelGGL(k_gather_batch, dim3(grid_for(n, 256)), dim3(256), 0, c->stream, b, perm, n);
         for (int f = 0; f < b.count; ++f) std::swap(*fields[off + f], c->alt[f]);
     }
-    hipLaunchKernelGGL(k_gather_int2, dim3(grid_for(n, 256)), dim3(256), 0, c->stream, (const int *)c->id, c->id_alt,
-                       (const int *)c->neighbor, c->tree.perm_alt, perm, n);
     std::swap(c->id, c->id_alt);
     std::swap(c->neighbor, c->tree.perm_alt);
     HIPCHK(c, hipGetLastError());
@@ -1231,12 +1258,13 @@ int tree_build(sphgpu_ctx *c)
     time_end(c);
 
     time_begin(c, "tree_nodes");
-    hipLaunchKernelGGL(k_kdig, dim3(grid_for(n, 256)), dim3(256), 0, c->stream, (const unsigned long long *)t.key, sh,
-                       t.kdig, skip ? cut : -1, t.sync_words);
+    if (sh.leaf > 64)
+        hipLaunchKernelGGL(k_kdig, dim3(grid_for(n, 256)), dim3(256), 0, c->stream, (const unsigned long long *)t.key, sh,
+                           t.kdig, skip ? cut : -1, t.sync_words);
     const size_t lam_lds = sh.leaf <= 64 ? (size_t)sh.leaf * kLambdaThreads : sizeof(short) * 2 * (size_t)(sh.ml + 1) * kLambdaThreads;
     hipLaunchKernelGGL(k_lambda, dim3(grid_for(n, kLambdaThreads)), dim3(kLambdaThreads), lam_lds,
-                       c->stream, (const unsigned char *)t.kdig, sh,
-                       t.lam, t.leaf_end, t.ncount);
+                       c->stream, (const unsigned long long *)t.key, t.kdig, sh, t.lam, t.leaf_end, t.ncount,
+                       skip ? cut : -1, t.sync_words);
     // the node count goes to nbase[n] and to sync_words[0] (read by the fill
     // on the device and copied to the host)
     scan_counts(c->stream, (const unsigned *)t.ncount, (unsigned *)t.nbase, n, t.scan_tmp, true,
@@ -1331,10 +1359,8 @@ int tree_set_kernel(sphgpu_ctx *c)
     const int n = c->n;
     const int nb1 = (n + 63) / 64, nb2 = (nb1 + 63) / 64;
     time_begin(c, "tree_set_kernel");
-    hipLaunchKernelGGL(k_block_max, dim3(grid_for((long long)nb1 * 64, 256)), dim3(256), 0, c->stream,
-                       (const double *)c->sc[S_SML], n, t.bmax1);
-    hipLaunchKernelGGL(k_block_max, dim3(grid_for((long long)nb2 * 64, 256)), dim3(256), 0, c->stream,
-                       (const double *)t.bmax1, nb1, t.bmax2);
+    hipLaunchKernelGGL(k_block_max, dim3(nb2), dim3(1024), 0, c->stream, (const double *)c->sc[S_SML], n, t.bmax1,
+                       t.bmax2);
     RangeTables rt{c->sc[S_SML], t.bmax1, t.bmax2};
     hipLaunchKernelGGL(k_node_ks, dim3(grid_for((long long)t.n_nodes * kNodeLanes, 128)), dim3(128), 0, c->stream, (const int *)t.start,
                        (const int *)t.end, t.n_nodes, rt, t.ks, t.nlink);

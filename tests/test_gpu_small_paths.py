@@ -316,3 +316,22 @@ def test_tree_ranges_and_children(n, dim, leaf):
         assert ((count[leafs] <= leaf) | (level[leafs] == p["max_tree_level"] + 1)).all()
         assert (count[~leafs][1:] > leaf).all()
     c.close()
+
+
+@pytest.mark.parametrize("dim,leaf", [(1, 1), (3, 8)])
+@pytest.mark.parametrize("n", [5, 63, 64, 65, 4095, 4096, 4097, 8193, 300001])
+def test_node_kernel_sizes(n, dim, leaf):
+    """Largest smoothing length below every node (maxima over blocks of 64 and
+    of 4096 particles, both levels in one launch), exactly."""
+    p, f = _random_state(n, dim, seed=3)
+    p["leaf_particle_num"] = leaf
+    f[ics.F_SML] = 0.01 + 0.1 * np.random.default_rng(n).random(n)
+    c = sphgpu.Context(p, n)
+    c.upload(f)
+    c.build_tree()
+    c.set_kernel()
+    d = c.tree_dump()
+    h = f[ics.F_SML][d["members"]]
+    top = [h[a:a + k].max() for a, k in zip(d["first"], d["count"])]
+    np.testing.assert_array_equal(d["kernel_size"], top)
+    c.close()
