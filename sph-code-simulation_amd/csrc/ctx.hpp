@@ -57,7 +57,8 @@ template <typename T> struct RecView {
 // 64 bytes, one wave-uniform load per visited node.
 struct alignas(16) GravNode {
     double cx, cy, cz, l2;
-    double mass, pad;
+    double mass;
+    float gm, pad;  // G * mass in FP32
     int start, end, skip, level;
 };
 

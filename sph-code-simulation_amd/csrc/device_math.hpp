@@ -535,6 +535,14 @@ template <typename T> struct BlockAcc {
         s = t;
         p = T(0);
     }
+    // a block that was summed elsewhere
+    SPH_DEV void add_block(T b)
+    {
+        const T t = s + b;
+        const T z = t - s;
+        c += (s - (t - z)) + (b - z);
+        s = t;
+    }
     SPH_DEV T get() const { return s + (c + p); }
 };
 template <> struct BlockAcc<double> {
@@ -542,6 +550,7 @@ template <> struct BlockAcc<double> {
     SPH_DEV BlockAcc() : s(0.0) {}
     SPH_DEV void add(double x) { s += x; }
     SPH_DEV void fold() {}
+    SPH_DEV void add_block(double b) { s += b; }
     SPH_DEV double get() const { return s; }
 };
 

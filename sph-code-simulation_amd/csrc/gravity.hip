@@ -13,14 +13,14 @@
 // every lane takes the reference's opening decision for its own particle in
 // FP64; lanes that accept the node add its monopole and sit out its subtree,
 // and the wave descends while any lane opens.  An opened leaf's members are
-// loaded once per wave into LDS and every opening lane sums its pair terms
-// from there.  Each particle therefore interacts with exactly the nodes and
-// leaf members of its own reference walk, in the same pre-order, while node
-// records are wave-uniform loads and member records are loaded once per wave
-// instead of once per lane.  The pair and monopole terms run in the pair
-// precision T with compensated sums taken in blocks of at most 16 terms.  The
-// node range is cut into pieces walked by different wavefronts; their sums are
-// added in a fixed order in FP64.
+// loaded once per wave into LDS, and the lanes share the opening lanes'
+// particles among themselves.  Each particle therefore interacts with exactly
+// the nodes and leaf members of its own reference walk, while node records are
+// wave-uniform scalar loads and member records are loaded once per wave instead
+// of once per lane.  The pair and monopole terms run in the pair precision T
+// with compensated sums taken in blocks of at most 16 terms.  The node range is
+// cut into pieces walked by different wavefronts; their sums are added in a
+// fixed order in FP64.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -37,6 +37,19 @@ SPH_DEV void wave_lds_fence()
 {
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
+}
+
+// x of the lane that a DPP control pairs with this one (all lanes active)
+template <int CTRL> SPH_DEV float dpp(float x)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL> SPH_DEV double dpp(double x)
+{
+    const long long b = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 
 // Hernquist & Katz (1989) softened potential and force factors
@@ -72,13 +85,16 @@ SPH_DEV void hk_fg(float r, float inv_r, float inv_e, float &f, float &g)
     const float u2 = u * u, u3 = u2 * u;
     const float inv_r3 = inv_r * inv_r * inv_r;
     const float inv_e3 = inv_e * inv_e * inv_e;
-    const float fa = (-0.5f * u2 * (1.0f / 3.0f - (3.0f / 20.0f) * u2 + u3 * (1.0f / 20.0f)) + 1.4f) * inv_e;
-    const float fb = -(1.0f / 15.0f) * inv_r + (-u2 * (4.0f / 3.0f - u + 0.3f * u2 - u3 * (1.0f / 30.0f)) + 1.6f) * inv_e;
-    const float ga = (4.0f / 3.0f - 1.2f * u2 + 0.5f * u3) * inv_e3;
-    const float gb = (-1.0f / 15.0f + u3 * (8.0f / 3.0f - 3.0f * u + 1.2f * u2 - u3 * (1.0f / 6.0f))) * inv_r3;
+    const float fa = fmaf(-0.5f * u2, fmaf(u3, 1.0f / 20.0f, fmaf(u2, -3.0f / 20.0f, 1.0f / 3.0f)), 1.4f) * inv_e;
+    const float fb = fmaf(fmaf(-u2, fmaf(u3, -1.0f / 30.0f, fmaf(u2, 0.3f, 4.0f / 3.0f - u)), 1.6f), inv_e,
+                          -(1.0f / 15.0f) * inv_r);
+    const float ga = fmaf(0.5f, u3, fmaf(-1.2f, u2, 4.0f / 3.0f)) * inv_e3;
+    const float gb = fmaf(u3, fmaf(u3, -1.0f / 6.0f, fmaf(1.2f, u2, fmaf(-3.0f, u, 8.0f / 3.0f))), -1.0f / 15.0f) * inv_r3;
     f = u < 1.0f ? fa : (u < 2.0f ? fb : inv_r);
     g = u < 1.0f ? ga : (u < 2.0f ? gb : inv_r3);
 }
+
+constexpr int kGravSideMax = 64;
 
 template <typename T> struct GravArgs {
     int n, n_nodes;
@@ -94,6 +110,7 @@ template <typename T> struct GravArgs {
     // the right and to the left; piece s writes its sums to
     // part[(4 s + c) n + i], c = phi, a_x, a_y, a_z
     int nside, ngroups;
+    int bound[kGravSideMax + 1];  // n_nodes k^2 / nside^2
     const int *nbase;
     double *part;
 };
@@ -103,7 +120,7 @@ template <typename T> struct GravArgs {
 __global__ void k_grav_nodes(int n_nodes, int cap, const double *__restrict__ com, const double *__restrict__ edge,
                              const double *__restrict__ mass, const int *__restrict__ start,
                              const int *__restrict__ end, const int *__restrict__ skip, const int *__restrict__ level,
-                             GravNode *__restrict__ out)
+                             float G, GravNode *__restrict__ out)
 {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n_nodes) return;
@@ -113,7 +130,8 @@ __global__ void k_grav_nodes(int n_nodes, int cap, const double *__restrict__ co
     g.cz = com[2 * (size_t)cap + k];
     g.l2 = edge[k] * edge[k];
     g.mass = mass[k];
-    g.pad = 0.0;
+    g.gm = G * (float)mass[k];
+    g.pad = 0.0f;
     g.start = start[k];
     g.end = end[k];
     g.skip = skip[k];
@@ -123,12 +141,16 @@ __global__ void k_grav_nodes(int n_nodes, int cap, const double *__restrict__ co
 
 template <typename T> struct GravStage;
 template <> struct GravStage<float> {
+    float4 own[kWave]; // the wavefront's particles: x, y, z, 1/e_i
     float4 p[kWave];   // x, y, z, 1/e_j
-    float gm[kWave];   // G m_j
+    float gm[kWave];   // G m_j / 2
+    int lane[kWave];   // the opening lanes, packed
 };
 template <> struct GravStage<double> {
+    double4 own[kWave];
     double4 p[kWave];  // x, y, z, h_j
     double gm[kWave];
+    int lane[kWave];
 };
 
 // minimum-image component for a periodic box, the plain difference otherwise
@@ -138,8 +160,22 @@ template <bool P, typename T> SPH_DEV T grav_rij(T xi, T xj, const Box &b, int k
     return P ? rij_axis<T>(xi, xj, b, k) : xi - xj;
 }
 
+// the 64-byte record of a node (the same for all lanes) in one scalar load; no
+// kernel that reads records writes them, which the address space states
+SPH_DEV GravNode load_node(const GravNode *p)
+{
+    typedef int I16 __attribute__((ext_vector_type(16)));
+    union {
+        I16 v;
+        GravNode g;
+    } u;
+    typedef const __attribute__((address_space(4))) I16 *Constant;
+    u.v = *(Constant)(unsigned long long)p;
+    return u.g;
+}
+
 template <int D, typename T, bool P>
-__global__ __launch_bounds__(256) void k_gravity(GravArgs<T> a)
+__global__ __launch_bounds__(256, sizeof(T) == 4 ? 8 : 4) void k_gravity(GravArgs<T> a)
 {
     __shared__ GravStage<T> stage[4];
     GravStage<T> &st = stage[(threadIdx.x >> 6) & 3];
@@ -164,9 +200,11 @@ __global__ __launch_bounds__(256) void k_gravity(GravArgs<T> a)
     double ri[3] = {0, 0, 0};
 #pragma unroll
     for (int k = 0; k < D; ++k) ri[k] = a.x64[k][i];
-    const V4 pi_ = RP[i];
-    const T xi[3] = {pi_.x, pi_.y, pi_.z};
-    const T hi = pi_.w;
+    {
+        const V4 pi_ = RP[i];
+        if constexpr (sizeof(T) == 4) st.own[lane] = make_float4(pi_.x, pi_.y, pi_.z, 2.0f / pi_.w);
+        else st.own[lane] = pi_;
+    }
     // half-box ties of the FP32 minimum image: the FP32 positions and their
     // difference carry at most 4 u X of rounding (X the largest coordinate
     // magnitude); 2^-18 (X + L) covers it
@@ -178,7 +216,6 @@ __global__ __launch_bounds__(256) void k_gravity(GravArgs<T> a)
             tie_band[k] = (float)((X + a.box.range[k]) * 3.814697265625e-06);
         }
     }
-    const T inv_ei = T(2) / hi;
     const T G = T(a.G);
     // compensated sums in blocks of at most 16 terms (fold below)
     BlockAcc<T> phi, ac[3];
@@ -188,7 +225,7 @@ __global__ __launch_bounds__(256) void k_gravity(GravArgs<T> a)
         for (int k = 0; k < D; ++k) ac[k].fold();
     };
     int since_fold = 0;  // node steps since the last fold (wave-uniform)
-    int inter = 0;
+    int inter = 0;  // of the wavefront
     // the lane takes part in the walk from node `resume` on; a lane that
     // accepted a node's monopole resumes at the node's subtree end
     int resume = valid ? 0 : INT_MAX;
@@ -204,12 +241,10 @@ __global__ __launch_bounds__(256) void k_gravity(GravArgs<T> a)
         return (g.l2 > a.theta2 * d2) || (d2 < g.l2);
     };
     const int mid = min((i0 & ~(kWave - 1)) + kWave / 2, a.n - 1);
-    const long long here = __builtin_amdgcn_readfirstlane(a.nbase[mid]);
-    const int k0 = seg >> 1;
-    const long long d0 = (long long)a.n_nodes * k0 * k0 / (a.nside * a.nside);
-    const long long d1 = (long long)a.n_nodes * (k0 + 1) * (k0 + 1) / (a.nside * a.nside);
-    int node = (int)((seg & 1) ? max(0ll, here - d1) : min((long long)a.n_nodes, here + d0));
-    const int node_end = (int)((seg & 1) ? max(0ll, here - d0) : min((long long)a.n_nodes, here + d1));
+    const int here = __builtin_amdgcn_readfirstlane(a.nbase[mid]);
+    const int d0 = a.bound[seg >> 1], d1 = a.bound[(seg >> 1) + 1];
+    int node = (seg & 1) ? max(0, here - d1) : min(a.n_nodes, here + d0);
+    const int node_end = (seg & 1) ? max(0, here - d0) : min(a.n_nodes, here + d1);
     if (node > 0 && node < node_end) {
         // a later piece: a lane that accepts an ancestor of the first node has
         // that subtree in the ancestor's piece and resumes behind it
@@ -233,102 +268,173 @@ __global__ __launch_bounds__(256) void k_gravity(GravArgs<T> a)
             fold();
             since_fold = 0;
         }
-        const GravNode g = a.node[node];
+        node = __builtin_amdgcn_readfirstlane(node);
+        const GravNode g = load_node(a.node + node);
         const bool act = node >= resume;
         double d[3] = {0, 0, 0};
         double d2 = 0.0;
-        const bool opened = opens(g, d, d2);
-        const bool open = act && opened;
-        if (act && !open) {
-            // monopole (src/bhtree.cpp:387-392)
-            const T r_inv = (sizeof(T) == 4) ? trsqrt(T(d2)) : tdiv(T(1.0), tsqrt(T(d2)));
-            const T gm = G * T(g.mass);
-            phi.add(-(gm * r_inv));
-            const T s = gm * (r_inv * r_inv * r_inv);
+        bool open = false;
+        // (a SIMD skips the 16 lanes of a pass that are all inactive: lanes that
+        // sit out the subtree are kept out of the test, too)
+        if (act) {
+            open = opens(g, d, d2);
+            if (!open) {
+                // monopole (src/bhtree.cpp:387-392)
+                const T r_inv = (sizeof(T) == 4) ? trsqrt(T(d2)) : tdiv(T(1.0), tsqrt(T(d2)));
+                const T gm = sizeof(T) == 4 ? T(g.gm) : G * T(g.mass);
+                const T s = gm * (r_inv * r_inv * r_inv);
+                if constexpr (sizeof(T) == 4) {
+                    phi.p = fmaf(-gm, r_inv, phi.p);
 #pragma unroll
-            for (int k = 0; k < D; ++k) ac[k].add(-(T(d[k]) * s));
-            ++inter;
-            resume = g.skip;
+                    for (int k = 0; k < D; ++k) ac[k].p = fmaf(-T(d[k]), s, ac[k].p);
+                } else {
+                    phi.add(-(gm * r_inv));
+#pragma unroll
+                    for (int k = 0; k < D; ++k) ac[k].add(-(T(d[k]) * s));
+                }
+                resume = g.skip;
+            }
         }
-        if (__ballot(open) == 0ull) {
+        const unsigned long long om = __builtin_amdgcn_ballot_w64(open);
+        inter += __popcll(__builtin_amdgcn_ballot_w64(act) & ~om);
+        if (om == 0ull) {
             node = g.skip;
             continue;
         }
         if (g.level < 0) {
-            // opened leaf: members staged 64 at a time, pair terms with every
-            // member j != i (src/bhtree.cpp:362-378)
-            for (int s0 = g.start; s0 < g.end; s0 += kWave) {
-                const int cnt = min(kWave, g.end - s0);
+            // opened leaf: pair terms with every member j != i
+            // (src/bhtree.cpp:362-378).  A quarter of the lanes open a leaf on
+            // average (of a third of the leaves at most four), so each opening
+            // lane's particle is given to G = 1, 2, 4, 8 or 16 lanes that take
+            // every G-th of the staged members; at most 16 terms a lane, then
+            // a tree over the G lanes, then one compensated addition.  1M
+            // Evrard, FP32: 3000 -> 2633 us a walk; 606k FP64: 8293 -> 5431.
+            // With fused multiply-adds, counts in scalar registers, the node
+            // record in one scalar load, the particles in LDS (64 VGPRs, 8
+            // waves a SIMD; 80 took 2640) and idle lanes out of the test: 2335
+            // and 5107.
+            const int np = __popcll(om);
+            const int lg = np > 32 ? 0 : np > 16 ? 1 : np > 8 ? 2 : np > 4 ? 3 : 4;
+            const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(om >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)om, 0));
+            const int chunk = lg == 1 ? 32 : kWave;
+            const int slot = lane >> lg;
+            for (int s0 = g.start; s0 < g.end; s0 += chunk) {
+                const int cnt = min(chunk, g.end - s0);
                 if (lane < cnt) {
                     const V4 pj = RP[s0 + lane];
                     const T mj = RV[s0 + lane].w;
                     if constexpr (sizeof(T) == 4) st.p[lane] = make_float4(pj.x, pj.y, pj.z, 2.0f / pj.w);
                     else st.p[lane] = pj;
-                    st.gm[lane] = G * mj;
+                    st.gm[lane] = T(0.5) * (G * mj);
                 }
+                if (open) st.lane[rank] = lane;
                 wave_lds_fence();
-                if (open) {
-                    fold();
-                    for (int t = 0; t < cnt; ++t) {
-                        if ((t & 15) == 15) fold();
-                        if (s0 + t == i) continue;
-                        const typename V4T<T>::type q = st.p[t];
-                        const T xj[3] = {q.x, q.y, q.z};
-                        T rij[3] = {0, 0, 0};
-                        T r2 = T(0);
+                const int src = lg == 0 ? lane : (slot < np ? st.lane[slot] : lane);
+                const bool work = lg == 0 ? open : slot < np;
+                const int is = (i0 & ~(kWave - 1)) + src;
+                const typename V4T<T>::type own = st.own[src];
+                const T xs[3] = {own.x, own.y, own.z};
+                const T es = own.w;
+                inter += np * cnt - __popcll(__builtin_amdgcn_ballot_w64(open && i >= s0 && i < s0 + cnt));
+                // blocks of 16 terms a lane: one, unless the particles keep
+                // their lanes
+                for (int t0 = lane & ((1 << lg) - 1); t0 < cnt || lg != 0; t0 += 16 << lg) {
+                    T bs[4] = {T(0), T(0), T(0), T(0)};
+                    if (work) {
+                        const int t1 = min(cnt, t0 + (16 << lg));
+                        for (int t = t0; t < t1; t += 1 << lg) {
+                            if (s0 + t == is) continue;
+                            const typename V4T<T>::type q = st.p[t];
+                            const T xj[3] = {q.x, q.y, q.z};
+                            T rij[3] = {0, 0, 0};
+                            T r2 = T(0);
 #pragma unroll
-                        for (int k = 0; k < D; ++k) rij[k] = grav_rij<P, T>(xi[k], xj[k], a.box, k);
-                        if constexpr (P && sizeof(T) == 4) {
-                            // a component within FP32 rounding of half the
-                            // box takes its image from the FP64 positions, as
-                            // the reference chooses it (the image, and with
-                            // it the sign, flips there)
-                            bool tie = false;
-#pragma unroll
-                            for (int k = 0; k < D; ++k)
-                                tie = tie || fabsf(fabsf(xi[k] - xj[k]) - 0.5f * a.box.rangef[k]) <= tie_band[k];
-                            if (tie)
+                            for (int k = 0; k < D; ++k) rij[k] = grav_rij<P, T>(xs[k], xj[k], a.box, k);
+                            if constexpr (P && sizeof(T) == 4) {
+                                // a component within FP32 rounding of half the
+                                // box takes its image from the FP64 positions, as
+                                // the reference chooses it (the image, and with
+                                // it the sign, flips there)
+                                bool tie = false;
 #pragma unroll
                                 for (int k = 0; k < D; ++k)
-                                    rij[k] = (T)rij_axis<double>(ri[k], a.x64[k][s0 + t], a.box, k);
-                        }
+                                    tie = tie || fabsf(fabsf(xs[k] - xj[k]) - 0.5f * a.box.rangef[k]) <= tie_band[k];
+                                if (tie)
 #pragma unroll
-                        for (int k = 0; k < D; ++k) r2 = (k == 0) ? rij[k] * rij[k] : r2 + rij[k] * rij[k];
-                        const T gm = st.gm[t];
-                        T fsum, gsum;
-                        if constexpr (sizeof(T) == 4) {
-                            // 1/r from one reciprocal square root, r = r^2 / r
-                            // (r = 0 for coincident particles: the polynomial
-                            // branch u < 1 takes no 1/r)
-                            const float inv_r = trsqrt(r2);
-                            const float r = r2 > 0.f ? r2 * inv_r : 0.f;
-                            // beyond both softening lengths (u >= 2 on both
-                            // sides, the usual case in an opened leaf) the
-                            // terms are 1/r and 1/r^3; the polynomials run
-                            // only when some lane of the wave has a near pair
-                            const bool near = r * inv_ei < 2.0f || r * q.w < 2.0f;
-                            if (__ballot(near)) {
-                                float fi, gi, fj, gj;
-                                hk_fg(r, inv_r, inv_ei, fi, gi);
-                                hk_fg(r, inv_r, q.w, fj, gj);
-                                fsum = fi + fj;
-                                gsum = gi + gj;
-                            } else {
-                                fsum = 2.0f * inv_r;
-                                gsum = 2.0f * (inv_r * inv_r * inv_r);
+                                    for (int k = 0; k < D; ++k)
+                                        rij[k] = (T)rij_axis<double>(a.x64[k][is], a.x64[k][s0 + t], a.box, k);
                             }
-                        } else {
-                            const T r = tsqrt(r2);
-                            fsum = hk_f(r, hi) + hk_f(r, q.w);
-                            gsum = hk_g(r, hi) + hk_g(r, q.w);
-                        }
-                        phi.add(-(gm * fsum * T(0.5)));
-                        const T s2 = gm * gsum * T(0.5);
 #pragma unroll
-                        for (int k = 0; k < D; ++k) ac[k].add(-(rij[k] * s2));
-                        ++inter;
+                            for (int k = 0; k < D; ++k) {
+                                if (k == 0) r2 = rij[k] * rij[k];
+                                else if constexpr (sizeof(T) == 4) r2 = fmaf(rij[k], rij[k], r2);
+                                else r2 += rij[k] * rij[k];
+                            }
+                            const T gm = st.gm[t];
+                            T fsum, gsum;
+                            if constexpr (sizeof(T) == 4) {
+                                // 1/r from one reciprocal square root, r = r^2 / r
+                                // (r = 0 for coincident particles: the polynomial
+                                // branch u < 1 takes no 1/r)
+                                const float inv_r = trsqrt(r2);
+                                const float r = r2 > 0.f ? r2 * inv_r : 0.f;
+                                // beyond both softening lengths (u >= 2 on both
+                                // sides, the usual case in an opened leaf) the
+                                // terms are 1/r and 1/r^3; the polynomials run
+                                // only when some lane of the wave has a near pair
+                                const bool near = r * es < 2.0f || r * q.w < 2.0f;
+                                if (__builtin_amdgcn_ballot_w64(near)) {
+                                    float fi, gi, fj, gj;
+                                    hk_fg(r, inv_r, es, fi, gi);
+                                    hk_fg(r, inv_r, q.w, fj, gj);
+                                    fsum = fi + fj;
+                                    gsum = gi + gj;
+                                } else {
+                                    fsum = 2.0f * inv_r;
+                                    gsum = 2.0f * (inv_r * inv_r * inv_r);
+                                }
+                            } else {
+                                const T r = tsqrt(r2);
+                                fsum = hk_f(r, es) + hk_f(r, q.w);
+                                gsum = hk_g(r, es) + hk_g(r, q.w);
+                            }
+                            const T s2 = gm * gsum;
+                            if constexpr (sizeof(T) == 4) {
+                                bs[3] = fmaf(-gm, fsum, bs[3]);
+#pragma unroll
+                                for (int k = 0; k < D; ++k) bs[k] = fmaf(-rij[k], s2, bs[k]);
+                            } else {
+                                bs[3] -= gm * fsum;
+#pragma unroll
+                                for (int k = 0; k < D; ++k) bs[k] -= rij[k] * s2;
+                            }
+                        }
                     }
-                    fold();
+                    // sum over the particle's lanes, back to its own lane
+                    if (lg != 0) {
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) bs[c] += dpp<0xB1>(bs[c]);
+                        if (lg > 1) {
+#pragma unroll
+                            for (int c = 0; c < 4; ++c) bs[c] += dpp<0x4E>(bs[c]);
+                        }
+                        if (lg > 2) {
+#pragma unroll
+                            for (int c = 0; c < 4; ++c) bs[c] += dpp<0x141>(bs[c]);
+                        }
+                        if (lg > 3) {
+#pragma unroll
+                            for (int c = 0; c < 4; ++c) bs[c] += dpp<0x140>(bs[c]);
+                        }
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) bs[c] = __shfl(bs[c], (rank << lg) & (kWave - 1), kWave);
+                    }
+                    if (open) {
+                        phi.add_block(bs[3]);
+#pragma unroll
+                        for (int k = 0; k < D; ++k) ac[k].add_block(bs[k]);
+                    }
+                    if (lg != 0) break;
                 }
                 wave_lds_fence();
             }
@@ -341,7 +447,6 @@ __global__ __launch_bounds__(256) void k_gravity(GravArgs<T> a)
 #pragma unroll
         for (int k = 0; k < D; ++k) q[(size_t)(k + 1) * a.n] = (double)ac[k].get();
     }
-    for (int off = kWave / 2; off > 0; off >>= 1) inter += __shfl_xor(inter, off, kWave);
     if (lane == 0) atomicAdd(stat_ptr(a.stats, 10), (unsigned long long)inter);
 }
 
@@ -368,9 +473,8 @@ __global__ void k_gravity_sum(int n, int nseg, const double *__restrict__ part, 
 // (8 fit a SIMD, 8192 the chip).  Evrard, FP32: 14k particles 801 -> 117 us,
 // 200k 1284 -> 807 (with 16384 / 32768 / 131072 wavefronts 914 / 812 / 873), 1M
 // 3603 -> 2961 (3326 / 3251 / 2911); FP64: 14k 1565 -> 318, 278k 5156 -> 4270,
-// 606k 9380 -> 8293.
+// 606k 9380 -> 8293 (all with one lane a particle in opened leaves).
 constexpr int kGravWaves = 65536;
-constexpr int kGravSideMax = 64;
 int grav_sides(int n)
 {
     const int waves = (n + kWave - 1) / kWave;
@@ -390,6 +494,7 @@ template <typename T> void launch_gravity(sphgpu_ctx *c, int nside)
     a.box = c->box;
     a.stats = c->dstats;
     a.nside = nside;
+    for (int k = 0; k <= nside; ++k) a.bound[k] = (int)((long long)a.n_nodes * k * k / ((long long)nside * nside));
     a.ngroups = grid_for(c->n, 256);
     a.nbase = c->tree.nbase;
     a.part = c->tree.gpart;
@@ -423,7 +528,7 @@ int gravity(sphgpu_ctx *c)
     }
     time_begin(c, "gravity_nodes");
     hipLaunchKernelGGL(k_grav_nodes, dim3(grid_for(t.n_nodes, 256)), dim3(256), 0, c->stream, t.n_nodes, t.node_cap,
-                       t.com, t.edge, t.mass, t.start, t.end, t.skip, t.level, t.gnode);
+                       t.com, t.edge, t.mass, t.start, t.end, t.skip, t.level, (float)c->prm.gravity_constant, t.gnode);
     time_end(c);
     const int nside = grav_sides(c->n), nseg = 2 * nside;
     if (nseg > t.gpart_seg) {

@@ -335,3 +335,67 @@ def test_node_kernel_sizes(n, dim, leaf):
     top = [h[a:a + k].max() for a, k in zip(d["first"], d["count"])]
     np.testing.assert_array_equal(d["kernel_size"], top)
     c.close()
+
+
+def _hk_pair(r, h):
+    """Softened f and g of one particle against several, by their own lengths."""
+    e = 0.5 * h
+    u = r / e
+    f1 = (-0.5 * u * u * (1 / 3 - 3 / 20 * u * u + u ** 3 / 20) + 1.4) / e
+    f2 = -1 / (15 * r) + (-u * u * (4 / 3 - u + 0.3 * u * u - u ** 3 / 30) + 1.6) / e
+    g1 = (4 / 3 - 1.2 * u * u + 0.5 * u ** 3) / e ** 3
+    g2 = (-1 / 15 + 8 / 3 * u ** 3 - 3 * u ** 4 + 1.2 * u ** 5 - u ** 6 / 6) / r ** 3
+    return np.where(u < 1, f1, np.where(u < 2, f2, 1 / r)), np.where(u < 1, g1, np.where(u < 2, g2, 1 / r ** 3))
+
+
+@pytest.mark.parametrize("prec,tol", [(ics.PAIR_FP64, 1e-12), (ics.PAIR_FP32, 2e-6)])
+@pytest.mark.parametrize("n,leaf,theta", [(40, 4, 0.5), (65, 1, 1.5), (700, 8, 0.5), (700, 33, 0.8), (900, 65, 0.5),
+                                          (1500, 140, 1.0), (3000, 32, 0.7)])
+def test_gravity_opened_leaves(n, leaf, theta, prec, tol):
+    """Leaves opened by any number of a wavefront's lanes (1, 2, 4, 8 or 16
+    lanes take one particle's members, 32 or 64 of them at a time) against the
+    walk of every particle by itself.  Tolerances as for the direct sum above:
+    20 u of the summed magnitudes in FP32."""
+    rng = np.random.default_rng([n, leaf, 5])
+    p = ics.default_params(3)
+    p.update(use_gravity=1, theta=theta, leaf_particle_num=leaf, pair_precision=prec, gravity_constant=0.7)
+    f = ics.empty_fields(n)
+    x = rng.normal(0, 1, (3, n))
+    f[ics.F_POS:ics.F_POS + 3] = x
+    m = f[ics.F_MASS] = rng.uniform(0.5, 1.5, n) / n
+    f[ics.F_DENS] = f[ics.F_ENE] = 1.0
+    h = f[ics.F_SML] = rng.uniform(0.1, 0.9, n)
+    c = sphgpu.Context(p, n)
+    c.upload(f)
+    c.build_tree()
+    d = c.tree_dump()
+    c.gravity()
+    out = c.download()
+    c.close()
+    level, e2, members = d["level"], d["edge"] ** 2, d["members"]
+    skip = [next((j for j in range(k + 1, len(level)) if level[j] <= level[k]), len(level)) for k in range(len(level))]
+    worst = 0.0
+    for i in range(0, n, max(1, n // 300)):
+        phi, acc, s_phi, s_acc, k = 0.0, np.zeros(3), 0.0, 0.0, 0
+        while k < len(level):
+            v = x[:, i] - d["com"][k]
+            r2 = (v * v).sum()
+            if e2[k] > theta * theta * r2 or r2 < e2[k]:
+                if d["is_leaf"][k]:
+                    j = members[d["first"][k]:d["first"][k] + d["count"][k]]
+                    j = j[j != i]
+                    dx = x[:, [i]] - x[:, j]
+                    r = np.sqrt((dx * dx).sum(axis=0))
+                    (fi, gi), (fj, gj) = _hk_pair(r, h[i]), _hk_pair(r, h[j])
+                    t = 0.35 * m[j] * (fi + fj)
+                    q = dx * (0.35 * m[j] * (gi + gj))
+                    phi, acc = phi - t.sum(), acc - q.sum(axis=1)
+                    s_phi, s_acc = s_phi + t.sum(), s_acc + (0.7 * m[j] / (r * r)).sum()
+                k += 1
+                continue
+            phi, acc = phi - 0.7 * d["mass"][k] / np.sqrt(r2), acc - 0.7 * d["mass"][k] / r2 ** 1.5 * v
+            s_phi, s_acc = s_phi + 0.7 * d["mass"][k] / np.sqrt(r2), s_acc + 0.7 * d["mass"][k] / r2
+            k = skip[k]
+        worst = max(worst, abs(out[ics.F_PHI, i] - phi) / s_phi,
+                    np.abs(out[ics.F_ACC:ics.F_ACC + 3, i] - acc).max() / s_acc)
+    assert worst < tol
