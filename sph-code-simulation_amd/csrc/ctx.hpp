@@ -40,6 +40,10 @@ enum RecField { R_POSH, R_VELM, R_THERMO, R_AUX, R_G0, R_G1, R_G2, R_G3, R_NREC 
 // in 3D go in one launch
 constexpr int kAlt = 20;
 
+// most pinned memory per context for uploads and downloads, two halves (a full
+// half takes 0.2 ms of DMA)
+constexpr size_t kBounceBytes = 16u << 20;
+
 // GSPH gradient rows in FP64 (grad_d[3], grad_p[3], grad_v[9])
 constexpr int kNGrad = 15;
 
@@ -177,6 +181,9 @@ struct sphgpu_ctx {
     bool mass_uniform = false;
     double mass_u = 0.0;
     double *stage = nullptr;     // host-exchange staging, [NFIELDS][n]
+    char *bounce = nullptr;      // pinned memory of the host exchange, two halves
+    size_t bounce_bytes = 0;
+    hipEvent_t bounce_moved[2] = {};  // a half's copy has ended
     double *red = nullptr;       // reduction partials
     int red_blocks = 0;
 

@@ -399,3 +399,37 @@ def test_gravity_opened_leaves(n, leaf, theta, prec, tol):
         worst = max(worst, abs(out[ics.F_PHI, i] - phi) / s_phi,
                     np.abs(out[ics.F_ACC:ics.F_ACC + 3, i] - acc).max() / s_acc)
     assert worst < tol
+
+
+@pytest.mark.parametrize("pinned", [False, True])
+@pytest.mark.parametrize("n", [1, 511, 4097, 13107, 26215, 52429, 131072, 1000003])
+def test_exchange_rows(n, pinned):
+    """Uploads and downloads of many and of few rows, in one or several rounds
+    through the pinned halves, and directly from pinned
+    memory: every masked row exactly, the others untouched."""
+    torch = pytest.importorskip("torch")
+    p = ics.default_params(3)
+    c = sphgpu.Context(p, n)
+    rows = [r for a in (ics.F_POS, ics.F_VEL, ics.F_ACC) for r in (a, a + 1, a + 2)]
+    rows += [ics.F_MASS, ics.F_DENS, ics.F_ENE, ics.F_SML]
+    rng = np.random.default_rng(n)
+    block = torch.empty((ics.NFIELDS if hasattr(ics, "NFIELDS") else sphgpu.NFIELDS, n), dtype=torch.float64,
+                        pin_memory=pinned)
+    f = block.numpy()
+    want = np.zeros_like(f)
+    f[:] = -7.0
+    for some in (rows, rows[2:6] + rows[11:], rows[:1]):
+        for r in some:
+            want[r] = f[r] = rng.random(n)
+        c.upload(f, sum(1 << r for r in some))
+        f[some] = -7.0  # the upload is complete when it returns
+        for part in (rows, rows[5:7], rows[-1:]):
+            got = c.download(sum(1 << r for r in part))
+            assert (got[part] == want[part]).all()
+            rest = np.setdiff1d(np.arange(f.shape[0]), part)
+            assert (got[rest] == 0).all()
+    f[:] = -7.0
+    c._check(c.lib.sphgpu_download(c.h, sphgpu._dp(f), sum(1 << r for r in rows)), "download")
+    assert (f[rows] == want[rows]).all()
+    assert (f[np.setdiff1d(np.arange(f.shape[0]), rows)] == -7.0).all()
+    c.close()
