@@ -111,13 +111,15 @@ struct Tree {
     int hist_blocks = 0;
     // node count and the partial-sort check, read together by the host
     int *sync_words = nullptr;         // [0] node count, [1] prefix run > leaf,
-                                       // [2] room taken in child
+                                       // [2] room taken in child, [3] a long
+                                       // run in the sort by the top bits
     int *host_words = nullptr;         // pinned host copy of sync_words
     hipEvent_t words_ready = nullptr;  // recorded after that copy
     // partial sorts order the keys on their top sorted_digits digits; a
     // failed check sorts that build fully (full_once) and adds 4 digits to
     // the later builds' partial sorts (full_sort once they cover the key)
     int sorted_digits = 8;
+    int sort_extra = 0;  // passes added to the top-bits sort of smaller sets
     bool full_once = false;
     bool full_sort = false;
     long long partial_sorts = 0, full_sorts = 0;

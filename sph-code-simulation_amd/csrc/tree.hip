@@ -141,6 +141,7 @@ __global__ void k_keys(const double *__restrict__ x, const double *__restrict__ 
         sync_words[0] = 0;
         sync_words[1] = 0;
         sync_words[2] = 0;
+        sync_words[3] = 0;
     }
     if (i >= sh.n) return;
     double pos[3] = {x[i], sh.dim > 1 ? y[i] : 0.0, sh.dim > 2 ? z[i] : 0.0};
@@ -460,16 +461,57 @@ __global__ __launch_bounds__(kScatterThreads) void k_radix_scatter(
         }
 }
 
+// Position of element e in the full order when the elements are in order of
+// key >> cut (and, among equals, in the order they came in): its run of equal
+// key >> cut is ordered by the whole key.  Keys are read four at a time.  A run
+// of more than kLongRun elements is reported.
+constexpr int kLongRun = 64;
+template <typename K> __device__ int place_in_run(const K *key, int n, int e, int cut, int *long_run)
+{
+    const unsigned long long k = key[e], top = k >> cut;
+    int dst = e, len = 1;
+    bool in = true;
+    for (int j = e - 1; in && j >= 0; j -= 4) {
+        unsigned long long q[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) q[u] = key[max(j - u, 0)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            in = in && j - u >= 0 && (q[u] >> cut) == top;
+            if (in) {
+                dst -= q[u] > k;
+                ++len;
+            }
+        }
+    }
+    in = true;
+    for (int j = e + 1; in && j < n; j += 4) {
+        unsigned long long q[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) q[u] = key[min(j + u, n - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            in = in && j + u < n && (q[u] >> cut) == top;
+            if (in) {
+                dst += q[u] < k;
+                ++len;
+            }
+        }
+    }
+    if (len > kLongRun) atomicOr(long_run, 1);
+    return dst;
+}
+
 // All passes of a small sort in one workgroup: at these sizes a pass of three
 // launches costs their latency alone (hist 4.3 us, scan 3.3, scatter 14.7 at
 // 4096 particles), so all passes run in one launch with the elements going
-// through LDS between them (5 passes of 4096: 25 us).  Element order, and with it the result, is that of
-// the tiled passes (both are stable).  One tile is the limit: at 14k (four times
+// through LDS between them (5 passes of 4096: 25 us, 2 and the order in the
+// cells: 16).  Element order, and with it the result, is that of the tiled passes (both are stable).  One tile is the limit: at 14k (four times
 // the rounds of one CU) a pass took 25 us, the tiled passes take 16.
 constexpr int kSmallMax = kSortTile;
-
 __global__ __launch_bounds__(kScatterThreads) void k_sort_small(unsigned long long *__restrict__ key, int *__restrict__ val,
-                                                                int n, int passes)
+                                                                int n, int cut,
+                                                                int passes, int *long_run)
 {
     __shared__ unsigned long long skey[kSmallMax];
     __shared__ int sval[kSmallMax];
@@ -492,7 +534,7 @@ __global__ __launch_bounds__(kScatterThreads) void k_sort_small(unsigned long lo
         v[r] = in ? val[e] : 0;
     }
     for (int p = 0; p < passes; ++p) {
-        const int shift = 8 * p;
+        const int shift = cut + 8 * p;
         for (int q = lane; q < 256; q += kWave) wcnt[w][q] = 0;
         sort_wave_fence();
 #pragma unroll
@@ -541,10 +583,23 @@ __global__ __launch_bounds__(kScatterThreads) void k_sort_small(unsigned long lo
     for (int r = 0; r < kScatterItems; ++r) {
         const int e = first + r * kWave;
         if (r < items && e < n) {
-            key[e] = k[r];
-            val[e] = v[r];
+            const int dst = cut > 0 ? place_in_run(skey, n, e, cut, long_run) : e;
+            key[dst] = k[r];
+            val[dst] = v[r];
         }
     }
+}
+
+// the same for larger sets, after the last of their passes
+__global__ void k_sort_runs(const unsigned long long *__restrict__ key, const int *__restrict__ val,
+                            unsigned long long *__restrict__ key_out, int *__restrict__ val_out, int n, int cut,
+                            int *long_run)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int dst = place_in_run(key, n, i, cut, long_run);
+    key_out[dst] = key[i];
+    val_out[dst] = val[i];
 }
 
 // ---- 3. permutation of the particle state -----------------------------------
@@ -1120,7 +1175,7 @@ int tree_alloc(sphgpu_ctx *c)
               al((void **)&t.child, 4ull * (t.node_cap + 8));
     const long long scan_max = std::max<long long>(std::max<long long>(n + 1, 256ll * t.hist_blocks), t.node_cap);
     ok = ok && al((void **)&t.scan_tmp, 4ull * ((scan_max + kScanTile - 1) / kScanTile + 1));
-    ok = ok && hipHostMalloc((void **)&t.host_words, 4ull * 2, hipHostMallocDefault) == hipSuccess &&
+    ok = ok && hipHostMalloc((void **)&t.host_words, 4ull * 4, hipHostMallocDefault) == hipSuccess &&
          hipEventCreateWithFlags(&t.words_ready, hipEventDisableTiming) == hipSuccess;
     if (!ok) return SPHGPU_E_NOMEM;
     if (c->prm.periodic) {
@@ -1233,19 +1288,44 @@ int tree_build(sphgpu_ctx *c)
             cut = key_bits - c->dim * ((key_bits - 8 * skip) / c->dim);
         }
     }
+    // Smaller sets take the passes over the top log2(n) + 2 bits, about as many
+    // cells as it takes to tell the particles apart, and put the few particles
+    // of a cell into the order of their whole keys by looking at each other
+    // (the order of the full sort).  3D, 14k particles: 2 passes of three
+    // launches and this one, 34 us, where 8 passes took 120; 2D, 4k in one
+    // workgroup: 25 -> 16 us.  It has to save two passes: one costs about what
+    // ordering the cells does.  A cell that holds many takes its square: when
+    // there is one, the context's later builds take two passes more.
+    int first_bit = 8 * skip, rounds = passes - skip, place = 0;
+    if (n < 65536) {
+        int bits = 2;
+        while ((1 << (bits - 2)) < n) ++bits;
+        const int keep = (bits + 7) / 8 + t.sort_extra;
+        if (keep + 2 <= passes) {
+            place = first_bit = key_bits - 8 * keep;
+            rounds = keep;
+        }
+    }
     // up to one tile of elements: all passes in one launch (k_sort_small)
     const bool small = n <= kSmallMax;
     if (small) {
-        hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(kScatterThreads), 0, c->stream, t.key, t.perm, n, passes);
+        hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(kScatterThreads), 0, c->stream, t.key, t.perm, n, first_bit, rounds,
+                           t.sync_words + 3);
     }
-    for (int p = skip; !small && p < passes; ++p) {
-        const int shift = 8 * p;
+    for (int p = 0; !small && p < rounds; ++p) {
+        const int shift = first_bit + 8 * p;
         hipLaunchKernelGGL(k_radix_hist, dim3(nb), dim3(kScatterThreads), 0, c->stream, (const unsigned long long *)t.key, n,
                            shift, t.hist, nb);
         scan_counts(c->stream, t.hist, t.hist, 256 * nb, t.scan_tmp, false);
         hipLaunchKernelGGL(k_radix_scatter, dim3(nb), dim3(kScatterThreads), 0, c->stream,
                            (const unsigned long long *)t.key, (const int *)t.perm, t.key_alt, t.perm_alt, n, shift,
                            (const unsigned int *)t.hist, nb);
+        std::swap(t.key, t.key_alt);
+        std::swap(t.perm, t.perm_alt);
+    }
+    if (!small && place > 0) {
+        hipLaunchKernelGGL(k_sort_runs, dim3(grid_for(n, 256)), dim3(256), 0, c->stream, (const unsigned long long *)t.key,
+                           (const int *)t.perm, t.key_alt, t.perm_alt, n, place, t.sync_words + 3);
         std::swap(t.key, t.key_alt);
         std::swap(t.perm, t.perm_alt);
     }
@@ -1270,7 +1350,7 @@ int tree_build(sphgpu_ctx *c)
     scan_counts(c->stream, (const unsigned *)t.ncount, (unsigned *)t.nbase, n, t.scan_tmp, true,
                 (unsigned *)t.sync_words);
     HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipMemcpyAsync(t.host_words, t.sync_words, 2 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipMemcpyAsync(t.host_words, t.sync_words, 4 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipEventRecord(t.words_ready, c->stream));
     hipLaunchKernelGGL(k_fill, dim3(grid_for(n, 128)), dim3(128), 0, c->stream, (const unsigned long long *)t.key,
                        (const unsigned char *)t.kdig, (const unsigned char *)t.lam, (const int *)t.nbase,
@@ -1310,6 +1390,7 @@ int tree_build(sphgpu_ctx *c)
     if (rc) return rc;
     HIPCHK(c, hipEventSynchronize(t.words_ready));
     const int total = t.host_words[0];
+    if (t.host_words[3]) t.sort_extra += 2;
     if (skip) {
         if (t.host_words[1]) {
             // a cell of the sorted depth holds more than a leaf: this build
