@@ -946,6 +946,12 @@ __device__ int group_end(const unsigned long long *__restrict__ key, int n, int 
     return lo + 1;
 }
 
+// A leaf of the deepest level holds any number of particles (coincident ones;
+// all of them where a run has blown up): eight lanes took 7.1 ms for the box of
+// a leaf of 1M, the whole workgroup takes 0.4.  The line lies well above the
+// leaf sizes in use, where a workgroup per leaf would leave its lanes idle.
+constexpr int kWideLeaf = 512, kWideLeaves = 32;
+
 // Per node: its end and skip, and the FP32 walk records of the neighbour search
 // (kernel_size is added by k_node_ks).  Internal nodes keep their cell (centre
 // rounded to nearest, half edge rounded up); a leaf gets the bounding box of its
@@ -966,6 +972,10 @@ __global__ __launch_bounds__(256) void k_node_records(
 {
     const int total = sync_words[0];
     if (total > cap || sync_words[1] != 0) return;
+    __shared__ int wide[kWideLeaves], n_wide;
+    __shared__ double part[2][256 / kWave];
+    if (threadIdx.x == 0) n_wide = 0;
+    __syncthreads();
     int leaves = 0, depth = 0;
     // kNodeLanes lanes per node share its search and a leaf's member loop
     const int sub = threadIdx.x % kNodeLanes;
@@ -981,7 +991,17 @@ __global__ __launch_bounds__(256) void k_node_records(
         else if (L > 1) e = group_end(key, sh.n, s, sh.bits * (sh.ml - (L - 1)), sub);
         double c[3] = {ncenter[idx], ncenter[(size_t)cap + idx], ncenter[2 * (size_t)cap + idx]};
         double h[3] = {0.5 * nedge[idx], 0.5 * nedge[idx], 0.5 * nedge[idx]};
-        if (leaf && e > s) {
+        // a wide leaf's box is left to the whole workgroup, while there is room
+        // to note it
+        bool later = false;
+        if (leaf && e - s > kWideLeaf) {
+            int slot = 0;
+            if (sub == 0) slot = atomicAdd(&n_wide, 1);
+            slot = __shfl(slot, 0, kNodeLanes);
+            later = slot < kWideLeaves;
+            if (later && sub == 0) wide[slot] = idx;
+        }
+        if (leaf && e > s && !later) {
             const double *p[3] = {px, py, pz};
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
@@ -1006,8 +1026,10 @@ __global__ __launch_bounds__(256) void k_node_records(
             const int skip = e < sh.n ? nbase[e] : total;
             nend[idx] = e;
             nskip[idx] = skip;
-            nbox[idx] = make_float4((float)c[0], (float)c[1], (float)c[2], float_up(h[0]));
-            nhalf[idx] = make_float2(float_up(h[1]), float_up(h[2]));
+            if (!later) {
+                nbox[idx] = make_float4((float)c[0], (float)c[1], (float)c[2], float_up(h[0]));
+                nhalf[idx] = make_float2(float_up(h[1]), float_up(h[2]));
+            }
             nlink[idx] = make_int4(s, e, skip, leaf ? (int)0x80000000 : 0);
             leaves += leaf ? 1 : 0;
             depth = max(depth, leaf ? L : 0);
@@ -1021,6 +1043,53 @@ __global__ __launch_bounds__(256) void k_node_records(
     if ((threadIdx.x & (kWave - 1)) == 0) {
         if (leaves) atomicAdd(stat_ptr(stats, 11), (unsigned long long)leaves);
         if (depth) atomicMax(stat_ptr(stats, 12), (unsigned long long)depth);
+    }
+    __syncthreads();
+    const int listed = min(n_wide, kWideLeaves);
+    for (int q = 0; q < listed; ++q) {
+        const int idx = wide[q], s = nstart[idx];
+        const int L = -nlevel[idx];
+        const int e = L <= sh.ml ? leaf_end[s] : group_end(key, sh.n, s, sh.bits * (sh.ml - (L - 1)), sub);
+        const double *p[3] = {px, py, pz};
+        double c[3] = {ncenter[idx], ncenter[(size_t)cap + idx], ncenter[2 * (size_t)cap + idx]};
+        double h[3] = {0.5 * nedge[idx], 0.5 * nedge[idx], 0.5 * nedge[idx]};
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            if (k >= sh.dim) break;
+            double lo = p[k][s], hi = lo;
+            for (int j = s + threadIdx.x; j < e; j += 8 * 256) {
+                double v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = p[k][min(j + u * 256, e - 1)];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    lo = v[u] < lo ? v[u] : lo;
+                    hi = v[u] > hi ? v[u] : hi;
+                }
+            }
+            for (int off = kWave / 2; off > 0; off >>= 1) {
+                const double ol = __shfl_xor(lo, off, kWave), oh = __shfl_xor(hi, off, kWave);
+                lo = ol < lo ? ol : lo;
+                hi = oh > hi ? oh : hi;
+            }
+            if ((threadIdx.x & (kWave - 1)) == 0) {
+                part[0][threadIdx.x / kWave] = lo;
+                part[1][threadIdx.x / kWave] = hi;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < 256 / kWave; ++w) {
+                lo = part[0][w] < lo ? part[0][w] : lo;
+                hi = part[1][w] > hi ? part[1][w] : hi;
+            }
+            __syncthreads();
+            c[k] = 0.5 * (lo + hi);
+            h[k] = 0.5 * (hi - lo) + 4.0 * 1.1102230246251565e-16 * (fabs(lo) + fabs(hi));
+        }
+        if (threadIdx.x == 0) {
+            nbox[idx] = make_float4((float)c[0], (float)c[1], (float)c[2], float_up(h[0]));
+            nhalf[idx] = make_float2(float_up(h[1]), float_up(h[2]));
+        }
     }
 }
 

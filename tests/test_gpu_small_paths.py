@@ -461,3 +461,27 @@ def test_key_sort_order_clustered(n, dim):
         moved = order != want
         assert (x[:, order[moved]] == x[:, want[moved]]).all()
     c.close()
+
+
+@pytest.mark.parametrize("dim,n,levels", [(2, 20000, 2), (3, 70000, 2), (1, 5000, 2), (3, 6000, 1)])
+def test_wide_leaves(dim, n, levels):
+    """Leaves of more than 512 particles (a shallow tree; more of them in one
+    workgroup than it notes, too): the search through their boxes finds the same
+    neighbours as through the leaves of the deep tree."""
+    p, f = _random_state(n, dim, seed=4)
+    f[ics.F_POS:ics.F_POS + dim] = np.random.default_rng(n).random((dim, n))
+    h = np.full(n, {1: 10 / n, 2: (10 / n) ** 0.5 / 2, 3: (10 / n) ** (1 / 3) / 2}[dim])
+    found = []
+    for ml in (levels, 20):
+        q = dict(p)
+        q["max_tree_level"] = ml
+        c = sphgpu.Context(q, n)
+        c.upload(f)
+        c.build_tree()
+        if ml == levels:
+            assert (c.tree_dump()["count"][c.tree_dump()["is_leaf"] == 1] > 512).any()
+        count, lists = c.neighbor_sets(h, 0, cap=128)
+        found.append((count, np.sort(np.where(np.arange(128) < count[:, None], lists, n), axis=1)))
+        c.close()
+    np.testing.assert_array_equal(found[0][0], found[1][0])
+    np.testing.assert_array_equal(found[0][1], found[1][1])
