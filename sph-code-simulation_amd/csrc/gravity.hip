@@ -174,8 +174,21 @@ SPH_DEV GravNode load_node(const GravNode *p)
     return u.g;
 }
 
+// Wavefronts a SIMD that the walk is compiled for (512 registers shared by
+// them).  The FP32 forms are bound by latency and arithmetic together and take 8
+// (64 registers), which spills 6 in open 3D (1M particles 1979 us; 7 wavefronts
+// without a spill 2038) and 12 in periodic 2D (262k 381 us; without a spill
+// 393).  Periodic 3D, with the image and its tie test for every pair, would
+// spill 37 into the pair loop: at 8 wavefronts 205k particles took 2838 us and
+// 1M 10776, at 6 (80 registers, 7 reloaded per opened leaf) 1231 and 5097, at 5
+// without a spill 1314 and 5397.  FP64 fits 4 without a spill (94 registers).
+template <int D, typename T, bool P> constexpr int grav_waves_per_simd()
+{
+    return sizeof(T) == 8 ? 4 : (P && D == 3 ? 6 : 8);
+}
+
 template <int D, typename T, bool P>
-__global__ __launch_bounds__(256, sizeof(T) == 4 ? 8 : 4) void k_gravity(GravArgs<T> a)
+__global__ __launch_bounds__(256, (grav_waves_per_simd<D, T, P>())) void k_gravity(GravArgs<T> a)
 {
     __shared__ GravStage<T> stage[4];
     GravStage<T> &st = stage[(threadIdx.x >> 6) & 3];
@@ -310,9 +323,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 8 : 4) void k_gravity(GravArg
             // a tree over the G lanes, then one compensated addition.  1M
             // Evrard, FP32: 3000 -> 2633 us a walk; 606k FP64: 8293 -> 5431.
             // With fused multiply-adds, counts in scalar registers, the node
-            // record in one scalar load, the particles in LDS (64 VGPRs, 8
-            // waves a SIMD; 80 took 2640) and idle lanes out of the test: 2335
-            // and 5107.
+            // record in one scalar load, the particles in LDS (8 waves a SIMD;
+            // 6 took 2640) and idle lanes out of the test: 2335 and 5107.
             const int np = __popcll(om);
             const int lg = np > 32 ? 0 : np > 16 ? 1 : np > 8 ? 2 : np > 4 ? 3 : 4;
             const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(om >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)om, 0));
