@@ -40,6 +40,8 @@ enum RecField { R_POSH, R_VELM, R_THERMO, R_AUX, R_G0, R_G1, R_G2, R_G3, R_NREC 
 // in 3D go in one launch
 constexpr int kAlt = 20;
 
+constexpr int kSyncWords = 5;  // Tree::sync_words
+
 // most pinned memory per context for uploads and downloads, two halves (a full
 // half takes 0.2 ms of DMA)
 constexpr size_t kBounceBytes = 16u << 20;
@@ -109,17 +111,18 @@ struct Tree {
     // radix sort scratch
     unsigned int *hist = nullptr;
     int hist_blocks = 0;
-    // node count and the partial-sort check, read together by the host
-    int *sync_words = nullptr;         // [0] node count, [1] prefix run > leaf,
-                                       // [2] room taken in child, [3] a long
-                                       // run in the sort by the top bits
+    // words that the build's kernels leave, read together by the host: [0] node
+    // count, [1] the sort's check failed (the build is repeated), [2] room taken
+    // in child, [3] top key bits that separate crowded cells, [4] the sort
+    // met a crowded cell
+    int *sync_words = nullptr;
     int *host_words = nullptr;         // pinned host copy of sync_words
     hipEvent_t words_ready = nullptr;  // recorded after that copy
     // partial sorts order the keys on their top sorted_digits digits; a
     // failed check sorts that build fully (full_once) and adds 4 digits to
     // the later builds' partial sorts (full_sort once they cover the key)
     int sorted_digits = 8;
-    int sort_extra = 0;  // passes added to the top-bits sort of smaller sets
+    int sort_keep = 0;  // passes of the top-bits sort of smaller sets, where cells are crowded
     bool full_once = false;
     bool full_sort = false;
     long long partial_sorts = 0, full_sorts = 0;

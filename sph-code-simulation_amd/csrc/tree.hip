@@ -137,11 +137,9 @@ __global__ void k_keys(const double *__restrict__ x, const double *__restrict__ 
                        int *__restrict__ perm, int *__restrict__ sync_words)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0) {  // node count, partial-sort check, child-list room
-        sync_words[0] = 0;
-        sync_words[1] = 0;
-        sync_words[2] = 0;
-        sync_words[3] = 0;
+    if (i == 0) {
+#pragma unroll
+        for (int q = 0; q < kSyncWords; ++q) sync_words[q] = 0;
     }
     if (i >= sh.n) return;
     double pos[3] = {x[i], sh.dim > 1 ? y[i] : 0.0, sh.dim > 2 ? z[i] : 0.0};
@@ -463,13 +461,17 @@ __global__ __launch_bounds__(kScatterThreads) void k_radix_scatter(
 
 // Position of element e in the full order when the elements are in order of
 // key >> cut (and, among equals, in the order they came in): its run of equal
-// key >> cut is ordered by the whole key.  Keys are read four at a time.  A run
-// of more than kLongRun elements is reported.
+// key >> cut is ordered by the whole key, read four keys at a time, and len is its
+// length.  In a run of more than MOST all elements find that out, by the length
+// or (in runs of thousands) by the element MOST before or behind, and stay where
+// they are, so the order stays a permutation.
 constexpr int kLongRun = 64;
-template <typename K> __device__ int place_in_run(const K *key, int n, int e, int cut, int *long_run)
+template <int MOST> __device__ int place_in_run(const unsigned long long *key, int n, int e, int cut, int &len)
 {
     const unsigned long long k = key[e], top = k >> cut;
-    int dst = e, len = 1;
+    auto in_run = [&](int j) { return j >= 0 && j < n && (key[j] >> cut) == top; };
+    int dst = e;
+    len = 1;
     bool in = true;
     for (int j = e - 1; in && j >= 0; j -= 4) {
         unsigned long long q[4];
@@ -483,8 +485,11 @@ template <typename K> __device__ int place_in_run(const K *key, int n, int e, in
                 ++len;
             }
         }
+        if (MOST > 256 && in && len == 5 && (in_run(e - MOST) || in_run(e + MOST))) len = MOST + 1;
+        if (len > MOST) return e;
     }
     in = true;
+    const int left = len;
     for (int j = e + 1; in && j < n; j += 4) {
         unsigned long long q[4];
 #pragma unroll
@@ -497,8 +502,9 @@ template <typename K> __device__ int place_in_run(const K *key, int n, int e, in
                 ++len;
             }
         }
+        if (MOST > 256 && in && len == left + 4 && in_run(e + MOST)) len = MOST + 1;
+        if (len > MOST) return e;
     }
-    if (len > kLongRun) atomicOr(long_run, 1);
     return dst;
 }
 
@@ -506,12 +512,15 @@ template <typename K> __device__ int place_in_run(const K *key, int n, int e, in
 // launches costs their latency alone (hist 4.3 us, scan 3.3, scatter 14.7 at
 // 4096 particles), so all passes run in one launch with the elements going
 // through LDS between them (5 passes of 4096: 25 us, 2 and the order in the
-// cells: 16).  Element order, and with it the result, is that of the tiled passes (both are stable).  One tile is the limit: at 14k (four times
-// the rounds of one CU) a pass took 25 us, the tiled passes take 16.
+// cells: 16).  Element order, and with it the result, is that of the tiled
+// passes (both are stable).  A cell with too many elements to order them there
+// adds all the passes, over the whole keys, and is reported.  One tile is the
+// limit: at 14k (four times the rounds of one CU) a pass took 25 us, the tiled
+// passes take 16.
 constexpr int kSmallMax = kSortTile;
 __global__ __launch_bounds__(kScatterThreads) void k_sort_small(unsigned long long *__restrict__ key, int *__restrict__ val,
-                                                                int n, int cut,
-                                                                int passes, int *long_run)
+                                                                int n, int cut, int passes, int all_passes,
+                                                                int *__restrict__ long_run)
 {
     __shared__ unsigned long long skey[kSmallMax];
     __shared__ int sval[kSmallMax];
@@ -533,73 +542,90 @@ __global__ __launch_bounds__(kScatterThreads) void k_sort_small(unsigned long lo
         k[r] = in ? key[e] : ~0ull;
         v[r] = in ? val[e] : 0;
     }
-    for (int p = 0; p < passes; ++p) {
-        const int shift = cut + 8 * p;
-        for (int q = lane; q < 256; q += kWave) wcnt[w][q] = 0;
-        sort_wave_fence();
+    for (;;) {
+        for (int p = 0; p < passes; ++p) {
+            const int shift = cut + 8 * p;
+            for (int q = lane; q < 256; q += kWave) wcnt[w][q] = 0;
+            sort_wave_fence();
 #pragma unroll
-        for (int r = 0; r < kScatterItems; ++r) {
-            if (r >= items) break;  // uniform
-            rank[r] = wave_digit_rank((unsigned)(k[r] >> shift) & 255u, lt, wcnt[w]);
-        }
-        __syncthreads();
-        // exclusive scan of the digits' counts (digit tid, four wavefronts)
-        unsigned sum = 0, x = 0;
-        if (tid < 256) {
-#pragma unroll
-            for (int q = 0; q < kScatterWaves; ++q) sum += wcnt[q][tid];
-            x = sum;
-            for (int off = 1; off < kWave; off <<= 1) {
-                const unsigned y = __shfl_up(x, off, kWave);
-                if (lane >= off) x += y;
+            for (int r = 0; r < kScatterItems; ++r) {
+                if (r >= items) break;  // uniform
+                rank[r] = wave_digit_rank((unsigned)(k[r] >> shift) & 255u, lt, wcnt[w]);
             }
-            if (lane == kWave - 1) wtot[w] = x;
-        }
-        __syncthreads();
-        if (tid < 256) {
-            unsigned run = x - sum;
-            for (int q = 0; q < w; ++q) run += wtot[q];
-            wave_digit_starts(wcnt, tid, run);
-        }
-        __syncthreads();
+            __syncthreads();
+            // exclusive scan of the digits' counts (digit tid, four wavefronts)
+            unsigned sum = 0, x = 0;
+            if (tid < 256) {
 #pragma unroll
-        for (int r = 0; r < kScatterItems; ++r)
-            if (r < items && first + r * kWave < n) {
-                const unsigned dst = wcnt[w][(unsigned)(k[r] >> shift) & 255u] + rank[r];
-                skey[dst] = k[r];
-                sval[dst] = v[r];
+                for (int q = 0; q < kScatterWaves; ++q) sum += wcnt[q][tid];
+                x = sum;
+                for (int off = 1; off < kWave; off <<= 1) {
+                    const unsigned y = __shfl_up(x, off, kWave);
+                    if (lane >= off) x += y;
+                }
+                if (lane == kWave - 1) wtot[w] = x;
             }
-        __syncthreads();
+            __syncthreads();
+            if (tid < 256) {
+                unsigned run = x - sum;
+                for (int q = 0; q < w; ++q) run += wtot[q];
+                wave_digit_starts(wcnt, tid, run);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < kScatterItems; ++r)
+                if (r < items && first + r * kWave < n) {
+                    const unsigned to = wcnt[w][(unsigned)(k[r] >> shift) & 255u] + rank[r];
+                    skey[to] = k[r];
+                    sval[to] = v[r];
+                }
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < kScatterItems; ++r) {
+                const int e = first + r * kWave;
+                if (r < items && e < n) {
+                    k[r] = skey[e];
+                    v[r] = sval[e];
+                }
+            }
+        }
+        bool crowded = false;
 #pragma unroll
         for (int r = 0; r < kScatterItems; ++r) {
             const int e = first + r * kWave;
             if (r < items && e < n) {
-                k[r] = skey[e];
-                v[r] = sval[e];
+                int dst = e, len = 0;
+                if (cut > 0) dst = place_in_run<kLongRun>(skey, n, e, cut, len);
+                crowded = crowded || len > kLongRun;
+                key[dst] = k[r];
+                val[dst] = v[r];
             }
         }
-    }
-#pragma unroll
-    for (int r = 0; r < kScatterItems; ++r) {
-        const int e = first + r * kWave;
-        if (r < items && e < n) {
-            const int dst = cut > 0 ? place_in_run(skey, n, e, cut, long_run) : e;
-            key[dst] = k[r];
-            val[dst] = v[r];
-        }
+        if (cut == 0 || !__syncthreads_or(crowded)) return;
+        if (tid == 0) *long_run = 1;
+        cut = 0;
+        passes = all_passes;
     }
 }
 
-// the same for larger sets, after the last of their passes
+// The order in the cells for larger sets, after the last of their passes.  A
+// cell of more than kLongRun elements is reported (flag[4]); where one holds more
+// than kMostRun, flag[1] says that this build is to be repeated (m elements of a
+// cell take 0.07 us each, 3000 of 60000 190 us; the repeated build 110 to 170).
+constexpr int kMostRun = 1024;
 __global__ void k_sort_runs(const unsigned long long *__restrict__ key, const int *__restrict__ val,
                             unsigned long long *__restrict__ key_out, int *__restrict__ val_out, int n, int cut,
-                            int *long_run)
+                            int *__restrict__ flag)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int dst = place_in_run(key, n, i, cut, long_run);
-    key_out[dst] = key[i];
-    val_out[dst] = val[i];
+    int len = 0;
+    if (i < n) {
+        const int dst = place_in_run<kMostRun>(key, n, i, cut, len);
+        key_out[dst] = key[i];
+        val_out[dst] = val[i];
+    }
+    const bool crowded = __ballot(len > kLongRun), repeat = __ballot(len > kMostRun);
+    if (crowded && (threadIdx.x & (kWave - 1)) == 0) atomicOr(flag + (repeat ? 1 : 4), 1);
 }
 
 // ---- 3. permutation of the particle state -----------------------------------
@@ -641,12 +667,28 @@ __device__ void check_prefix(const unsigned long long *key, const TreeShape &sh,
     if (__ballot(bad) && (threadIdx.x & (kWave - 1)) == 0) atomicOr(flag + 1, 1);
 }
 
+// The top bits of the key that separate the particles into cells of at most
+// kLongRun / 2, at position i (seen >= 0): flag[3] = their largest number, where
+// it is more than `seen`
+__device__ void cell_bits(const unsigned long long *key, const TreeShape &sh, int i, int seen, int *flag)
+{
+    int need = 0;
+    if (i + kLongRun / 2 < sh.n) {
+        const unsigned long long x = key[i] ^ key[i + kLongRun / 2];
+        const int key_bits = sh.bits * sh.ml;
+        need = x == 0 ? key_bits + 1 : key_bits - (63 - __clzll((long long)x));
+    }
+    for (int off = kWave / 2; off > 0; off >>= 1) need = max(need, __shfl_xor(need, off, kWave));
+    if ((threadIdx.x & (kWave - 1)) == 0 && need > seen && need > *(volatile int *)(flag + 3)) atomicMax(flag + 3, need);
+}
+
 // (leaves of more than 64 particles; k_lambda does it itself otherwise)
 __global__ void k_kdig(const unsigned long long *__restrict__ key, TreeShape sh, unsigned char *__restrict__ kdig,
-                       int cut, int *__restrict__ flag)
+                       int cut, int seen, int *__restrict__ flag)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (cut >= 0) check_prefix(key, sh, i, cut, flag);
+    if (seen >= 0) cell_bits(key, sh, i, seen, flag);
     if (i >= sh.n) return;
     if (i == 0) { kdig[0] = 0; return; }
     kdig[i] = (unsigned char)first_difference(key[i - 1], key[i], sh);
@@ -657,7 +699,7 @@ constexpr int kLambdaThreads = 128;
 
 __global__ void k_lambda(const unsigned long long *__restrict__ key, unsigned char *__restrict__ kdig, TreeShape sh,
                          unsigned char *__restrict__ lam, int *__restrict__ leaf_end, int *__restrict__ ncount, int cut,
-                         int *__restrict__ flag)
+                         int seen, int *__restrict__ flag)
 {
     // per thread and level t: the nearest boundary with kdig <= t to the
     // left (offset <= 0) and to the right (offset >= 1) of i, in LDS (a
@@ -675,6 +717,7 @@ __global__ void k_lambda(const unsigned long long *__restrict__ key, unsigned ch
             s_kd[t] = (j <= 0 || j >= sh.n) ? (unsigned char)0 : (unsigned char)first_difference(key[j - 1], key[j], sh);
         }
         if (cut >= 0) check_prefix(key, sh, i, cut, flag);
+        if (seen >= 0) cell_bits(key, sh, i, seen, flag);
         __syncthreads();
         if (i >= sh.n) return;
         kdig[i] = s_kd[i - wb];
@@ -1229,7 +1272,7 @@ int tree_alloc(sphgpu_ctx *c)
     t.hist_blocks = (n + kSortTile - 1) / kSortTile;
     bool ok = al((void **)&t.key, 8ull * n) && al((void **)&t.key_alt, 8ull * n) && al((void **)&t.perm, 4ull * n) &&
               al((void **)&t.perm_alt, 4ull * n) && al((void **)&t.kdig, n) && al((void **)&t.lam, n) &&
-              al((void **)&t.sync_words, 4ull * 4) &&
+              al((void **)&t.sync_words, 4ull * kSyncWords) &&
               al((void **)&t.leaf_end, 4ull * n) && al((void **)&t.ncount, 4ull * (n + 1)) &&
               al((void **)&t.nbase, 4ull * (n + 1)) && al((void **)&t.start, 4ull * t.node_cap) &&
               al((void **)&t.end, 4ull * t.node_cap) && al((void **)&t.skip, 4ull * t.node_cap) &&
@@ -1244,7 +1287,7 @@ int tree_alloc(sphgpu_ctx *c)
               al((void **)&t.child, 4ull * (t.node_cap + 8));
     const long long scan_max = std::max<long long>(std::max<long long>(n + 1, 256ll * t.hist_blocks), t.node_cap);
     ok = ok && al((void **)&t.scan_tmp, 4ull * ((scan_max + kScanTile - 1) / kScanTile + 1));
-    ok = ok && hipHostMalloc((void **)&t.host_words, 4ull * 4, hipHostMallocDefault) == hipSuccess &&
+    ok = ok && hipHostMalloc((void **)&t.host_words, 4ull * kSyncWords, hipHostMallocDefault) == hipSuccess &&
          hipEventCreateWithFlags(&t.words_ready, hipEventDisableTiming) == hipSuccess;
     if (!ok) return SPHGPU_E_NOMEM;
     if (c->prm.periodic) {
@@ -1363,23 +1406,27 @@ int tree_build(sphgpu_ctx *c)
     // (the order of the full sort).  3D, 14k particles: 2 passes of three
     // launches and this one, 34 us, where 8 passes took 120; 2D, 4k in one
     // workgroup: 25 -> 16 us.  It has to save two passes: one costs about what
-    // ordering the cells does.  A cell that holds many takes its square: when
-    // there is one, the context's later builds take two passes more.
-    int first_bit = 8 * skip, rounds = passes - skip, place = 0;
+    // ordering the cells does.  A cell costs its square, so after a build with a
+    // cell of more than kLongRun particles the next one sorts on the whole keys
+    // (the same one, where a cell is far larger), and later ones take as many
+    // passes as leave no cell more than half of that; all of these look again how
+    // many that is, down to the first number.
+    int first_bit = 8 * skip, rounds = passes - skip, place = 0, seen = -1;
     if (n < 65536) {
         int bits = 2;
         while ((1 << (bits - 2)) < n) ++bits;
-        const int keep = (bits + 7) / 8 + t.sort_extra;
+        const int least = (bits + 7) / 8, keep = std::max(least, t.sort_keep);
         if (keep + 2 <= passes) {
             place = first_bit = key_bits - 8 * keep;
             rounds = keep;
         }
+        if (least + 2 <= passes && keep > least) seen = 8 * least;
     }
     // up to one tile of elements: all passes in one launch (k_sort_small)
     const bool small = n <= kSmallMax;
     if (small) {
         hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(kScatterThreads), 0, c->stream, t.key, t.perm, n, first_bit, rounds,
-                           t.sync_words + 3);
+                           passes, t.sync_words + 4);
     }
     for (int p = 0; !small && p < rounds; ++p) {
         const int shift = first_bit + 8 * p;
@@ -1394,7 +1441,7 @@ int tree_build(sphgpu_ctx *c)
     }
     if (!small && place > 0) {
         hipLaunchKernelGGL(k_sort_runs, dim3(grid_for(n, 256)), dim3(256), 0, c->stream, (const unsigned long long *)t.key,
-                           (const int *)t.perm, t.key_alt, t.perm_alt, n, place, t.sync_words + 3);
+                           (const int *)t.perm, t.key_alt, t.perm_alt, n, place, t.sync_words);
         std::swap(t.key, t.key_alt);
         std::swap(t.perm, t.perm_alt);
     }
@@ -1409,17 +1456,17 @@ int tree_build(sphgpu_ctx *c)
     time_begin(c, "tree_nodes");
     if (sh.leaf > 64)
         hipLaunchKernelGGL(k_kdig, dim3(grid_for(n, 256)), dim3(256), 0, c->stream, (const unsigned long long *)t.key, sh,
-                           t.kdig, skip ? cut : -1, t.sync_words);
+                           t.kdig, skip ? cut : -1, seen, t.sync_words);
     const size_t lam_lds = sh.leaf <= 64 ? (size_t)sh.leaf * kLambdaThreads : sizeof(short) * 2 * (size_t)(sh.ml + 1) * kLambdaThreads;
     hipLaunchKernelGGL(k_lambda, dim3(grid_for(n, kLambdaThreads)), dim3(kLambdaThreads), lam_lds,
                        c->stream, (const unsigned long long *)t.key, t.kdig, sh, t.lam, t.leaf_end, t.ncount,
-                       skip ? cut : -1, t.sync_words);
+                       skip ? cut : -1, seen, t.sync_words);
     // the node count goes to nbase[n] and to sync_words[0] (read by the fill
     // on the device and copied to the host)
     scan_counts(c->stream, (const unsigned *)t.ncount, (unsigned *)t.nbase, n, t.scan_tmp, true,
                 (unsigned *)t.sync_words);
     HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipMemcpyAsync(t.host_words, t.sync_words, 4 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipMemcpyAsync(t.host_words, t.sync_words, kSyncWords * sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipEventRecord(t.words_ready, c->stream));
     hipLaunchKernelGGL(k_fill, dim3(grid_for(n, 128)), dim3(128), 0, c->stream, (const unsigned long long *)t.key,
                        (const unsigned char *)t.kdig, (const unsigned char *)t.lam, (const int *)t.nbase,
@@ -1459,7 +1506,14 @@ int tree_build(sphgpu_ctx *c)
     if (rc) return rc;
     HIPCHK(c, hipEventSynchronize(t.words_ready));
     const int total = t.host_words[0];
-    if (t.host_words[3]) t.sort_extra += 2;
+    if (place && t.host_words[1]) {
+        // a cell held too many to order them there: sort on the whole keys
+        // (the state is in the order of the top bits; equal keys keep theirs)
+        t.sort_keep = passes;
+        return tree_build(c);
+    }
+    if (t.host_words[4]) t.sort_keep = passes;
+    else if (seen >= 0) t.sort_keep = std::min(t.sort_keep, (t.host_words[3] + 7) / 8);
     if (skip) {
         if (t.host_words[1]) {
             // a cell of the sorted depth holds more than a leaf: this build

@@ -43,3 +43,90 @@ def test_periodic_fp32_walk_cost():
         t[prec] = c.kernel_times()["gravity"][0]
         c.close()
     assert t[ics.PAIR_FP32] < 0.8 * t[ics.PAIR_FP64], t
+
+
+def _keys(p, x):
+    """Octant keys (src/bhtree.cpp:211-239: one digit per level from pos > centre,
+    centres by the same FP64 recursion) in the unit box."""
+    c = np.full_like(x, 0.5)
+    e, key = 1.0, np.zeros(x.shape[1], dtype=np.uint64)
+    for _ in range(p["max_tree_level"]):
+        up = x > c
+        c = c + np.where(up, 1.0, -1.0) * (e * 0.25)
+        e *= 0.5
+        key = (key << np.uint64(x.shape[0])) | sum(u.astype(np.uint64) << np.uint64(k) for k, u in enumerate(up))
+    return key
+
+
+def _sort_ms(c):
+    """GPU time of the next tree build's sort (all its launches)."""
+    c.enable_timing(0)
+    c.enable_timing(1)
+    c.build_tree()
+    avg, count = c.kernel_times()["tree_sort"]
+    return avg * count
+
+
+def _crowded(dim, n, m, seed=0):
+    """_box with m particles in a cube of 1e-4 inside one cell of level 13 (one
+    cell for the sort's top bits: at most 24)."""
+    p, f = _box(dim, n, seed)
+    p["leaf_particle_num"] = 8
+    x = f[ics.F_POS:ics.F_POS + dim]
+    spread = x.copy()
+    x[:, :m] = 1228 / 4096 + 1e-5 + 1e-4 * x[:, :m]
+    return p, f, spread
+
+
+@pytest.mark.parametrize("dim,n,m", [(3, 60000, 15000), (2, 60000, 15000), (3, 60000, 60000), (3, 4000, 4000), (2, 4000, 1000)])
+def test_sort_cost_of_a_crowded_cell(dim, n, m):
+    """Sets whose particles crowd into one of the cells that the sort below 65536
+    particles orders by itself: at the most its passes over the top bits, and
+    then all passes, where the square of the crowd took 20 times the sort of
+    spread particles (bound here: 8 times; all passes are 3 to 4 times), and the
+    context sorts spread particles as fast as ever afterwards."""
+    p, f, spread = _crowded(dim, n, m)
+    first, plain, after = [], [], []
+    for _ in range(3):
+        c = sphgpu.Context(p, n)
+        g = f.copy()
+        g[ics.F_POS:ics.F_POS + dim] = spread
+        c.upload(g)
+        for _ in range(3):
+            plain.append(_sort_ms(c))
+        c.close()
+        c = sphgpu.Context(p, n)
+        c.upload(f)
+        first.append(max(_sort_ms(c) for _ in range(4)))
+        c.upload(g)
+        for _ in range(3):
+            after.append(_sort_ms(c))
+        c.close()
+    assert min(first) < 8 * min(plain), (first, plain)
+    assert min(after) < 1.3 * min(plain), (after, plain)
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("n", [1500, 4096, 9001, 65535])
+@pytest.mark.parametrize("m", [31, 32, 33, 63, 64, 65, 66, 700, 1023, 1024, 1025, 1030])
+def test_sort_order_of_a_crowded_cell(dim, n, m):
+    """The stable order of the whole keys, with one cell on either side of the
+    sizes that the sort orders in place (64 up to 4096 particles, 1024 beyond, 32
+    in later builds), for the first builds of a context and after the crowd has dispersed."""
+    p, f, spread = _crowded(dim, n, m, seed=m)
+    x = f[ics.F_POS:ics.F_POS + dim]
+    x[:, m // 2] = x[:, 0]  # equal keys inside the crowd
+    x[:] = x[:, np.random.default_rng(m).permutation(n)]
+    c = sphgpu.Context(p, n)
+    before = np.arange(n)
+    for state in (x.copy(), None, None, spread, None, x.copy(), None):
+        if state is not None:
+            f[ics.F_POS:ics.F_POS + dim] = state
+            key = _keys(p, state)
+            c.upload(f)
+        c.build_tree()
+        # the stable order of the keys, equal ones as the build before left them
+        want = before[np.argsort(key[before], kind="stable")]
+        before = c.tree_dump()["members"]
+        np.testing.assert_array_equal(before, want)
+    c.close()
