@@ -1475,13 +1475,17 @@ int tree_build(sphgpu_ctx *c)
     HIPCHK(c, hipGetLastError());
     time_end(c);
     // the node passes loop over the device's node count; their grids follow the
-    // last build's (or a guess), so nothing waits for the host here.  Positions
-    // are read from the permuted (key-ordered) arrays.
+    // last build's (or a guess), so nothing waits for the host here.  They are no
+    // smaller than for one node to 16 particles: after a build with few nodes
+    // (coincident particles) the grid would be left with some blocks for all of
+    // the next ones (200000 particles, leaves of 8: 1100 us instead of 23).
+    // Positions are read from the permuted (key-ordered) arrays.
     px = c->pos[0];
     py = c->dim > 1 ? c->pos[1] : c->pos[0];
     pz = c->dim > 2 ? c->pos[2] : c->pos[0];
     time_begin(c, "tree_node_records");
-    const long long guess = std::min<long long>(t.node_cap, (t.n_nodes > 0 ? t.n_nodes : n / 4) * 5ll / 4 + 256);
+    const long long nodes = t.n_nodes > 0 ? std::max(t.n_nodes, n / 16) : n / 4;
+    const long long guess = std::min<long long>(t.node_cap, nodes * 5 / 4 + 256);
     hipLaunchKernelGGL(k_node_records, dim3(grid_for(guess * kNodeLanes, 256)), dim3(256), 0, c->stream,
                        (const int *)t.sync_words, sh, (const unsigned long long *)t.key, (const int *)t.leaf_end,
                        (const int *)t.nbase, (const int *)t.start, t.end, t.skip, (const int *)t.level,

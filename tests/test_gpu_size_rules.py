@@ -58,12 +58,13 @@ def _keys(p, x):
     return key
 
 
-def _sort_ms(c):
-    """GPU time of the next tree build's sort (all its launches)."""
+def _sort_ms(c, group="tree_sort"):
+    """GPU time of the next tree build's sort (all its launches), or of another
+    group of its kernels."""
     c.enable_timing(0)
     c.enable_timing(1)
     c.build_tree()
-    avg, count = c.kernel_times()["tree_sort"]
+    avg, count = c.kernel_times()[group]
     return avg * count
 
 
@@ -130,3 +131,26 @@ def test_sort_order_of_a_crowded_cell(dim, n, m):
         before = c.tree_dump()["members"]
         np.testing.assert_array_equal(before, want)
     c.close()
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+def test_node_passes_after_a_build_with_few_nodes(dim):
+    """The node passes are sized before the node count is known: the build that
+    follows one with a chain of 20 nodes for 200000 coincident particles takes at
+    most four times the usual (its grids may be a quarter), not tens of times."""
+    n = 200000
+    p, f = _box(dim, n)
+    p["leaf_particle_num"] = 8
+    g = f.copy()
+    g[ics.F_POS:ics.F_POS + dim] = 0.3
+    first, usual = [], []
+    for _ in range(3):
+        c = sphgpu.Context(p, n)
+        c.upload(g)
+        c.build_tree()
+        assert c.stats()["nodes"] < 100
+        c.upload(f)
+        first.append(_sort_ms(c, "tree_node_records"))
+        usual += [_sort_ms(c, "tree_node_records") for _ in range(3)]
+        c.close()
+    assert min(first) < 4 * min(usual), (first, usual)
