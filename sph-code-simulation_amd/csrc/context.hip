@@ -369,6 +369,19 @@ struct RowRange {
     }
 };
 
+// One row gains nothing from the pinned halves but the shorter wait of a small
+// download (500 particles 23 -> 16 us) and the copies of a large one (400k 205 ->
+// 165 us); between them, and for uploads, HIP's own copy is the faster: upload
+// 21 us against 25 at 500, 29 / 32 at 16k, 145 / 170 at 400k; download 25 / 30 at
+// 5000, 36 / 42 at 40k, 84 / 79 at 133k.  Two large rows up are like one (133k 112 /
+// 120), two small ones not (5000 37 / 30).
+constexpr size_t kRowSmall = 32u << 10, kRowLarge = 512u << 10;
+bool copy_rows_directly(int count, size_t row_bytes, bool up)
+{
+    if (up) return count == 1 || (count == 2 && row_bytes >= kRowLarge);
+    return count == 1 && row_bytes > kRowSmall && row_bytes < kRowLarge;
+}
+
 // memory that HIP knows (pinned, managed or device) is copied as it is
 bool known_to_hip(const void *p)
 {
@@ -390,7 +403,7 @@ int exchange_rows(sphgpu_ctx *c, double *fields, uint64_t mask, bool up)
         if (mask & SPHGPU_MASK(f)) rows.row[count++] = fields + (size_t)f * c->n;
     if (count == 0) return 0;
     const size_t total = rows.row_bytes * count;
-    if (!c->bounce || known_to_hip(fields)) {
+    if (!c->bounce || copy_rows_directly(count, rows.row_bytes, up) || known_to_hip(fields)) {
         for (int r = 0; r < count; ++r) {
             double *const dev = c->stage + (size_t)r * c->n;
             HIPCHK(c, up ? hipMemcpyAsync(dev, rows.row[r], rows.row_bytes, hipMemcpyHostToDevice, c->stream)
@@ -399,7 +412,10 @@ int exchange_rows(sphgpu_ctx *c, double *fields, uint64_t mask, bool up)
         return 0;
     }
     const size_t half = c->bounce_bytes / 2;
-    const size_t chunk = std::min(half, std::max<size_t>(1u << 20, (total / 8 + 4095) & ~(size_t)4095));
+    // 16 rounds, of 2 MB at least: the first one's copy and the last one's DMA are
+    // not hidden (8 rounds of 1 MB at least: four rows of 133k up 195 us, now 180;
+    // 14 of 400k 1565, now 1530), and a round costs some 10 us itself
+    const size_t chunk = std::min(half, std::max<size_t>(2u << 20, (total / 16 + 4095) & ~(size_t)4095));
     const int rounds = (int)((total + chunk - 1) / chunk);
     char *const dev = reinterpret_cast<char *>(c->stage);
     auto dma = [&](int r) {

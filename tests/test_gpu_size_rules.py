@@ -154,3 +154,25 @@ def test_node_passes_after_a_build_with_few_nodes(dim):
         usual += [_sort_ms(c, "tree_node_records") for _ in range(3)]
         c.close()
     assert min(first) < 4 * min(usual), (first, usual)
+
+
+@pytest.mark.parametrize("n", [1, 4096, 4097, 65535, 65536, 262144, 262145])
+def test_exchange_of_one_and_two_rows(n):
+    """Uploads and downloads of one and of two rows, which are copied directly or
+    through the pinned halves by their size: the masked rows exactly, the others
+    untouched, with both kinds in turn."""
+    c = sphgpu.Context(ics.default_params(3), n)
+    rng = np.random.default_rng(n)
+    f = np.full((sphgpu.NFIELDS, n), -7.0)
+    want = np.zeros_like(f)
+    for rows in ([ics.F_MASS], [ics.F_POS, ics.F_ENE], [ics.F_POS, ics.F_POS + 1, ics.F_POS + 2], [ics.F_VEL], [ics.F_DENS, ics.F_SML]):
+        for r in rows:
+            want[r] = f[r] = rng.random(n)
+        c.upload(f, sum(1 << r for r in rows))
+        f[rows] = -7.0  # the upload is complete when it returns
+        for part in ([ics.F_MASS], [ics.F_POS, ics.F_ENE], rows):
+            out = np.full_like(f, -9.0)
+            c._check(c.lib.sphgpu_download(c.h, sphgpu._dp(out), sum(1 << r for r in part)), "download")
+            np.testing.assert_array_equal(out[part], want[part])
+            assert (np.delete(out, part, axis=0) == -9.0).all()
+    c.close()
