@@ -101,8 +101,7 @@ struct Tree {
     // gravity walk records (one per node, refreshed by each gravity call)
     GravNode *gnode = nullptr;
     int gnode_cap = 0;
-    double *gpart = nullptr;         // sums of a walk in gpart_seg pieces, [gpart_seg][4][n]
-    int gpart_seg = 0;
+    double *gpart = nullptr;  // sums of a walk in many pieces, [pieces][4][n] (fewer use sphgpu_ctx::stage)
     // root geometry (device): center[3], edge
     double *root = nullptr;
     int node_cap = 0;
@@ -185,7 +184,7 @@ struct sphgpu_ctx {
     // SPH steps never change them): the density sums then skip the mass loads
     bool mass_uniform = false;
     double mass_u = 0.0;
-    double *stage = nullptr;     // host-exchange staging, [NFIELDS][n]
+    double *stage = nullptr;     // host-exchange staging, [NFIELDS][n]; idle between exchanges
     char *bounce = nullptr;      // pinned memory of the host exchange, two halves
     size_t bounce_bytes = 0;
     hipEvent_t bounce_moved[2] = {};  // a half's copy has ended

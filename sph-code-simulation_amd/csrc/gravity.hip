@@ -493,7 +493,7 @@ int grav_sides(int n)
     return std::max(1, std::min(kGravWaves / waves / 2, kGravSideMax));
 }
 
-template <typename T> void launch_gravity(sphgpu_ctx *c, int nside)
+template <typename T> void launch_gravity(sphgpu_ctx *c, int nside, double *part)
 {
     GravArgs<T> a;
     a.n = c->n;
@@ -509,7 +509,7 @@ template <typename T> void launch_gravity(sphgpu_ctx *c, int nside)
     for (int k = 0; k <= nside; ++k) a.bound[k] = (int)((long long)a.n_nodes * k * k / ((long long)nside * nside));
     a.ngroups = grid_for(c->n, 256);
     a.nbase = c->tree.nbase;
-    a.part = c->tree.gpart;
+    a.part = part;
     const dim3 g((a.ngroups + kNumXcd - 1) / kNumXcd * kNumXcd * 2 * nside), b(256);
 #define LAUNCH(D)                                                                          \
     if (c->box.periodic) hipLaunchKernelGGL((k_gravity<D, T, true>), g, b, 0, c->stream, a); \
@@ -542,20 +542,27 @@ int gravity(sphgpu_ctx *c)
     hipLaunchKernelGGL(k_grav_nodes, dim3(grid_for(t.n_nodes, 256)), dim3(256), 0, c->stream, t.n_nodes, t.node_cap,
                        t.com, t.edge, t.mass, t.start, t.end, t.skip, t.level, (float)c->prm.gravity_constant, t.gnode);
     time_end(c);
-    const int nside = grav_sides(c->n), nseg = 2 * nside;
-    if (nseg > t.gpart_seg) {
-        if (t.gpart) hipFree(t.gpart);
-        t.gpart = nullptr;
-        t.gpart_seg = 0;
-        if (hipMalloc((void **)&t.gpart, sizeof(double) * 4 * (size_t)nseg * c->n) != hipSuccess)
-            return fail(c, SPHGPU_E_NOMEM, "gravity piece sums");
-        t.gpart_seg = nseg;
+    // the pieces' sums: in the exchange's staging block, which is idle here and
+    // has room for kStageSides pieces a side (the sets that take that few are the
+    // large ones), else in memory of their own; without that, fewer pieces
+    constexpr int kStageSides = SPHGPU_NFIELDS / 8;
+    int nside = grav_sides(c->n);
+    double *part = c->stage;
+    if (nside > kStageSides) {
+        if (!t.gpart && hipMalloc((void **)&t.gpart, sizeof(double) * 8 * (size_t)nside * c->n) != hipSuccess) {
+            (void)hipGetLastError();
+            t.gpart = nullptr;
+            nside = kStageSides;
+        } else {
+            part = t.gpart;
+        }
     }
+    const int nseg = 2 * nside;
     time_begin(c, "gravity");
-    if (c->prm.pair_precision == SPHGPU_PAIR_FP64) launch_gravity<double>(c, nside);
-    else launch_gravity<float>(c, nside);
+    if (c->prm.pair_precision == SPHGPU_PAIR_FP64) launch_gravity<double>(c, nside, part);
+    else launch_gravity<float>(c, nside, part);
     hipLaunchKernelGGL(k_gravity_sum, dim3(grid_for(c->n, 256), c->dim + 1), dim3(256), 0, c->stream, c->n, nseg,
-                       (const double *)t.gpart, c->sc[S_PHI], c->acc[0], c->acc[1], c->acc[2]);
+                       (const double *)part, c->sc[S_PHI], c->acc[0], c->acc[1], c->acc[2]);
     time_end(c);
     HIPCHK(c, hipGetLastError());
     return 0;

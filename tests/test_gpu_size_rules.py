@@ -176,3 +176,85 @@ def test_exchange_of_one_and_two_rows(n):
             np.testing.assert_array_equal(out[part], want[part])
             assert (np.delete(out, part, axis=0) == -9.0).all()
     c.close()
+
+
+@pytest.mark.parametrize("prec,tol", [(ics.PAIR_FP64, 1e-12), (ics.PAIR_FP32, 2e-6)])
+@pytest.mark.parametrize("n", [32768, 32769, 70001, 205003, 349504, 349505, 1048576, 1048577])
+def test_gravity_walk_pieces_by_size(n, prec, tol):
+    """The walk is cut into 64, 63, 29, 10, 6, 5, 2 and 1 pieces a side at these
+    sizes (six and more keep their sums in memory of their own, five and fewer in
+    the exchange's block): the field of a sample of particles (the first and last
+    in key order among them) against the walk of each by itself over the whole
+    tree.  Tolerances on the summed magnitudes: FP32 20 u (positions rounded to
+    FP32, compensated sums), FP64 far below."""
+    from test_gpu_small_paths import _hk_pair
+    theta, G = 0.7, 0.7
+    rng = np.random.default_rng(n)
+    p = ics.default_params(3)
+    p.update(use_gravity=1, theta=theta, leaf_particle_num=32, pair_precision=prec, gravity_constant=G)
+    f = ics.empty_fields(n)
+    x = rng.normal(0, 1, (3, n))
+    f[ics.F_POS:ics.F_POS + 3] = x
+    m = f[ics.F_MASS] = rng.uniform(0.5, 1.5, n) / n
+    f[ics.F_DENS] = f[ics.F_ENE] = 1.0
+    h = f[ics.F_SML] = rng.uniform(0.5, 1.5, n) * n ** (-1 / 3)
+    rows = [ics.F_PHI, ics.F_ACC, ics.F_ACC + 1, ics.F_ACC + 2]
+    c = sphgpu.Context(p, n)
+    c.upload(f)
+    c.build_tree()
+    d = c.tree_dump()
+    c.gravity()
+    out = c.download(sum(1 << r for r in rows))[rows]
+    # a second evaluation adds to the accelerations again
+    c.gravity()
+    again = c.download(sum(1 << r for r in rows))[rows]
+    c.close()
+    np.testing.assert_array_equal(again[0], out[0])
+    np.testing.assert_allclose(again[1:], 2 * out[1:], rtol=1e-15)
+    level, first, count = d["level"], d["first"], d["count"]
+    by_level = [np.flatnonzero(level == k) for k in range(1, level.max() + 1)]
+    parent = np.zeros(len(level), dtype=int)
+    for above, below in zip(by_level, by_level[1:]):
+        parent[below] = above[np.searchsorted(above, below) - 1]  # pre-order
+    com, e2 = d["com"].T, d["edge"] ** 2
+    leaf, members = d["is_leaf"] == 1, d["members"]
+    picked = np.concatenate([members[[0, 63, 64, n // 2, n - 65, n - 1]], rng.integers(0, n, 20)])
+    worst = 0.0
+    for i in picked:
+        v = x[:, [i]] - com
+        r2 = (v * v).sum(axis=0)
+        opened = (e2 > theta * theta * r2) | (r2 < e2)
+        seen = np.ones(len(level), dtype=bool)
+        for below in by_level[1:]:
+            seen[below] = seen[parent[below]] & opened[parent[below]]
+        far = seen & ~opened
+        w = G * d["mass"][far]
+        phi, s_phi = -(w / np.sqrt(r2[far])).sum(), (w / np.sqrt(r2[far])).sum()
+        acc, s_acc = -(w / r2[far] ** 1.5 * v[:, far]).sum(axis=1), (w / r2[far]).sum()
+        near = seen & opened & leaf
+        j = np.concatenate([members[a:a + k] for a, k in zip(first[near], count[near])])
+        j = j[j != i]
+        dx = x[:, [i]] - x[:, j]
+        r = np.sqrt((dx * dx).sum(axis=0))
+        (fi, gi), (fj, gj) = _hk_pair(r, h[i]), _hk_pair(r, h[j])
+        t = 0.5 * G * m[j] * (fi + fj)
+        phi, acc = phi - t.sum(), acc - (dx * (0.5 * G * m[j] * (gi + gj))).sum(axis=1)
+        s_phi, s_acc = s_phi + t.sum(), s_acc + (G * m[j] / (r * r)).sum()
+        worst = max(worst, abs(out[0, i] - phi) / s_phi, np.abs(out[1:, i] - acc).max() / s_acc)
+    assert worst < tol
+
+
+def test_gravity_memory_of_large_sets():
+    """The pieces of the walk of 1M particles need no device memory beyond the
+    context's own (the node records are 64 B for each of some 100000 nodes)."""
+    torch = pytest.importorskip("torch")
+    p, f = _box(3, 1000000)
+    p["use_gravity"] = 1
+    c = sphgpu.Context(p, f.shape[1])
+    c.upload(f)
+    c.build_tree()
+    free = torch.cuda.mem_get_info()[0]
+    c.gravity()
+    taken = free - torch.cuda.mem_get_info()[0]
+    c.close()
+    assert taken < 32 << 20, taken
