@@ -258,3 +258,132 @@ def test_gravity_memory_of_large_sets():
     taken = free - torch.cuda.mem_get_info()[0]
     c.close()
     assert taken < 32 << 20, taken
+
+
+@pytest.mark.parametrize("prec,tol", [(ics.PAIR_FP64, 1e-12), (ics.PAIR_FP32, 2e-6)])
+@pytest.mark.parametrize("dim,side,leaf,theta", [(3, 16, 8, 0.21), (3, 16, 32, 0.2), (3, 12, 1, 0.1), (2, 64, 8, 0.05), (1, 512, 8, 0.01)])
+def test_periodic_walk_half_box_ties(dim, side, leaf, theta, prec, tol):
+    """Periodic gravity where many pairs lie exactly half a box apart (a lattice of
+    a binary spacing, three in ten particles off it) and such leaves are opened by
+    some of a wavefront's particles only, so that other lanes evaluate their pairs:
+    the image at a tie, and with it the sign, is the one of the FP64 positions of
+    the particle itself.  Against the walk of each particle of a sample by itself;
+    tolerances as for the open walk, and in FP32 the rounding of the positions,
+    which moves a pair's distance by up to 2^-24 and its 1/r and 1/r^2 terms by
+    that over r, and three times that (close pairs in 1D)."""
+    from test_gpu_small_paths import _hk_pair
+    n = side ** dim
+    rng = np.random.default_rng([n, leaf])
+    x = np.stack(np.meshgrid(*[np.arange(side) / side] * dim, indexing="ij")).reshape(dim, n) + 0.5 / side
+    off = rng.random(n) < 0.3
+    x[:, off] = rng.random((dim, off.sum()))
+    p, f = _box(dim, n)
+    G = 0.7
+    p.update(use_gravity=1, theta=theta, leaf_particle_num=leaf, pair_precision=prec, gravity_constant=G)
+    f[ics.F_POS:ics.F_POS + dim] = x
+    m = f[ics.F_MASS] = rng.uniform(0.5, 1.5, n) / n
+    h = f[ics.F_SML] = rng.uniform(0.5, 1.5, n) / side
+    c = sphgpu.Context(p, n)
+    c.upload(f)
+    c.build_tree()
+    d = c.tree_dump()
+    c.gravity()
+    out = c.download()
+    c.close()
+
+    def image(v):  # the smaller of d and d -+ L, d itself at a tie
+        return np.where(np.abs(v) <= np.abs(np.abs(v) - 1.0), v, v - np.sign(v))
+
+    level, first, count, members = d["level"], d["first"], d["count"], d["members"]
+    by_level = [np.flatnonzero(level == k) for k in range(1, level.max() + 1)]
+    parent = np.zeros(len(level), dtype=int)
+    for above, below in zip(by_level, by_level[1:]):
+        parent[below] = above[np.searchsorted(above, below) - 1]
+    com, e2, is_leaf = d["com"].T[:dim], d["edge"] ** 2, d["is_leaf"] == 1
+    worst, ties = 0.0, 0
+    for i in rng.permutation(n)[:150]:
+        v = image(x[:, [i]] - com)
+        r2 = (v * v).sum(axis=0)
+        opened = (e2 > theta * theta * r2) | (r2 < e2)
+        seen = np.ones(len(level), dtype=bool)
+        for below in by_level[1:]:
+            seen[below] = seen[parent[below]] & opened[parent[below]]
+        far = seen & ~opened
+        w = G * d["mass"][far]
+        near = seen & opened & is_leaf
+        j = np.concatenate([members[a:a + k] for a, k in zip(first[near], count[near])])
+        j = j[j != i]
+        dx = image(x[:, [i]] - x[:, j])
+        ties += int((np.abs(dx) == 0.5).any(axis=0).sum())
+        r = np.sqrt((dx * dx).sum(axis=0))
+        (fi, gi), (fj, gj) = _hk_pair(r, h[i]), _hk_pair(r, h[j])
+        t = 0.5 * G * m[j] * (fi + fj)
+        phi = -(w / np.sqrt(r2[far])).sum() - t.sum()
+        acc = -(w / r2[far] ** 1.5 * v[:, far]).sum(axis=1) - (dx * (0.5 * G * m[j] * (gi + gj))).sum(axis=1)
+        s_acc = (w / r2[far]).sum() + (G * m[j] / (r * r)).sum()
+        moved = 2.0 ** -24 if prec == ics.PAIR_FP32 else 0.0
+        e_phi, e_acc = (moved * G * m[j] / r ** 2).sum(), (3 * moved * G * m[j] / r ** 3).sum()
+        worst = max(worst, (abs(out[ics.F_PHI, i] - phi) - e_phi) / abs(phi),
+                    (np.abs(out[ics.F_ACC:ics.F_ACC + dim, i] - acc).max() - e_acc) / s_acc)
+    assert ties > 50
+    assert worst < tol
+
+
+@pytest.mark.parametrize("prec", [ics.PAIR_FP32, ics.PAIR_FP64])
+@pytest.mark.parametrize("shell,lo,hi", [(12, 1, 16), (40, 17, 64), (110, 65, 128), (180, 129, 192), (240, 193, 256),
+                                         (330, 257, 1000)])
+def test_force_list_order_by_run_length(shell, lo, hi, prec):
+    """Force lists end with the particles j that reach i from outside its own
+    radius (h_j > r >= h_i), in ascending order of the sorted particles whatever
+    order they were appended in: by the lane's own registers (16), by 64, 128, 192
+    and 256 lanes' entries of the wavefront, and beyond.  Clumps of light
+    particles, each inside a shell of heavy ones whose spheres all reach it: the
+    longest run is the shell, which the test asserts."""
+    rng = np.random.default_rng(shell)
+    systems, clump = 12, 64
+    k = np.arange(shell) + 0.5  # points spread over the unit sphere
+    polar, turn = np.arccos(1 - 2 * k / shell), np.pi * (1 + 5 ** 0.5) * k
+    ball = np.stack([np.sin(polar) * np.cos(turn), np.sin(polar) * np.sin(turn), np.cos(polar)])
+    grid = 0.01 * (np.stack(np.meshgrid(*[np.arange(4) - 1.5] * 3, indexing="ij")).reshape(3, clump))
+    one = np.concatenate([ball, grid], axis=1)
+    one += 1e-3 * rng.uniform(-1, 1, one.shape)
+    at = 10.0 * np.stack(np.unravel_index(np.arange(systems), (3, 2, 2)))
+    x = (at[:, :, None] + one[:, None, :]).reshape(3, -1)
+    heavy = np.tile(np.arange(shell + clump) < shell, systems)
+    # sum of W h^3 over the shell's particles within h = 1.1 (a cap of the sphere)
+    nn = int(4 * np.pi / 3 * (8 / np.pi + 0.1114 * shell * 1.1 ** 2))
+    n = x.shape[1]
+    p = ics.default_params(3)
+    p.update(neighbor_number=nn, leaf_particle_num=8, pair_precision=prec)
+    f = ics.empty_fields(n)
+    f[ics.F_POS:ics.F_POS + 3] = x
+    f[ics.F_MASS] = np.where(heavy, 1.0, 1e-6)
+    guess = np.where(heavy, 1.1, 0.04)
+    f[ics.F_DENS] = nn * f[ics.F_MASS] * 3 / (4 * np.pi * guess ** 3)
+    f[ics.F_ENE] = f[ics.F_SOUND] = 1.0
+    c = sphgpu.Context(p, n)
+    c.upload(f)
+    c.build_tree()
+    for _ in range(6):
+        c.pre_interaction()
+    count, lists = c.neighbor_sets(None, 2, cap=2048)
+    place = np.empty(n, dtype=int)
+    place[c.tree_dump()["members"]] = np.arange(n)
+    h = c.download(1 << ics.F_SML)[ics.F_SML]
+    c.close()
+    longest = 0
+    for i in range(n):
+        j = lists[i, :count[i]]
+        d = x[:, [i]] - x[:, j]
+        r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2]
+        own = np.sqrt(r2) < h[i]
+        run = place[j[~own]]
+        assert not own[np.argmin(own):].any() if run.size else own.all()  # appended entries come last
+        assert (np.diff(run) > 0).all()
+        longest = max(longest, run.size)
+        if i % 7 == 0:
+            d = x[:, [i]] - x
+            r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2]
+            want = (np.sqrt(r2) < np.maximum(h[i], h)) & (r2 != 0)
+            np.testing.assert_array_equal(np.sort(j), np.flatnonzero(want))
+    assert lo <= longest <= hi, longest
