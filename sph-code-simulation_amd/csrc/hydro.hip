@@ -1895,16 +1895,34 @@ __global__ __launch_bounds__(256) void k_riemann_batch_learned(int n, const doub
 
 // ---------------------------------------------------------------------------------
 // Particles up to which a pair loop runs with a quad per particle.  The quad
-// form has a quarter of the serial chain and four times the wavefronts (one
-// lane per particle fills the chip from about 200k particles on), but repeats
-// the additions in four lanes.  Measured (us, one lane / quad):
-//   PreInteraction FP32: 4k FP64 83 / 29, 65k 2D 142 / 79, 104k 234 / 153,
-//     133k 173 / 185, 185k 148 / 179, 1M 684 / 811
-//   PreInteraction FP64: 16k 289 / 96, 262k 489 / 394, 1M 1419 / 1476
-//   GSPH force FP32: 104k 399 / 177, 133k 195 / 159, 185k 214 / 205, 262k 257 /
-//     272, 512k 479 / 525, 1M 1029 / 998
+// form has a quarter of the serial chain and four times the wavefronts, but
+// repeats the additions in four lanes.  One lane per particle takes whole rounds
+// of resident wavefronts (two a SIMD hold 131072 particles), so it loses most
+// where neighbours differ much in their iterations (a blast) or where a round is
+// just begun, and comes closest on quiet sets that fill one.  Measured on either
+// side of the lines (us, one lane / quad; lattice boxes and shear layers unless
+// said):
+//   PreInteraction FP32 3D: DISPH 97k 98 / 83, 125k 100 / 101, 195k 122 / 144;
+//     SSPH 97k 98 / 82, 125k 100 / 98, 195k 123 / 139; GSPH 97k 98 / 87, 125k
+//     100 / 105, 195k 178 / 156, 262k 193 / 203, Sedov 125k 220 / 146, 1M 684 / 811
+//   1D and 2D: DISPH 160k 184 / 150, 260k 284 / 219, 360k 332 / 302; SSPH 260k
+//     216 / 163, 360k 255 / 222; 1D 300k 106 / 101
+//   FP64: 3D DISPH 262k 380 / 356, 512k 724 / 706; GSPH 262k 377 / 394, 512k
+//     732 / 789, Sedov 262k 595 / 411, 389k 1045 / 763, 512k 894 / 740; 2D DISPH
+//     490k 754 / 667
+//   GDISPH (gradients beside the pressure sums) FP32 3D 80k 100 / 95, 91k 102 /
+//     108, 125k 104 / 139; FP64 3D 80k 202 / 182, 91k 207 / 209, 262k 400 / 540;
+//     2D 260k 280 / 268, 360k 336 / 375; FP64 2D 260k 536 / 480; 1D 260k 116 / 115
+//   GSPH force FP32: Sedov 125k 281 / 170, 195k 357 / 245, 262k 371 / 286, 1M
+//     1029 / 998; box 125k 119 / 129, 149k 176 / 156, 195k 181 / 187, 262k 218 / 242
 //   GSPH force FP64: 4k 67 / 23, 262k 785 / 599, 1M 2317 / 2209: always a quad
-constexpr int kQuadPre32 = 131072, kQuadPre64 = 524288, kQuadGsph32 = 196608;
+template <int D, int TYPE, typename T> constexpr int quad_pre_limit()
+{
+    if (TYPE == SPHGPU_GDISPH) return D == 3 ? 86016 : 262144;
+    if (sizeof(T) == 8) return 524288;
+    return D == 3 ? 131072 : 262144;
+}
+constexpr int kQuadGsph32 = 196608;
 
 template <int D, int K, int TYPE, typename T> void launch_pre(sphgpu_ctx *c)
 {
@@ -1953,7 +1971,7 @@ template <int D, int K, int TYPE, typename T> void launch_pre(sphgpu_ctx *c)
     a.tight = c->pre_rscale < 1.0 && c->prm.iterative_sml;
     a.pre_flag = c->dflag;
     a.alpha_in = c->alpha_snap_on ? c->alpha_snap : nullptr;
-    if (c->n <= (sizeof(T) == 8 ? kQuadPre64 : kQuadPre32))
+    if (c->n <= quad_pre_limit<D, TYPE, T>())
         hipLaunchKernelGGL((k_pre<D, K, TYPE, T, 4>), dim3(grid_for(4ll * c->n, 256)), dim3(256), 0, c->stream, a);
     else
         hipLaunchKernelGGL((k_pre<D, K, TYPE, T, 1>), dim3(grid_for(c->n, 256)), dim3(256), 0, c->stream, a);

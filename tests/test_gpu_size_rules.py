@@ -387,3 +387,84 @@ def test_force_list_order_by_run_length(shell, lo, hi, prec):
             want = (np.sqrt(r2) < np.maximum(h[i], h)) & (r2 != 0)
             np.testing.assert_array_equal(np.sort(j), np.flatnonzero(want))
     assert lo <= longest <= hi, longest
+
+
+def test_gdisph_density_cost():
+    """PreInteraction of GDISPH (the pressure sums and the gradients) takes at most
+    1.3 times that of DISPH on the same particles (1.1 with one lane per particle,
+    1.5 with four at this size)."""
+    t = {}
+    for kind in (ics.DISPH, ics.GDISPH):
+        p, f = ics.sedov_3d(64, jitter=0.1)
+        f[ics.F_ENE] = 1.0
+        p.update(sph_type=kind, neighbor_number=50, leaf_particle_num=32, pair_precision=ics.PAIR_FP64, gsph_2nd_order=1)
+        c = sphgpu.Context(p, f.shape[1])
+        c.upload(f)
+        c.build_tree()
+        for _ in range(3):
+            c.pre_interaction()
+        c.enable_timing(1)
+        for _ in range(5):
+            c.pre_interaction()
+        t[kind] = c.kernel_times()["pre_interaction"][0]
+        c.close()
+    assert t[ics.GDISPH] < 1.3 * t[ics.DISPH], t
+
+
+def _strip_with_cluster(total, side):
+    """2D counterpart of _slab_with_cluster: `total` jittered lattice particles in
+    the lower half of the unit box, first in key order and the same for every
+    `side`, and side^2 at the upper corner, out of their reach."""
+    rng = np.random.default_rng(2)
+    nx = int(np.ceil((2.2 * total) ** 0.5))
+    g = np.stack(np.meshgrid(np.arange(nx), np.arange(nx // 2), indexing="xy")).reshape(2, -1) + 0.5
+    g = ((g + rng.uniform(-0.2, 0.2, g.shape)) / nx)[:, :total]
+    assert g.shape[1] == total and g[1].max() < 0.5
+    g[:, 0] = 0.0  # the lower corner of the root cell
+    c = np.stack(np.meshgrid(*[1.0 - 0.0005 * np.arange(side)] * 2, indexing="ij")).reshape(2, -1)
+    n = total + side ** 2
+    f = ics.empty_fields(n)
+    f[ics.F_POS:ics.F_POS + 2] = np.concatenate([g, c], axis=1)
+    f[ics.F_VEL:ics.F_VEL + 2, :total] = 0.3 * np.sin(7.0 * g)
+    f[ics.F_MASS] = 1.0 / nx ** 2
+    f[ics.F_DENS, :total] = 1.0
+    f[ics.F_DENS, total:] = 1.0 / (0.0005 * nx) ** 2
+    f[ics.F_ENE, :total] = 1.0 + 0.3 * np.sin(9.0 * g[0]) + 0.05 * rng.random(total)
+    f[ics.F_ENE, total:] = 1.0
+    f[ics.F_SOUND] = np.sqrt(10.0 / 9.0 * f[ics.F_ENE])
+    f[ics.F_ALPHA] = f[ics.F_BALSARA] = 1.0
+    return f
+
+
+@pytest.mark.parametrize("dim,limit,prec,over", [
+    (3, 86016, ics.PAIR_FP32, dict(sph_type=ics.GDISPH, gsph_2nd_order=1)),
+    (3, 86016, ics.PAIR_FP64, dict(sph_type=ics.GDISPH, gsph_2nd_order=1)),
+    (2, 262144, ics.PAIR_FP32, dict(sph_type=ics.GDISPH, gsph_2nd_order=1)),
+    (2, 262144, ics.PAIR_FP32, dict(sph_type=ics.DISPH, kernel=ics.WENDLAND)),
+    (2, 262144, ics.PAIR_FP32, dict(sph_type=ics.SSPH, use_time_dependent_av=1)),
+    (2, 262144, ics.PAIR_FP64, dict(sph_type=ics.GDISPH, gsph_2nd_order=1)),
+])
+def test_lane_forms_agree_at_their_limits(dim, limit, prec, over):
+    """PreInteraction with a quad of lanes per particle and with one lane, below and
+    above the limits by type and dimension: the particles that both sizes share
+    come out bit for bit equal."""
+    from test_gpu_small_paths import _slab_with_cluster
+    total, out = limit - 150, []
+    for side in ((5, 6) if dim == 3 else (10, 14)):  # 125 or 216, 100 or 196 more
+        f = _slab_with_cluster(total, side) if dim == 3 else _strip_with_cluster(total, side)
+        assert (f.shape[1] <= limit) == (len(out) == 0)
+        p = ics.default_params(dim)
+        p.update(neighbor_number=40 if dim == 3 else 24, leaf_particle_num=32, pair_precision=prec, gamma=5.0 / 3.0, **over)
+        c = sphgpu.Context(p, f.shape[1])
+        c.upload(f)
+        c.dt = 1e-4
+        c.build_tree()
+        for _ in range(5):
+            c.pre_interaction()
+        c.fluid_force()
+        out.append(c.download()[:, :total])
+        assert c.stats()["flist_searches"] == 0
+        c.close()
+    assert np.isfinite(out[0]).all() and np.abs(out[0][ics.F_ACC]).max() > 0
+    for row in range(out[0].shape[0]):
+        np.testing.assert_array_equal(out[0][row], out[1][row], err_msg=f"field row {row}")
