@@ -8,6 +8,11 @@
  * blocking on return (stream-ordered work is complete).  One host thread per
  * context; a context is not thread-safe.
  *
+ * Memory of a context beside the particle rows, lists and tree: up to 16 MB of
+ * pinned host memory for uploads and downloads (they copy the caller's rows
+ * directly where it cannot be had), and with gravity up to 135 MB of device
+ * memory below 349505 particles (fewer pieces of the walk without it).
+ *
  * The entry points replace, one for one, the calls the reference driver makes
  * on its Module objects (reference: include/module.hpp:10-14,
  * src/solver.cpp:941-978):
@@ -140,7 +145,10 @@ typedef struct sphgpu_stats {
     int64_t force_pairs;         /* accepted force pairs (directed)           */
     int64_t force_candidates;    /* force candidate-list entries              */
     int64_t riemann_iters;       /* sum of Newton iterations in the Riemann solver */
-    int64_t riemann_wave_max_iters; /* sum over wavefronts of max iterations  */
+    int64_t riemann_wave_max_iters; /* sum over the wavefronts' rounds of the
+                                    largest iteration count among the round's 64
+                                    pairs (one of 64 particles each, or four of
+                                    16, by the particle count and precision)  */
     int64_t riemann_calls;       /* Riemann problems solved                   */
     int64_t riemann_fallbacks;   /* learned guesses rejected for the plain one */
     int64_t riemann_learned;     /* pairs that used the learned guess         */

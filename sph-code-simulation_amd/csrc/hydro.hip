@@ -930,7 +930,9 @@ struct FlistArgs {
 // The lanes of a quad take every fourth entry, four of them at a time (the
 // appends are atomic and ordered later, so the split changes nothing).  Bound
 // by the gathers of the neighbours' records; one lane per particle took 231 us
-// at 1M (Sedov, now 190; Evrard 88, now 89), 105 at 104k (36), 26 at 65k in 2D (13).
+// at 1M (Sedov, now 190; Evrard 88, now 89), 105 at 104k (36), 26 at 65k in 2D
+// (13), and from a million particles in quiet sets on a little less (3M box 367,
+// now 411; 1M shear layer 139, now 155).
 template <int D, bool FP64>
 __global__ __launch_bounds__(256) void k_flist_scatter(FlistArgs a)
 {

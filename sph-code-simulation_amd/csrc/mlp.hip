@@ -85,7 +85,7 @@ __global__ void k_mlp_predict(int n, const float *__restrict__ rows, MLPDev m, f
 
 
 // ---- bf16 MFMA training --------------------------------------------------------
-// One workgroup (4 waves) takes a tile of 64 rows through forward and backward
+// One workgroup (16 wavefronts) takes a tile of 64 rows through forward and backward
 // with v_mfma_f32_16x16x32_bf16: operands bf16 in LDS, accumulation FP32.
 // Lane layout of the 16x16x32 tile (CDNA4): A[16][32] -- lane l holds row
 // l%16, k = 8*(l/16)..+7; B[32][16] -- lane l holds column l%16, the same k

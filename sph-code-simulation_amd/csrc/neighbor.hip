@@ -207,8 +207,10 @@ SPH_DEV void test_range_expand(const float4 *srec, int t0, int t1, const float m
 
 // LP lanes per particle (1, 2, 4 or 8): a wavefront owns 64 / LP consecutive
 // particles, and the lanes of a particle test a contiguous LP-th of each
-// candidate batch each; their kept candidates follow one another in the list,
-// so the lists do not depend on LP.
+// candidate batch each; their kept candidates follow one another in the list, so
+// the sets do not depend on LP, and neither does their order while no frontier of
+// the walk overflows (the leaves under an overflowing batch come in depth-first
+// order, and which batch that is depends on the wavefront's particles).
 template <int D, int IS_IJ, int LP>
 __global__ __launch_bounds__(256, 4) void k_search(SearchArgs a)
 {

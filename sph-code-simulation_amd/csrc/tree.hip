@@ -989,9 +989,9 @@ __device__ int group_end(const unsigned long long *__restrict__ key, int n, int 
     return lo + 1;
 }
 
-// A leaf of the deepest level holds any number of particles (coincident ones;
-// all of them where a run has blown up): eight lanes took 7.1 ms for the box of
-// a leaf of 1M, the whole workgroup takes 0.4.  The line lies well above the
+// A leaf of the deepest level holds any number of particles (coincident ones, or
+// those of a cell of a shallow tree): eight lanes took 7.1 ms for the box of a
+// leaf of 1M, the whole workgroup takes 0.4.  The line lies well above the
 // leaf sizes in use, where a workgroup per leaf would leave its lanes idle.
 constexpr int kWideLeaf = 512, kWideLeaves = 32;
 
