@@ -8,10 +8,12 @@
  * blocking on return (stream-ordered work is complete).  One host thread per
  * context; a context is not thread-safe.
  *
- * Memory of a context beside the particle rows, lists and tree: up to 16 MB of
- * pinned host memory for uploads and downloads (they copy the caller's rows
- * directly where it cannot be had), and with gravity up to 135 MB of device
- * memory below 349505 particles (fewer pieces of the walk without it).
+ * Memory beside the particle rows, lists and tree: 4 MB of pinned host memory
+ * for uploads and downloads, shared by the contexts of the process, set up when
+ * one of them exchanges several rows for the third time and freed with the last
+ * (the caller's rows are copied directly where it cannot be had, or while
+ * another thread's exchange has it); and with gravity up to 135 MB of device
+ * memory a context below 349505 particles (fewer pieces of the walk without it).
  *
  * The entry points replace, one for one, the calls the reference driver makes
  * on its Module objects (reference: include/module.hpp:10-14,

@@ -5,6 +5,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 
 #include "ctx.hpp"
@@ -161,6 +162,73 @@ static FieldPtrs field_ptrs(sphgpu_ctx *c)
 }
 
 // --------------------------------------------------------------------------
+// --------------------------------------------------------------------------
+// Pinned memory of the host exchange, two halves, shared by the contexts of the
+// process: one exchange has it at a time and another one that comes meanwhile
+// copies its rows directly.  It is set up when a context exchanges rows for the
+// third time and freed with the last context: pinned pages cost 0.4 us per KB
+// when they are first written and 0.3 ms to have (memory of each context's own
+// made the first upload of 65k particles 1.0 ms instead of 0.25 and the creation
+// of a context up to twice as long), which a program that uploads, runs and
+// downloads once does not get back.  2 MB a half: with 0.25 MB 14 rows of 133k
+// take 750 us instead of 440, with 8 MB no less.
+constexpr size_t kBounceHalf = 2u << 20;
+constexpr int kBounceAfter = 2;  // exchanges of a context without it
+
+namespace {
+struct Bounce {
+    std::mutex lock;
+    char *mem = nullptr;
+    int users = 0;
+} g_bounce;
+
+void bounce_enter()
+{
+    std::lock_guard<std::mutex> l(g_bounce.lock);
+    ++g_bounce.users;
+}
+
+void bounce_leave()
+{
+    std::lock_guard<std::mutex> l(g_bounce.lock);
+    if (--g_bounce.users > 0 || !g_bounce.mem) return;
+    hipHostFree(g_bounce.mem);
+    g_bounce.mem = nullptr;
+}
+
+// the halves for one exchange of a context, given back when its stream is idle
+class BounceHold {
+    std::unique_lock<std::mutex> l;
+    hipStream_t stream = nullptr;
+
+public:
+    bool take(sphgpu_ctx *c)
+    {
+        l = std::unique_lock<std::mutex>(g_bounce.lock, std::try_to_lock);
+        if (!l.owns_lock()) return false;
+        stream = c->stream;
+        if (!g_bounce.mem && c->exchanges++ >= kBounceAfter &&
+            hipHostMalloc((void **)&g_bounce.mem, 2 * kBounceHalf, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            g_bounce.mem = nullptr;
+            c->exchanges = 0;
+        }
+        if (!g_bounce.mem) l.unlock();
+        return l.owns_lock();
+    }
+    char *mem() const { return g_bounce.mem; }
+    // after the stream was waited for (a call that fails before leaves that here)
+    void give_back()
+    {
+        if (l.owns_lock()) l.unlock();
+    }
+    ~BounceHold()
+    {
+        if (l.owns_lock()) hipStreamSynchronize(stream);
+    }
+};
+} // namespace
+
 extern "C" {
 
 void sphgpu_params_default(sphgpu_params *p, int dim)
@@ -228,6 +296,7 @@ int sphgpu_create(const sphgpu_params *p, int n, sphgpu_ctx **out)
     std::string why;
     if (!check_params(p, why)) { *out = nullptr; return SPHGPU_E_ARG; }
     sphgpu_ctx *c = new sphgpu_ctx;
+    bounce_enter();
     c->prm = *p;
     c->n = n;
     c->dim = p->dim;
@@ -258,12 +327,6 @@ int sphgpu_create(const sphgpu_params *p, int n, sphgpu_ctx **out)
     if (p->pair_precision == SPHGPU_PAIR_FP64)
         for (int r = 0; r < R_NREC && ok; ++r) ok = alloc((void **)&c->rec64[r], sizeof(double4) * (size_t)n);
     ok = ok && alloc((void **)&c->hs, dn) && hipMalloc((void **)&c->stage, dn * SPHGPU_NFIELDS) == hipSuccess;
-    // without pinned memory the exchange copies the user's rows directly
-    c->bounce_bytes = std::min<size_t>(kBounceBytes, 2 * (dn * SPHGPU_NFIELDS + 4096));
-    if (ok && (hipHostMalloc((void **)&c->bounce, c->bounce_bytes, hipHostMallocDefault) != hipSuccess)) {
-        (void)hipGetLastError();
-        c->bounce = nullptr;
-    }
     for (auto &e : c->bounce_moved) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
     if (p->use_time_dependent_av) ok = ok && alloc((void **)&c->alpha_snap, dn);
     c->red_blocks = 1024;
@@ -313,7 +376,7 @@ int sphgpu_destroy(sphgpu_ctx *c)
     }
     hipFree(c->hs); hipFree(c->alpha_snap); hipFree(c->stage); hipFree(c->red);
     hipFree(c->dscal); hipFree(c->dmin); hipFree(c->dstats); hipFree(c->dflag);
-    if (c->bounce) hipHostFree(c->bounce);
+    bounce_leave();
     for (auto e : c->bounce_moved)
         if (e) hipEventDestroy(e);
     if (c->hscal) hipHostFree(c->hscal);
@@ -344,13 +407,12 @@ int sphgpu_get_params(const sphgpu_ctx *c, sphgpu_params *p, int32_t *n)
 
 // Masked rows between the user's memory and the front of the staging block.
 // A copy of pageable memory costs a pinning or a staging of its own per row, one
-// after the other: the rows go through two halves of the context's pinned memory
-// instead, the DMA of one running while the other is copied.  Download of 14
-// rows of 1M particles 10.5 -> 8.4 ms (the copy into fresh pages sets the
-// time), 7 rows of 133k 885 -> 516 us, of 16k 177 -> 108; upload of 13 rows 3.8
-// -> 3.4 ms, 535 -> 444 us and 174 -> 99.  Copying with three helper threads
-// took 4.1 ms for the first and 10 ms more for the second where the process
-// shares its cores: one thread does it.
+// after the other: the rows go through two halves of pinned memory instead, the
+// DMA of one running while the other is copied.  Download of 14 rows of 1M
+// particles 6.1 -> 3.9 ms, 7 rows of 133k 510 -> 310 us, of 16k 134 -> 68; upload
+// of 14 rows of 133k 560 -> 445 us, of 16k 178 -> 95 (1M the same, 3.8 ms).
+// Copying with three helper threads took half of that at 1M and 10 ms more at
+// 133k where the process shares its cores: one thread does it.
 namespace {
 struct RowRange {
     double *row[SPHGPU_NFIELDS];
@@ -371,14 +433,14 @@ struct RowRange {
 
 // One row gains nothing from the pinned halves but the shorter wait of a small
 // download (500 particles 23 -> 16 us) and the copies of a large one (400k 205 ->
-// 165 us); between them, and for uploads, HIP's own copy is the faster: upload
-// 21 us against 25 at 500, 29 / 32 at 16k, 145 / 170 at 400k; download 25 / 30 at
-// 5000, 36 / 42 at 40k, 84 / 79 at 133k.  Two large rows up are like one (133k 112 /
-// 120), two small ones not (5000 37 / 30).
-constexpr size_t kRowSmall = 32u << 10, kRowLarge = 512u << 10;
+// 170 us); between them, and for uploads, HIP's own copy is the faster: upload
+// 21 us against 25 at 500, 29 / 32 at 16k, 150 / 167 at 400k; download 25 / 30 at
+// 5000, 36 / 42 at 40k, 84 / 80 at 133k.  Two large rows up are like one (133k 112 /
+// 119, 400k 240 / 275) and so are two of 16 KB (25 / 31), others not (5000 37 / 30).
+constexpr size_t kRowTiny = 16u << 10, kRowSmall = 32u << 10, kRowLarge = 512u << 10;
 bool copy_rows_directly(int count, size_t row_bytes, bool up)
 {
-    if (up) return count == 1 || (count == 2 && row_bytes >= kRowLarge);
+    if (up) return count == 1 || (count == 2 && (row_bytes <= kRowTiny || row_bytes >= kRowLarge));
     return count == 1 && row_bytes > kRowSmall && row_bytes < kRowLarge;
 }
 
@@ -394,7 +456,9 @@ bool known_to_hip(const void *p)
     return a.type != hipMemoryTypeUnregistered;
 }
 
-int exchange_rows(sphgpu_ctx *c, double *fields, uint64_t mask, bool up)
+// `hold` has the pinned halves when they are in use; the caller keeps it until
+// its stream is idle
+int exchange_rows(sphgpu_ctx *c, double *fields, uint64_t mask, bool up, BounceHold &hold)
 {
     RowRange rows;
     rows.row_bytes = sizeof(double) * (size_t)c->n;
@@ -403,7 +467,7 @@ int exchange_rows(sphgpu_ctx *c, double *fields, uint64_t mask, bool up)
         if (mask & SPHGPU_MASK(f)) rows.row[count++] = fields + (size_t)f * c->n;
     if (count == 0) return 0;
     const size_t total = rows.row_bytes * count;
-    if (!c->bounce || copy_rows_directly(count, rows.row_bytes, up) || known_to_hip(fields)) {
+    if (copy_rows_directly(count, rows.row_bytes, up) || known_to_hip(fields) || !hold.take(c)) {
         for (int r = 0; r < count; ++r) {
             double *const dev = c->stage + (size_t)r * c->n;
             HIPCHK(c, up ? hipMemcpyAsync(dev, rows.row[r], rows.row_bytes, hipMemcpyHostToDevice, c->stream)
@@ -411,16 +475,12 @@ int exchange_rows(sphgpu_ctx *c, double *fields, uint64_t mask, bool up)
         }
         return 0;
     }
-    const size_t half = c->bounce_bytes / 2;
-    // 16 rounds, of 2 MB at least: the first one's copy and the last one's DMA are
-    // not hidden (8 rounds of 1 MB at least: four rows of 133k up 195 us, now 180;
-    // 14 of 400k 1565, now 1530), and a round costs some 10 us itself
-    const size_t chunk = std::min(half, std::max<size_t>(2u << 20, (total / 16 + 4095) & ~(size_t)4095));
+    constexpr size_t chunk = kBounceHalf;
     const int rounds = (int)((total + chunk - 1) / chunk);
     char *const dev = reinterpret_cast<char *>(c->stage);
     auto dma = [&](int r) {
         const size_t a = (size_t)r * chunk, len = std::min(chunk, total - a);
-        char *const host = c->bounce + (r & 1) * half;
+        char *const host = hold.mem() + (r & 1) * chunk;
         const hipError_t e = up ? hipMemcpyAsync(dev + a, host, len, hipMemcpyHostToDevice, c->stream)
                                 : hipMemcpyAsync(host, dev + a, len, hipMemcpyDeviceToHost, c->stream);
         return e == hipSuccess ? hipEventRecord(c->bounce_moved[r & 1], c->stream) : e;
@@ -428,7 +488,7 @@ int exchange_rows(sphgpu_ctx *c, double *fields, uint64_t mask, bool up)
     if (!up) HIPCHK(c, dma(0));
     auto copy = [&](int r) {
         const size_t a = (size_t)r * chunk;
-        rows.copy(c->bounce + (r & 1) * half, a, a, std::min(total, a + chunk), up);
+        rows.copy(hold.mem() + (r & 1) * chunk, a, a, std::min(total, a + chunk), up);
     };
     for (int r = 0; r < rounds; ++r) {
         if (up) {
@@ -449,7 +509,8 @@ int sphgpu_upload(sphgpu_ctx *c, const double *fields, uint64_t mask)
 {
     if (!c || !fields) return SPHGPU_E_ARG;
     mask &= SPHGPU_MASK_ALL & ~SPHGPU_MASK(SPHGPU_F_ID);
-    int rc = exchange_rows(c, const_cast<double *>(fields), mask, true);
+    BounceHold hold;
+    int rc = exchange_rows(c, const_cast<double *>(fields), mask, true, hold);
     if (rc) return rc;
     FieldPtrs fp = field_ptrs(c);
     hipLaunchKernelGGL(k_gather_fields, dim3(grid_for(c->n, 256)), dim3(256), 0, c->stream, fp,
@@ -474,6 +535,7 @@ int sphgpu_upload(sphgpu_ctx *c, const double *fields, uint64_t mask)
     if (mask & pos_rows) c->tree.valid = false;
     const bool ok = refresh_mirrors(c) == 0;
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    hold.give_back();
     return ok ? 0 : SPHGPU_E_HIP;
 }
 
@@ -486,9 +548,11 @@ int sphgpu_download(sphgpu_ctx *c, double *fields, uint64_t mask)
     hipLaunchKernelGGL(k_scatter_fields, dim3(grid_for(c->n, 256)), dim3(256), 0, c->stream, fp, c->stage,
                        (const int *)c->id, c->n, (unsigned long long)mask);
     HIPCHK(c, hipGetLastError());
-    int rc = exchange_rows(c, fields, mask, false);
+    BounceHold hold;
+    int rc = exchange_rows(c, fields, mask, false, hold);
     if (rc) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    hold.give_back();
     return 0;
 }
 

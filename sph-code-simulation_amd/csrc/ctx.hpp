@@ -42,10 +42,6 @@ constexpr int kAlt = 20;
 
 constexpr int kSyncWords = 5;  // Tree::sync_words
 
-// most pinned memory per context for uploads and downloads, two halves (a full
-// half takes 0.2 ms of DMA)
-constexpr size_t kBounceBytes = 16u << 20;
-
 // GSPH gradient rows in FP64 (grad_d[3], grad_p[3], grad_v[9])
 constexpr int kNGrad = 15;
 
@@ -185,8 +181,7 @@ struct sphgpu_ctx {
     bool mass_uniform = false;
     double mass_u = 0.0;
     double *stage = nullptr;     // host-exchange staging, [NFIELDS][n]; idle between exchanges
-    char *bounce = nullptr;      // pinned memory of the host exchange, two halves
-    size_t bounce_bytes = 0;
+    int exchanges = 0;           // of several rows, until the pinned halves are there
     hipEvent_t bounce_moved[2] = {};  // a half's copy has ended
     double *red = nullptr;       // reduction partials
     int red_blocks = 0;
