@@ -8,7 +8,7 @@
  * blocking on return (stream-ordered work is complete).  One host thread per
  * context; a context is not thread-safe.
  *
- * Memory beside the particle rows, lists and tree: 4 MB of pinned host memory
+ * Memory beside the particle rows, lists and tree: 8 MB of pinned host memory
  * for uploads and downloads, shared by the contexts of the process, set up when
  * one of them exchanges several rows for the third time and freed with the last
  * (the caller's rows are copied directly where it cannot be had, or while

@@ -170,9 +170,10 @@ static FieldPtrs field_ptrs(sphgpu_ctx *c)
 // when they are first written and 0.3 ms to have (memory of each context's own
 // made the first upload of 65k particles 1.0 ms instead of 0.25 and the creation
 // of a context up to twice as long), which a program that uploads, runs and
-// downloads once does not get back.  2 MB a half: with 0.25 MB 14 rows of 133k
-// take 750 us instead of 440, with 8 MB no less.
-constexpr size_t kBounceHalf = 2u << 20;
+// downloads once does not get back.  4 MB a half: with 2 MB the rows of 1M
+// particles came back as fast, but the program's 16 threads that converted them
+// right after took 10 to 45 ms in a third of the passes instead of 1 to 3.
+constexpr size_t kBounceHalf = 4u << 20;
 constexpr int kBounceAfter = 2;  // exchanges of a context without it
 
 namespace {
@@ -475,12 +476,16 @@ int exchange_rows(sphgpu_ctx *c, double *fields, uint64_t mask, bool up, BounceH
         }
         return 0;
     }
-    constexpr size_t chunk = kBounceHalf;
+    // up 16 rounds, of 2 MB at least, down 8, of 1 MB: what the first and the last
+    // round do alone is not hidden, and a round costs some 10 us itself (7 rows of
+    // 133k up 290 us in rounds of 1 MB, 243 of 2; down 300 and 312, 336 of 4)
+    const size_t least = up ? 2u << 20 : 1u << 20, part = (total / (up ? 16 : 8) + 4095) & ~(size_t)4095;
+    const size_t chunk = std::min(kBounceHalf, std::max(least, part));
     const int rounds = (int)((total + chunk - 1) / chunk);
     char *const dev = reinterpret_cast<char *>(c->stage);
     auto dma = [&](int r) {
         const size_t a = (size_t)r * chunk, len = std::min(chunk, total - a);
-        char *const host = hold.mem() + (r & 1) * chunk;
+        char *const host = hold.mem() + (r & 1) * kBounceHalf;
         const hipError_t e = up ? hipMemcpyAsync(dev + a, host, len, hipMemcpyHostToDevice, c->stream)
                                 : hipMemcpyAsync(host, dev + a, len, hipMemcpyDeviceToHost, c->stream);
         return e == hipSuccess ? hipEventRecord(c->bounce_moved[r & 1], c->stream) : e;
@@ -488,7 +493,7 @@ int exchange_rows(sphgpu_ctx *c, double *fields, uint64_t mask, bool up, BounceH
     if (!up) HIPCHK(c, dma(0));
     auto copy = [&](int r) {
         const size_t a = (size_t)r * chunk;
-        rows.copy(hold.mem() + (r & 1) * chunk, a, a, std::min(total, a + chunk), up);
+        rows.copy(hold.mem() + (r & 1) * kBounceHalf, a, a, std::min(total, a + chunk), up);
     };
     for (int r = 0; r < rounds; ++r) {
         if (up) {
