@@ -162,7 +162,6 @@ static FieldPtrs field_ptrs(sphgpu_ctx *c)
 }
 
 // --------------------------------------------------------------------------
-// --------------------------------------------------------------------------
 // Pinned memory of the host exchange, two halves, shared by the contexts of the
 // process: one exchange has it at a time and another one that comes meanwhile
 // copies its rows directly.  It is set up when a context exchanges rows for the
